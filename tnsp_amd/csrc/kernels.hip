@@ -1,8 +1,8 @@
 // CDNA4 (gfx950) kernels for the block-sparse tensor path.
 //
 //  permute  : batched strided block copy with the fermion sign folded in; one
-//             flat element space over all tasks, destination-ordered so that
-//             stores coalesce.
+//             wave per unit of a task, destination-ordered so that stores
+//             coalesce.
 //  gemm     : grouped GEMM over heterogeneous sector blocks, one workgroup per
 //             32x32 output tile, 4 waves x MFMA 16x16x4 (fp64 / fp32).
 //  qr       : batched Householder QR / LQ, one workgroup per sector block.
@@ -64,103 +64,73 @@ __device__ inline void perm_decode(uint32_t local, int rank, const int32_t* dims
     }
 }
 
-// Each workgroup copies PERM_CHUNK consecutive elements of the flat element
-// space of all tasks; each thread handles PERM_CHUNK / WG of them, WG apart,
-// all loads issued before the stores.  A chunk inside one task (the common
-// case: most elements belong to tasks larger than a chunk) reads that task's
-// descriptor once for the whole workgroup; a chunk spanning several tasks
-// locates each element's task through the prefix sums.
+// One wave per unit: FLAT_LANE x 64 consecutive elements of one task per
+// step, `elems` elements per unit, all loads of a step issued before its
+// stores.  What bounds the small launches is the time to the first load, not
+// bytes: a PEPS of bond dimension 4 makes thousands of tasks of 1 to 30
+// elements per launch.  The unit names its task, so a wave reads one
+// descriptor, through scalar loads, and searches nothing (walking prefix sums
+// thread by thread took 94 us per launch of 128 configurations of the 4x4
+// D=4 PEPS, the units 4.2 us; 50 and 32 us on the 8x8 D=8 one).  Lanes idle on a tiny task cost less than
+// the per-element descriptor reads that packing several tasks per wave needs.
 template<typename TS, typename T>
-__global__ __launch_bounds__(WG) void permute_kernel(const PermDev* __restrict__ tasks, const int64_t* __restrict__ prefix,
-                                                     const int32_t* __restrict__ wg_first) {
-    constexpr int PER = PERM_CHUNK / WG;
-    const int64_t base = int64_t(blockIdx.x) * PERM_CHUNK;
-    const int t0 = wg_first[blockIdx.x];
-    const int t_end = wg_first[gridDim.x];
-    const int64_t p0 = prefix[t0], p1 = prefix[t0 + 1];
-    if (base + PERM_CHUNK <= p1 || t0 + 1 == t_end) {
-        const PermDev& tk = tasks[t0];
-        const int rank = tk.rank;
-        int32_t dims[DEV_MAXR], ss[DEV_MAXR], ds[DEV_MAXR], sh[DEV_MAXR];
-        uint32_t mul[DEV_MAXR];
+__global__ __launch_bounds__(WG) void permute_kernel(const PermDev* __restrict__ tasks, const FlatUnit* __restrict__ units,
+                                                     int num_units, int elems) {
+    const int u = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * (WG / WAVE) + int(threadIdx.x) / WAVE);
+    if (u >= num_units) return;
+    const FlatUnit unit = units[u];
+    const PermDev& tk = tasks[unit.task];
+    const int rank = tk.rank;
+    int32_t dims[DEV_MAXR], ss[DEV_MAXR], ds[DEV_MAXR], sh[DEV_MAXR];
+    uint32_t mul[DEV_MAXR];
 #pragma unroll
-        for (int r = 0; r < DEV_MAXR; r++) {
-            dims[r] = tk.dims[r];
-            ss[r] = tk.ss[r];
-            ds[r] = tk.ds[r];
-            mul[r] = tk.mul[r];
-            sh[r] = tk.sh[r];
+    for (int r = 0; r < DEV_MAXR; r++) {
+        dims[r] = tk.dims[r];
+        ss[r] = tk.ss[r];
+        ds[r] = tk.ds[r];
+        mul[r] = tk.mul[r];
+        sh[r] = tk.sh[r];
+    }
+    const gptr<const TS> src = to_global(static_cast<const TS*>(tk.src));
+    const gptr<T> dst = to_global(static_cast<T*>(tk.dst));
+    const int neg = tk.neg;
+    const uint32_t n = uint32_t(tk.n), lane = threadIdx.x % WAVE;
+    const uint32_t first = uint32_t(unit.step) * uint32_t(elems), end = min(n, first + uint32_t(elems));
+    if (end - first <= WAVE) {
+        if (first + lane < end) {
+            int64_t so, dof;
+            perm_decode(first + lane, rank, dims, ss, ds, mul, sh, so, dof);
+            dst[dof] = neg_if(T(src[so]), neg);
         }
-        const gptr<const TS> src = to_global(static_cast<const TS*>(tk.src));
-        const gptr<T> dst = to_global(static_cast<T*>(tk.dst));
-        const bool neg = tk.neg != 0;
-        const int64_t left = p1 - base;  // elements of task t0 from base on
-        const uint32_t off = uint32_t(base - p0);
-        int64_t so[PER], dof[PER];
-#pragma unroll
-        for (int j = 0; j < PER; j++) {
-            const int e = threadIdx.x + j * WG;
-            so[j] = dof[j] = 0;
-            if (e < left) perm_decode(off + uint32_t(e), rank, dims, ss, ds, mul, sh, so[j], dof[j]);
-        }
-        T v[PER];
-#pragma unroll
-        for (int j = 0; j < PER; j++) v[j] = (threadIdx.x + j * WG < left) ? T(src[so[j]]) : T(0);
-#pragma unroll
-        for (int j = 0; j < PER; j++)
-            if (threadIdx.x + j * WG < left) dst[dof[j]] = neg_if(v[j], neg ? 1 : 0);
         return;
     }
-    int t = t0;
-    gptr<const TS> src[PER];
-    gptr<T> dst[PER];
-    int64_t so[PER], dof[PER];
-    bool neg[PER], ok[PER];
-    int64_t end = p1;
+    for (uint32_t base = first; base < end; base += FLAT_LANE * WAVE) {
+        int64_t so[FLAT_LANE], dof[FLAT_LANE];
 #pragma unroll
-    for (int j = 0; j < PER; j++) {
-        const int64_t e = base + threadIdx.x + int64_t(j) * WG;
-        // advance to the task containing e (tasks are contiguous in e)
-        while (end <= e && t < t_end) {
-            t++;
-            if (t < t_end) end = prefix[t + 1];
+        for (int j = 0; j < FLAT_LANE; j++) {
+            const uint32_t e = base + lane + j * WAVE;
+            so[j] = dof[j] = 0;
+            if (e < end) perm_decode(e, rank, dims, ss, ds, mul, sh, so[j], dof[j]);
         }
-        ok[j] = t < t_end;
-        so[j] = dof[j] = 0;
-        src[j] = nullptr;
-        dst[j] = nullptr;
-        neg[j] = false;
-        if (ok[j]) {
-            const PermDev& tk = tasks[t];
-            perm_decode(uint32_t(e - prefix[t]), tk.rank, tk.dims, tk.ss, tk.ds, tk.mul, tk.sh, so[j], dof[j]);
-            src[j] = to_global(static_cast<const TS*>(tk.src));
-            dst[j] = to_global(static_cast<T*>(tk.dst));
-            neg[j] = tk.neg != 0;
-        }
+        T v[FLAT_LANE];
+#pragma unroll
+        for (int j = 0; j < FLAT_LANE; j++) v[j] = (base + lane + j * WAVE < end) ? T(src[so[j]]) : T(0);
+#pragma unroll
+        for (int j = 0; j < FLAT_LANE; j++)
+            if (base + lane + j * WAVE < end) dst[dof[j]] = neg_if(v[j], neg);
     }
-    T v[PER];
-#pragma unroll
-    for (int j = 0; j < PER; j++) v[j] = ok[j] ? T(src[j][so[j]]) : T(0);
-#pragma unroll
-    for (int j = 0; j < PER; j++)
-        if (ok[j]) dst[j][dof[j]] = neg_if(v[j], neg[j] ? 1 : 0);
 }
 
 template<typename T>
-__global__ __launch_bounds__(WG) void fill_kernel(const FillDev* __restrict__ tasks, const int64_t* __restrict__ prefix,
-                                                  const int32_t* __restrict__ wg_first) {
-    const int64_t base = int64_t(blockIdx.x) * PERM_CHUNK;
-    int t = wg_first[blockIdx.x];
-    for (int j = 0; j < PERM_CHUNK / WG; j++) {
-        const int64_t e = base + threadIdx.x + int64_t(j) * WG;
-        int64_t end = prefix[t + 1];
-        while (end <= e) {
-            t++;
-            if (t >= wg_first[gridDim.x]) return;
-            end = prefix[t + 1];
-        }
-        to_global(static_cast<T*>(tasks[t].p))[e - prefix[t]] = T(0);
-    }
+__global__ __launch_bounds__(WG) void fill_kernel(const FillDev* __restrict__ tasks, const FlatUnit* __restrict__ units,
+                                                  int num_units, int elems) {
+    const int u = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * (WG / WAVE) + int(threadIdx.x) / WAVE);
+    if (u >= num_units) return;
+    const FlatUnit unit = units[u];
+    const FillDev& tk = tasks[unit.task];
+    const gptr<T> p = to_global(static_cast<T*>(tk.p));
+    const int64_t first = int64_t(unit.step) * elems, end = min(tk.n, first + int64_t(elems));
+    for (int64_t e = first + threadIdx.x % WAVE; e < end; e += WAVE) p[e] = T(0);
 }
 
 // ------------------------------------------------------------------- gemm
@@ -1739,39 +1709,44 @@ inline void check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// one wave per unit, WG / WAVE units per workgroup
+inline unsigned flat_blocks(int64_t num_units) { return unsigned((num_units + WG / WAVE - 1) / (WG / WAVE)); }
+
 }  // namespace
 
-void launch_permute(const PermDev* tasks, const int64_t* prefix, const int32_t* wg_first, int64_t num_wg, int dtype,
+void launch_permute(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems, int dtype,
                     hipStream_t stream) {
-    if (num_wg <= 0) return;
+    if (num_units <= 0) return;
     if (dtype == 0)
-        hipLaunchKernelGGL((permute_kernel<double, double>), dim3(unsigned(num_wg)), dim3(WG), 0, stream, tasks, prefix,
-                           wg_first);
+        hipLaunchKernelGGL((permute_kernel<double, double>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
+                           units, int(num_units), elems);
     else
-        hipLaunchKernelGGL((permute_kernel<float, float>), dim3(unsigned(num_wg)), dim3(WG), 0, stream, tasks, prefix,
-                           wg_first);
+        hipLaunchKernelGGL((permute_kernel<float, float>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
+                           units, int(num_units), elems);
     check(hipGetLastError(), "permute launch");
 }
 
-void launch_permute_from_f64(const PermDev* tasks, const int64_t* prefix, const int32_t* wg_first, int64_t num_wg,
+void launch_permute_from_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems,
                              int dtype, hipStream_t stream) {
-    if (num_wg <= 0) return;
+    if (num_units <= 0) return;
     if (dtype == 0)
-        hipLaunchKernelGGL((permute_kernel<double, double>), dim3(unsigned(num_wg)), dim3(WG), 0, stream, tasks, prefix,
-                           wg_first);
+        hipLaunchKernelGGL((permute_kernel<double, double>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
+                           units, int(num_units), elems);
     else
-        hipLaunchKernelGGL((permute_kernel<double, float>), dim3(unsigned(num_wg)), dim3(WG), 0, stream, tasks, prefix,
-                           wg_first);
+        hipLaunchKernelGGL((permute_kernel<double, float>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
+                           units, int(num_units), elems);
     check(hipGetLastError(), "permute launch");
 }
 
-void launch_fill(const FillDev* tasks, const int64_t* prefix, const int32_t* wg_first, int64_t num_wg, int dtype,
+void launch_fill(const FillDev* tasks, const FlatUnit* units, int64_t num_units, int elems, int dtype,
                  hipStream_t stream) {
-    if (num_wg <= 0) return;
+    if (num_units <= 0) return;
     if (dtype == 0)
-        hipLaunchKernelGGL(fill_kernel<double>, dim3(unsigned(num_wg)), dim3(WG), 0, stream, tasks, prefix, wg_first);
+        hipLaunchKernelGGL(fill_kernel<double>, dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
+                           units, int(num_units), elems);
     else
-        hipLaunchKernelGGL(fill_kernel<float>, dim3(unsigned(num_wg)), dim3(WG), 0, stream, tasks, prefix, wg_first);
+        hipLaunchKernelGGL(fill_kernel<float>, dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
+                           units, int(num_units), elems);
     check(hipGetLastError(), "fill launch");
 }
 
@@ -1788,11 +1763,11 @@ void launch_gather_f64(const GatherDev* tasks, int64_t num, double* dst, hipStre
     check(hipGetLastError(), "gather launch");
 }
 
-void launch_permute_to_f64(const PermDev* tasks, const int64_t* prefix, const int32_t* wg_first, int64_t num_wg,
+void launch_permute_to_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems,
                            hipStream_t stream) {
-    if (num_wg <= 0) return;
-    hipLaunchKernelGGL((permute_kernel<float, double>), dim3(unsigned(num_wg)), dim3(WG), 0, stream, tasks, prefix,
-                       wg_first);
+    if (num_units <= 0) return;
+    hipLaunchKernelGGL((permute_kernel<float, double>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
+                           units, int(num_units), elems);
     check(hipGetLastError(), "permute launch");
 }
 

@@ -23,7 +23,7 @@ namespace {
 // workspace part (contract operands and product, QR factors and the global
 // scratch of large sectors) and task-record part of the array
 constexpr int64_t NOALLOC_WORKSPACE_BYTES = int64_t(64) << 20;
-constexpr int64_t NOALLOC_TASK_BYTES = int64_t(4) << 20;
+constexpr int64_t NOALLOC_TASK_BYTES = (int64_t(4) << 20) + (int64_t(128) << 10);  // 4 MiB and the units' excess
 
 __device__ __align__(256) unsigned char scratch[NOALLOC_WORKSPACE_BYTES + NOALLOC_TASK_BYTES];
 

@@ -184,26 +184,22 @@ void Batch::flush_flat(Kind kind, std::vector<PermDev>& pd, std::vector<FillDev>
     const bool isfill = kind == FILL;
     const size_t T = isfill ? fd.size() : pd.size();
     if (T == 0) return;
-    std::vector<int64_t> prefix(T + 1, 0);
-    for (size_t i = 0; i < T; i++) prefix[i + 1] = prefix[i] + (isfill ? fd[i].n : pd[i].n);
-    const int64_t total = prefix[T];
-    const int64_t nwg = (total + PERM_CHUNK - 1) / PERM_CHUNK;
-    if (nwg >= (int64_t(1) << 31)) throw Error("permute launch too large");
-    std::vector<int32_t> wg(nwg + 1);
-    size_t t = 0;
-    for (int64_t w = 0; w < nwg; w++) {
-        const int64_t e = w * PERM_CHUNK;
-        while (t + 1 < T && prefix[t + 1] <= e) t++;
-        wg[w] = int32_t(t);
+    int64_t total = 0;
+    for (size_t i = 0; i < T; i++) total += isfill ? fd[i].n : pd[i].n;
+    const int64_t elems = flat_unit_elems(total);
+    std::vector<FlatUnit> units;
+    units.reserve(T + size_t(total / elems));
+    for (size_t i = 0; i < T; i++) {
+        const int64_t n = isfill ? fd[i].n : pd[i].n;
+        for (int64_t k = 0; k * elems < n; k++) units.push_back(FlatUnit{int32_t(i), int32_t(k)});
     }
-    wg[nwg] = int32_t(T);
+    if (int64_t(units.size()) >= (int64_t(1) << 31)) throw Error("permute launch too large");
     Cmd c;
     c.kind = kind;
     c.tasks = isfill ? put(fd) : put(pd);
-    c.prefix = put(prefix);
-    c.wg = put(wg);
-    c.count = int64_t(T);
-    c.nwg = nwg;
+    c.prefix = put(units);
+    c.count = elems;
+    c.nwg = int64_t(units.size());
     c.units = pend_units_[kind];
     pend_units_[kind] = 0;
     cmds_.push_back(c);
@@ -294,7 +290,6 @@ void Batch::flush_gemm() {
         c.kind = GEMM;
         c.tasks = tasks;
         c.prefix = put(ptile_[v]);
-        c.wg = 0;
         c.count = int64_t(pgemm_.size());
         c.nwg = int64_t(ptile_[v].size());
         c.units = pgemm_units_[v];
@@ -366,7 +361,7 @@ void Batch::flush_decomp(Kind kind, std::vector<D>& tasks, std::vector<double>& 
         Cmd c;
         c.kind = kind;
         c.tasks = put(v);
-        c.prefix = c.wg = 0;
+        c.prefix = 0;
         c.count = c.nwg = int64_t(v.size());
         c.units = units[part];
         c.lds = (part == 0 || part >= 4) ? 0 : (need[part] + 255) / 256 * 256;  // fixed inside the launcher
@@ -434,26 +429,21 @@ void Batch::run(hipStream_t st) {
             case PERM:
                 if (c.conv == 1)
                     launch_permute_from_f64(reinterpret_cast<const PermDev*>(base + c.tasks),
-                                            reinterpret_cast<const int64_t*>(base + c.prefix),
-                                            reinterpret_cast<const int32_t*>(base + c.wg), c.nwg, 1, st);
+                                            reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), 1, st);
                 else if (c.conv == 2)
                     launch_permute_to_f64(reinterpret_cast<const PermDev*>(base + c.tasks),
-                                          reinterpret_cast<const int64_t*>(base + c.prefix),
-                                          reinterpret_cast<const int32_t*>(base + c.wg), c.nwg, st);
+                                          reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), st);
                 else
                     launch_permute(reinterpret_cast<const PermDev*>(base + c.tasks),
-                                   reinterpret_cast<const int64_t*>(base + c.prefix),
-                                   reinterpret_cast<const int32_t*>(base + c.wg), c.nwg, dtype_, st);
+                                   reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), dtype_, st);
                 break;
             case DIAG:
                 launch_permute_from_f64(reinterpret_cast<const PermDev*>(base + c.tasks),
-                                        reinterpret_cast<const int64_t*>(base + c.prefix),
-                                        reinterpret_cast<const int32_t*>(base + c.wg), c.nwg, dtype_, st);
+                                        reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), dtype_, st);
                 break;
             case FILL:
                 launch_fill(reinterpret_cast<const FillDev*>(base + c.tasks),
-                            reinterpret_cast<const int64_t*>(base + c.prefix),
-                            reinterpret_cast<const int32_t*>(base + c.wg), c.nwg, c.dt >= 0 ? c.dt : dtype_, st);
+                            reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), c.dt >= 0 ? c.dt : dtype_, st);
                 break;
             case GEMM:
                 launch_gemm(reinterpret_cast<const GemmDev*>(base + c.tasks),
