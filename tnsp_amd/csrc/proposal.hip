@@ -7,9 +7,11 @@
 // sampling are written here; the caller owns every buffer.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 
 #include "proposal.hpp"
 
@@ -17,6 +19,7 @@ namespace tns {
 namespace {
 
 constexpr int NT = 256;
+constexpr size_t CONV_LDS_MAX = 160 * 1024;
 
 __device__ inline float bf16_to_f(uint16_t h) { return __uint_as_float(uint32_t(h) << 16); }
 
@@ -26,152 +29,226 @@ __device__ inline uint16_t f_to_bf16(float x) {
     return uint16_t(u >> 16);
 }
 
-// y[b, co] = bias[co] + sum_ci w[co, ci] (*) x[b, ci]; one workgroup per
-// sample; the padded input plane stack and the weights sit in LDS.
-__global__ __launch_bounds__(NT) void conv_fwd_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
-                                                     const float* __restrict__ bias, float* __restrict__ y, int cin,
-                                                     int cout, int H, int W, int relu) {
-    extern __shared__ float sm[];
-    const int HP = H + 2, WP = W + 2;
-    float* xs = sm;                       // cin x HP x WP
-    float* ws = sm + cin * HP * WP;       // cout x cin x 9
-    const int b = blockIdx.x, tid = threadIdx.x;
-    const float* xb = x + int64_t(b) * cin * H * W;
-    for (int e = tid; e < cin * HP * WP; e += NT) {
-        const int c = e / (HP * WP), r = (e / WP) % HP, q = e % WP;
-        const int i = r - 1, j = q - 1;
-        xs[e] = (i >= 0 && i < H && j >= 0 && j < W) ? xb[(c * H + i) * W + j] : 0.f;
-    }
-    for (int e = tid; e < cout * cin * 9; e += NT) ws[e] = bf16_to_f(w[e]);
-    __syncthreads();
-    float* yb = y + int64_t(b) * cout * H * W;
-    for (int o = tid; o < cout * H * W; o += NT) {
-        const int co = o / (H * W), i = (o / W) % H, j = o % W;
-        float acc = bias[co];
-        for (int ci = 0; ci < cin; ci++) {
-            const float* xp = xs + (ci * HP + i) * WP + j;
-            const float* wp = ws + (co * cin + ci) * 9;
-#pragma unroll
-            for (int ky = 0; ky < 3; ky++)
-#pragma unroll
-                for (int kx = 0; kx < 3; kx++) acc += wp[ky * 3 + kx] * xp[ky * WP + kx];
-        }
-        yb[o] = relu ? fmaxf(acc, 0.f) : acc;
-    }
+typedef float f4 __attribute__((ext_vector_type(4)));
+
+// LDS row of one padded channel plane of HP x WP values: with a stride of 4
+// modulo 8 words the 16 channels x 4 positions (or 16 positions x 4 channels)
+// of an MFMA operand read fall into different banks.  Without the padding
+// where it would not fit.
+inline int plane_stride(int HP, int WP) {
+    int s = HP * WP;
+    while (s % 8 != 4) s++;
+    return s;
 }
 
-// dx[b, ci] = sum_co w[co, ci] (*)^T dy[b, co]; dy is masked by the ReLU of
-// the layer output y when relu_y is non-null.
-__global__ __launch_bounds__(NT) void conv_bwd_data_kernel(const float* __restrict__ dy, const float* __restrict__ relu_y,
-                                                           const uint16_t* __restrict__ w, float* __restrict__ dx,
-                                                           int cin, int cout, int H, int W) {
+// One 3x3 convolution as a product on the fp32 MFMA (16x16x4), for the forward
+// pass (out = y, in = x, channels m = co, k = ci) and for the data gradient
+// (out = dx, in = dy masked by the ReLU of y, m = ci, k = co, flipped taps):
+//   out[b, m, p] = bias[m] + sum_{tap, k} w[m, k, tap] in[b, k, p + tap]
+// Rows of a tile are 16 output channels, columns 16 positions; the reduction
+// runs tap by tap over groups of 4 input channels.  A workgroup keeps the
+// weights (bf16) in LDS and walks samples; the padded input planes of the
+// sample sit in LDS, so a tap is an offset.  Each wave takes every fourth
+// column tile and all MT row tiles.
+// Lane l holds w(m0 + l % 16, k0 + l / 16) and in(k0 + l / 16, p0 + l % 16);
+// accumulator rows 4 (l / 16) + i.
+// The VALU version read LDS twice per multiply-add: 66 (forward) and 84 us
+// (data gradient) per launch on 1024 samples of 32 channels, 8 x 8; this
+// kernel 25 us for either.  The floor is 8 us of fp32 arithmetic.
+template<int MT>
+__global__ __launch_bounds__(NT) void conv_mfma_kernel(const float* __restrict__ in, const float* __restrict__ relu_y,
+                                                       const uint16_t* __restrict__ w, const float* __restrict__ bias,
+                                                       float* __restrict__ out, int B, int M, int K, int H, int W,
+                                                       int S, int flip, int relu) {
     extern __shared__ float sm[];
-    const int HP = H + 2, WP = W + 2;
-    float* gs = sm;                   // cout x HP x WP (padded, masked dy)
-    float* ws = sm + cout * HP * WP;  // cout x cin x 9
-    const int b = blockIdx.x, tid = threadIdx.x;
-    const float* gb = dy + int64_t(b) * cout * H * W;
-    const float* yb = relu_y ? relu_y + int64_t(b) * cout * H * W : nullptr;
-    for (int e = tid; e < cout * HP * WP; e += NT) {
-        const int c = e / (HP * WP), r = (e / WP) % HP, q = e % WP;
-        const int i = r - 1, j = q - 1;
-        float v = 0.f;
-        if (i >= 0 && i < H && j >= 0 && j < W) {
-            const int k = (c * H + i) * W + j;
-            v = gb[k];
-            if (yb && !(yb[k] > 0.f)) v = 0.f;
-        }
-        gs[e] = v;
+    const int HP = H + 2, WP = W + 2, HW = H * W;
+    float* xs = sm;                                             // K planes of stride S
+    uint16_t* ws = reinterpret_cast<uint16_t*>(sm + K * S);     // [tap][k][m]
+    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+    const int lm = lane % 16, lk = lane / 16;
+    for (int q = tid; q < M * K; q += NT) {
+        const int m = flip ? q % M : q / K, k = flip ? q / M : q % K;
+#pragma unroll
+        for (int tap = 0; tap < 9; tap++) ws[((flip ? 8 - tap : tap) * K + k) * M + m] = w[q * 9 + tap];
     }
-    for (int e = tid; e < cout * cin * 9; e += NT) ws[e] = bf16_to_f(w[e]);
-    __syncthreads();
-    float* xb = dx + int64_t(b) * cin * H * W;
-    for (int o = tid; o < cin * H * W; o += NT) {
-        const int ci = o / (H * W), i = (o / W) % H, j = o % W;
-        float acc = 0.f;
-        for (int co = 0; co < cout; co++) {
-            // y(i', j') uses x(i' + ky - 1, j' + kx - 1): x(i, j) feeds
-            // y(i - ky + 1, j - kx + 1), i.e. padded row i - ky + 2
-            const float* gp = gs + (co * HP + i) * WP + j;
-            const float* wp = ws + (co * cin + ci) * 9;
-#pragma unroll
-            for (int ky = 0; ky < 3; ky++)
-#pragma unroll
-                for (int kx = 0; kx < 3; kx++) acc += wp[ky * 3 + kx] * gp[(2 - ky) * WP + (2 - kx)];
+    // the border of every plane stays zero
+    for (int e = tid; e < K * S; e += NT) xs[e] = 0.f;
+    for (int b = blockIdx.x; b < B; b += gridDim.x) {
+        __syncthreads();
+        const float* ib = in + int64_t(b) * K * HW;
+        const float* yb = relu_y ? relu_y + int64_t(b) * K * HW : nullptr;
+        for (int e = tid; e < K * HW; e += NT) {
+            const int k = e / HW, p = e - k * HW, i = p / W, j = p - i * W;
+            float v = ib[e];
+            if (yb && !(yb[e] > 0.f)) v = 0.f;
+            xs[k * S + (i + 1) * WP + j + 1] = v;
         }
-        xb[o] = acc;
+        __syncthreads();
+        float* ob = out + int64_t(b) * M * HW;
+        for (int p0 = 16 * wave; p0 < HW; p0 += 16 * (NT / 64)) {
+            // columns beyond HW read position 0 and are not stored, rows
+            // beyond M likewise read channel M - 1
+            const int p = p0 + lm < HW ? p0 + lm : 0;
+            const float* xp = xs + (p / W) * WP + p % W;
+            f4 acc[MT];
+            int mrow[MT];
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                mrow[t] = min(16 * t + lm, M - 1);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int m = 16 * t + 4 * lk + i;
+                    acc[t][i] = bias && m < M ? bias[m] : 0.f;
+                }
+            }
+            for (int tap = 0; tap < 9; tap++) {
+                const float* xt = xp + (tap / 3) * WP + tap % 3;
+                const uint16_t* wt = ws + tap * K * M;
+#pragma unroll 2
+                for (int k0 = 0; k0 < K; k0 += 4) {
+                    // channels beyond K count nothing on either side
+                    const int k = k0 + lk, kc = min(k, K - 1);
+                    const bool ok = k < K;
+                    const float x = ok ? xt[kc * S] : 0.f;
+#pragma unroll
+                    for (int t = 0; t < MT; t++) {
+                        const float a = ok ? bf16_to_f(wt[kc * M + mrow[t]]) : 0.f;
+                        acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x, acc[t], 0, 0, 0);
+                    }
+                }
+            }
+            if (p0 + lm < HW) {
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const int m = 16 * t + 4 * lk + i;
+                        if (m < M) ob[m * HW + p0 + lm] = relu ? fmaxf(acc[t][i], 0.f) : acc[t][i];
+                    }
+            }
+        }
     }
 }
 
 // Partial weight / bias gradients over a chunk of samples per workgroup:
-// part[chunk][co][ci][9] and partb[chunk][co].
+// part[chunk][co][ci][9] and partb[chunk][co], as a product on the fp32 MFMA
+// with the positions as the reduction dimension:
+//   part[co, n] = sum_{b, i, j} dy[b, co, i, j] x[b, ci, i + ky, j + kx],
+//   n = (ci, ky, kx) flattened.
+// A k step is 4 positions of one row; both operands are zero beyond the row.  Each wave takes every fourth tile of 16
+// columns n and all MT row tiles of 16 channels co.
+// Lane l holds dy(co0 + l % 16, p + l / 16) and x(p + l / 16, n0 + l % 16).
+// The VALU version (one thread per weight, 64 samples per workgroup, 16
+// workgroups for 1024 samples) took 3.8 ms per launch on 1024 samples of 32
+// channels, 8 x 8; this kernel 31 us and its reduction 12.
+template<int MT, int NPW>
 __global__ __launch_bounds__(NT) void conv_bwd_weight_kernel(const float* __restrict__ dy,
                                                              const float* __restrict__ relu_y,
                                                              const float* __restrict__ x, float* __restrict__ part,
                                                              float* __restrict__ partb, int B, int per_chunk, int cin,
-                                                             int cout, int H, int W) {
+                                                             int cout, int H, int W, int S, int G) {
     extern __shared__ float sm[];
-    const int HP = H + 2, WP = W + 2;
-    float* xs = sm;                   // cin x HP x WP
-    float* gs = sm + cin * HP * WP;   // cout x H x W
-    const int tid = threadIdx.x, chunk = blockIdx.x;
-    const int nw = cout * cin * 9;
-    constexpr int MAXPT = 64;  // accumulators per thread: nw <= NT * MAXPT
-    float acc[MAXPT];
-    float accb = 0.f;
+    const int WP = W + 2, HW = H * W;
+    float* xs = sm;            // cin padded planes of stride S
+    float* gs = sm + cin * S;  // cout planes H x W of stride G
+    const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64, chunk = blockIdx.x;
+    const int lm = lane % 16, lk = lane / 16;
+    const int nw = cout * cin * 9, N = cin * 9;
+    f4 acc[MT][NPW];
+    int xoff[NPW], goff[MT];
 #pragma unroll
-    for (int q = 0; q < MAXPT; q++) acc[q] = 0.f;
+    for (int u = 0; u < NPW; u++) {
+        // columns beyond N read column N - 1 and are not stored
+        const int n = min(16 * (wave + 4 * u) + lm, N - 1);
+        xoff[u] = (n / 9) * S + ((n % 9) / 3) * WP + n % 3;
+#pragma unroll
+        for (int t = 0; t < MT; t++) acc[t][u] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int t = 0; t < MT; t++) goff[t] = min(16 * t + lm, cout - 1) * G;
+    for (int e = tid; e < cin * S + cout * G; e += NT) sm[e] = 0.f;
+    // bias: TB threads per channel, a power of two of neighbouring lanes
+    int TB = 4;
+    while (TB < 64 && 2 * TB * cout <= NT) TB *= 2;
+    float accb = 0.f;
     const int b0 = chunk * per_chunk, b1 = min(B, b0 + per_chunk);
     for (int b = b0; b < b1; b++) {
-        const float* xb = x + int64_t(b) * cin * H * W;
-        const float* gb = dy + int64_t(b) * cout * H * W;
-        const float* yb = relu_y ? relu_y + int64_t(b) * cout * H * W : nullptr;
+        const float* xb = x + int64_t(b) * cin * HW;
+        const float* gb = dy + int64_t(b) * cout * HW;
+        const float* yb = relu_y ? relu_y + int64_t(b) * cout * HW : nullptr;
         __syncthreads();
-        for (int e = tid; e < cin * HP * WP; e += NT) {
-            const int c = e / (HP * WP), r = (e / WP) % HP, q = e % WP;
-            const int i = r - 1, j = q - 1;
-            xs[e] = (i >= 0 && i < H && j >= 0 && j < W) ? xb[(c * H + i) * W + j] : 0.f;
+        for (int e = tid; e < cin * HW; e += NT) {
+            const int c = e / HW, p = e - c * HW, i = p / W, j = p - i * W;
+            xs[c * S + (i + 1) * WP + j + 1] = xb[e];
         }
-        for (int e = tid; e < cout * H * W; e += NT) {
+        for (int e = tid; e < cout * HW; e += NT) {
+            const int c = e / HW, p = e - c * HW;
             float v = gb[e];
             if (yb && !(yb[e] > 0.f)) v = 0.f;
-            gs[e] = v;
+            gs[c * G + p] = v;
         }
         __syncthreads();
+        for (int i = 0; i < H; i++) {
+            for (int j = 0; j < W; j += 4) {
+                // beyond the row both operands are zero
+                const bool ok = j + lk < W;
+                const int go = ok ? i * W + j + lk : 0, xo = ok ? i * WP + j + lk : 0;
+                float a[MT];
 #pragma unroll
-        for (int q = 0; q < MAXPT; q++) {
-            const int k = tid + q * NT;
-            if (k < nw) {
-                const int co = k / (cin * 9), ci = (k / 9) % cin, kk = k % 9, ky = kk / 3, kx = kk % 3;
-                const float* gp = gs + co * H * W;
-                const float* xp = xs + (ci * HP + ky) * WP + kx;
-                float s = 0.f;
-                for (int i = 0; i < H; i++)
-                    for (int j = 0; j < W; j++) s += gp[i * W + j] * xp[i * WP + j];
-                acc[q] += s;
+                for (int t = 0; t < MT; t++) {
+                    const float v = gs[goff[t] + go];
+                    a[t] = ok ? v : 0.f;
+                }
+#pragma unroll
+                for (int u = 0; u < NPW; u++) {
+                    const float r = xs[xoff[u] + xo];
+                    const float v = ok ? r : 0.f;
+#pragma unroll
+                    for (int t = 0; t < MT; t++)
+                        acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], v, acc[t][u], 0, 0, 0);
+                }
             }
         }
-        if (tid < cout) {
-            const float* gp = gs + tid * H * W;
-            float s = 0.f;
-            for (int e = 0; e < H * W; e++) s += gp[e];
-            accb += s;
+        if (tid / TB < cout) {
+            const float* gp = gs + (tid / TB) * G;
+            for (int e = tid % TB; e < HW; e += TB) accb += gp[e];
         }
     }
 #pragma unroll
-    for (int q = 0; q < MAXPT; q++) {
-        const int k = tid + q * NT;
-        if (k < nw) part[int64_t(chunk) * nw + k] = acc[q];
-    }
-    if (tid < cout) partb[int64_t(chunk) * cout + tid] = accb;
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int u = 0; u < NPW; u++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int co = 16 * t + 4 * lk + i, n = 16 * (wave + 4 * u) + lm;
+                if (co < cout && n < N) part[int64_t(chunk) * nw + co * N + n] = acc[t][u][i];
+            }
+    for (int o = 1; o < TB; o <<= 1) accb += __shfl_xor(accb, o, 64);
+    if (tid / TB < cout && tid % TB == 0) partb[int64_t(chunk) * cout + tid / TB] = accb;
 }
 
-__global__ void reduce_chunks_kernel(const float* __restrict__ part, int chunks, int n, float* __restrict__ out) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
+// out[k] = sum over the chunks of part[c][k], k < n, for the weights and the
+// biases in one launch: 64 outputs per workgroup, its four waves take every
+// fourth chunk and their sums meet in LDS (one thread per output left most of
+// the chip idle behind a serial chain over the chunks).
+__global__ __launch_bounds__(NT) void reduce_chunks_kernel(const float* __restrict__ part, const float* __restrict__ partb,
+                                                           int chunks, int nw, int nb, float* __restrict__ dw,
+                                                           float* __restrict__ db) {
+    __shared__ float red[NT / 64][64];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int wblocks = (nw + 63) / 64;
+    const bool bias = int(blockIdx.x) >= wblocks;
+    const int n = bias ? nb : nw;
+    const float* src = bias ? partb : part;
+    const int k = (int(blockIdx.x) - (bias ? wblocks : 0)) * 64 + lane;
     float s = 0.f;
-    for (int c = 0; c < chunks; c++) s += part[int64_t(c) * n + k];
-    out[k] = s;
+    if (k < n) {
+#pragma unroll 4
+        for (int c = wave; c < chunks; c += NT / 64) s += src[int64_t(c) * n + k];
+    }
+    red[wave][lane] = s;
+    __syncthreads();
+    if (wave == 0 && k < n) (bias ? db : dw)[k] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
 
 // hop h = d * H W + s: valid when site s is filled and its neighbour in
@@ -308,14 +385,37 @@ void conv_check(int cin, int cout, int H, int W) {
     if (cout * cin * 9 > NT * 64) throw std::runtime_error("conv3x3: too many weights for the gradient kernel");
 }
 
+namespace {
+void launch_conv_mfma(const float* in, const float* relu_y, const uint16_t* w, const float* bias, float* out, int B,
+                      int M, int K, int H, int W, int flip, int relu, hipStream_t st) {
+    const size_t wbytes = size_t(M) * K * 9 * sizeof(uint16_t);
+    int S = plane_stride(H + 2, W + 2);
+    if (size_t(K) * S * sizeof(float) + wbytes > CONV_LDS_MAX) S = (H + 2) * (W + 2);
+    const size_t lds = size_t(K) * S * sizeof(float) + wbytes;
+    // up to four workgroups per CU with the same number of samples each (one
+    // more for some), the weights staged once per workgroup
+    const int per = (B + 1023) / 1024;
+    const dim3 grid(unsigned((B + per - 1) / per));
+    auto go = [&](auto kernel) {
+        allow(reinterpret_cast<const void*>(kernel), lds);
+        hipLaunchKernelGGL(kernel, grid, dim3(NT), lds, st, in, relu_y, w, bias, out, B, M, K, H, W, S, flip, relu);
+    };
+    if (M <= 16)
+        go(conv_mfma_kernel<1>);
+    else if (M <= 32)
+        go(conv_mfma_kernel<2>);
+    else
+        go(conv_mfma_kernel<4>);
+}
+}  // namespace
+
 void launch_conv_fwd(const float* x, const uint16_t* w, const float* bias, float* y, int B, int cin, int cout, int H,
                      int W, int relu, hipStream_t st) {
     conv_check(cin, cout, H, W);
     if (B <= 0) return;
-    const size_t lds = size_t(cin * (H + 2) * (W + 2) + cout * cin * 9) * sizeof(float);
-    if (lds > 160 * 1024) throw std::runtime_error("conv3x3: working set exceeds LDS");
-    allow(reinterpret_cast<const void*>(conv_fwd_kernel), lds);
-    hipLaunchKernelGGL(conv_fwd_kernel, dim3(unsigned(B)), dim3(NT), lds, st, x, w, bias, y, cin, cout, H, W, relu);
+    if (size_t(cin * (H + 2) * (W + 2) + cout * cin * 9) * sizeof(float) > CONV_LDS_MAX)
+        throw std::runtime_error("conv3x3: working set exceeds LDS");
+    launch_conv_mfma(x, nullptr, w, bias, y, B, cout, cin, H, W, 0, relu, st);
     check(hipGetLastError(), "conv forward launch");
 }
 
@@ -323,15 +423,23 @@ void launch_conv_bwd_data(const float* dy, const float* relu_y, const uint16_t* 
                           int H, int W, hipStream_t st) {
     conv_check(cin, cout, H, W);
     if (B <= 0) return;
-    const size_t lds = size_t(cout * (H + 2) * (W + 2) + cout * cin * 9) * sizeof(float);
-    if (lds > 160 * 1024) throw std::runtime_error("conv3x3: working set exceeds LDS");
-    allow(reinterpret_cast<const void*>(conv_bwd_data_kernel), lds);
-    hipLaunchKernelGGL(conv_bwd_data_kernel, dim3(unsigned(B)), dim3(NT), lds, st, dy, relu_y, w, dx, cin, cout, H, W);
+    if (size_t(cout * (H + 2) * (W + 2) + cout * cin * 9) * sizeof(float) > CONV_LDS_MAX)
+        throw std::runtime_error("conv3x3: working set exceeds LDS");
+    launch_conv_mfma(dy, relu_y, w, nullptr, dx, B, cin, cout, H, W, 1, 0, st);
     check(hipGetLastError(), "conv backward-data launch");
 }
 
+namespace {
+// Samples per workgroup of the weight gradient: enough workgroups to fill the
+// chip (each CU holds a few), few enough that their partial gradients (37 KB
+// each at 32 channels) stay a small part of the traffic.  1024 samples of 32
+// channels, 8 x 8, all four layers with the reductions: 143 us with 2 samples
+// per workgroup, 165 us with 4, 296 us with 8.
+int conv_chunk(int B) { return std::max(1, (B + 511) / 512); }
+}  // namespace
+
 int64_t conv_bwd_weight_workspace(int B, int cin, int cout) {
-    const int chunks = (B + CONV_CHUNK - 1) / CONV_CHUNK;
+    const int chunks = B > 0 ? (B + conv_chunk(B) - 1) / conv_chunk(B) : 0;
     return int64_t(chunks) * (int64_t(cout) * cin * 9 + cout) * int64_t(sizeof(float));
 }
 
@@ -339,19 +447,46 @@ void launch_conv_bwd_weight(const float* dy, const float* relu_y, const float* x
                             int cout, int H, int W, float* workspace, hipStream_t st) {
     conv_check(cin, cout, H, W);
     if (B <= 0) return;
-    const int chunks = (B + CONV_CHUNK - 1) / CONV_CHUNK;
+    if (size_t(cin * (H + 2) * (W + 2) + cout * H * W) * sizeof(float) > CONV_LDS_MAX)
+        throw std::runtime_error("conv3x3: working set exceeds LDS");
+    const int per = conv_chunk(B), chunks = (B + per - 1) / per;
     const int nw = cout * cin * 9;
     float* part = workspace;
     float* partb = workspace + int64_t(chunks) * nw;
-    const size_t lds = size_t(cin * (H + 2) * (W + 2) + cout * H * W) * sizeof(float);
-    if (lds > 160 * 1024) throw std::runtime_error("conv3x3: working set exceeds LDS");
-    allow(reinterpret_cast<const void*>(conv_bwd_weight_kernel), lds);
-    hipLaunchKernelGGL(conv_bwd_weight_kernel, dim3(unsigned(chunks)), dim3(NT), lds, st, dy, relu_y, x, part, partb, B,
-                       CONV_CHUNK, cin, cout, H, W);
+    int S = plane_stride(H + 2, W + 2), G = plane_stride(H, W);
+    auto bytes = [&] { return (size_t(cin) * S + size_t(cout) * G) * sizeof(float); };
+    if (bytes() > CONV_LDS_MAX) {
+        S = (H + 2) * (W + 2);
+        G = H * W;
+    }
+    const size_t lds = bytes();
+    const dim3 grid(static_cast<unsigned>(chunks));
+    auto go = [&](auto kernel) {
+        allow(reinterpret_cast<const void*>(kernel), lds);
+        hipLaunchKernelGGL(kernel, grid, dim3(NT), lds, st, dy, relu_y, x, part, partb, B, per, cin, cout, H, W, S, G);
+    };
+    // column tiles per wave: ceil(ceil(9 cin / 16) / 4), 9 at 64 channels
+    const int npw = ((cin * 9 + 15) / 16 + 3) / 4;
+    auto pick = [&](auto mt) {
+        constexpr int MT = decltype(mt)::value;
+        if (npw <= 1)
+            go(conv_bwd_weight_kernel<MT, 1>);
+        else if (npw <= 3)
+            go(conv_bwd_weight_kernel<MT, 3>);
+        else if (npw <= 5)
+            go(conv_bwd_weight_kernel<MT, 5>);
+        else
+            go(conv_bwd_weight_kernel<MT, 9>);
+    };
+    if (cout <= 16)
+        pick(std::integral_constant<int, 1>());
+    else if (cout <= 32)
+        pick(std::integral_constant<int, 2>());
+    else
+        pick(std::integral_constant<int, 4>());
     check(hipGetLastError(), "conv backward-weight launch");
-    hipLaunchKernelGGL(reduce_chunks_kernel, dim3(unsigned((nw + 255) / 256)), dim3(256), 0, st, part, chunks, nw, dw);
-    hipLaunchKernelGGL(reduce_chunks_kernel, dim3(unsigned((cout + 255) / 256)), dim3(256), 0, st, partb, chunks, cout,
-                       db);
+    hipLaunchKernelGGL(reduce_chunks_kernel, dim3(unsigned((nw + 63) / 64 + (cout + 63) / 64)), dim3(NT), 0, st, part,
+                       partb, chunks, nw, cout, dw, db);
     check(hipGetLastError(), "conv gradient reduction launch");
 }
 

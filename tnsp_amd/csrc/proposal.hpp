@@ -9,8 +9,6 @@
 
 namespace tns {
 
-constexpr int CONV_CHUNK = 64;  // samples per workgroup of the weight gradient
-
 void launch_conv_fwd(const float* x, const uint16_t* w, const float* bias, float* y, int B, int cin, int cout, int H,
                      int W, int relu, hipStream_t st);
 void launch_conv_bwd_data(const float* dy, const float* relu_y, const uint16_t* w, float* dx, int B, int cin, int cout,
