@@ -69,6 +69,7 @@ struct SvdDev {
     int32_t m, n;
     int32_t max_sweeps;  // Jacobi sweep limit; a sector not converged by then gets NaN singular values
     int32_t pad1;
+    const int32_t* done;  // non-null: nothing to do where *done is set (the eigenvector path took the sector)
 };
 // default Jacobi sweep limit (the host can lower it to force the
 // non-convergence path in tests)
@@ -120,7 +121,32 @@ constexpr int64_t QR_LDS_MAX = LDS_CLASS[2];
 constexpr int64_t SVD_LDS_MAX = LDS_CLASS[2];
 // scratch of a QR / LQ task beyond LDS: the block and its taus
 inline int64_t qr_doubles(int64_t m, int64_t n) { return m * n + (m < n ? m : n); }
+// Sectors that go through the eigenvectors of their Gram matrix first
+// (svd_eig.hip).  Whole SVD passes with the Jacobi kernels alone and with this
+// path: 64 tensors with sectors up to about 200 x 190 (some beyond the register
+// kernel's 192 rows) 98.6 -> 4.8 ms; 4 tensors with sectors up to about
+// 310 x 260 199 -> 5.4 ms; one stage of 128 8x8 D=8 configurations (register
+// 24 / 16 and LDS kernels, one after the other) 11.1 -> 4.9 ms.  Below 32
+// columns a whole sector fits a few waves' LDS rounds and the path's ~25
+// launches cost more than they save; above 640 the eigenvector strips no
+// longer fit the registers of one wave.
+constexpr int SVD_EIG_MIN_COLS = 32, SVD_EIG_MAX_COLS = 640;
+inline bool svd_eig_fits(int64_t m, int64_t n) {
+    const int64_t mx = m > n ? m : n, kx = m < n ? m : n;
+    return kx >= SVD_EIG_MIN_COLS && kx <= SVD_EIG_MAX_COLS && mx * kx <= (int64_t(1) << 28);
+}
+// blocks of 16 reflectors of that path
+inline int64_t svd_eig_blocks(int64_t kx) { return (kx + 15) / 16; }
+// scratch of an SVD task: the Jacobi kernels' columns, V and singular values;
+// the eigenvector path's two column sets, four kx x kx matrices, the
+// tridiagonal form, the block reflectors' factors, the order and the flags
 inline int64_t svd_doubles(int64_t m, int64_t n) {
+    const int64_t mx = m > n ? m : n, kx = m < n ? m : n;
+    if (svd_eig_fits(m, n)) return 2 * mx * kx + 4 * kx * kx + 256 * svd_eig_blocks(kx) + 5 * kx + (kx + 1) / 2 + 2;
+    return mx * kx + kx * kx + kx;
+}
+// the Jacobi kernels' LDS working set
+inline int64_t svd_lds_doubles(int64_t m, int64_t n) {
     const int64_t mx = m > n ? m : n, kx = m < n ? m : n;
     return mx * kx + kx * kx + kx;
 }
@@ -135,6 +161,32 @@ constexpr int64_t QB_MAX_ROWS = (QB_LDS - 8 * (16 * 16 * 2 + 16 * 128 + 16)) / (
 // (rpt in {8, 16, 24}), V recovered from U; otherwise LDS (lds_bytes > 0)
 // or global scratch.
 void launch_svd(const SvdDev* tasks, int64_t num, int64_t lds_bytes, int rpt, int dtype, hipStream_t stream);
+
+// A sector on the eigenvector path.  Rows are contiguous: row c of xt is
+// column c of X.
+struct SvdEigDev {
+    SvdDev t;
+    double *xt, *xt2;         // kx x mx
+    double *b, *z, *s, *vt;   // kx x kx
+    double *tb;               // 16 x 16 per block of reflectors
+    double *de, *e, *tau;     // 2 kx (diagonal, squared off-diagonal), kx, kx
+    double *sig;              // kx
+    int32_t *order, *flags;   // kx; done, not for this path, scale exponent
+    int32_t mx, kx;
+};
+enum SvdEigStage {
+    SVD_EIG_LOAD,     // per task
+    SVD_EIG_TRIDIAG,  // per task; variant 0..2: at most 64 / 128 / 192 columns, 3: more
+    SVD_EIG_TFACTOR,  // per task and 16 columns (units)
+    SVD_EIG_VECTORS,  // per task and 64 columns (units)
+    SVD_EIG_BACK,     // per task and 64 columns (units); variant: 64 / 128 / 192 / 320 / 640 columns
+    SVD_EIG_POLISH,   // per task
+    SVD_EIG_REFINE,   // per task
+    SVD_EIG_ORDER,    // per task
+    SVD_EIG_WRITE     // per task and 32 columns (units)
+};
+void launch_svd_eig(int stage, int variant, const SvdEigDev* tasks, const TileDev* units, int64_t num, int dtype,
+                    hipStream_t stream);
 
 // Copy n_i doubles from src_i to dst + off_i for every task, one workgroup
 // per task: gathers the singular values of a batch of decompositions into

@@ -396,7 +396,151 @@ void Batch::svd(const std::vector<SvdTask>& ts, void* const* bufs, int64_t es, d
     }
 }
 
-void Batch::flush_svd() { flush_decomp(SVD, psvd_, psvd_cost_, SVD_LDS_MAX, svd_doubles); }
+// The eigenvector path over every sector it takes, largest first, as stages
+// of one launch each (products: one per tile variant); the Jacobi launches
+// that follow skip what it finished.
+void Batch::flush_svd_eig() {
+    std::vector<size_t> sel;
+    for (size_t i = 0; i < psvd_.size(); i++)
+        if (fast_svd_ && svd_eig_fits(psvd_[i].m, psvd_[i].n)) sel.push_back(i);
+    if (sel.empty()) return;
+    auto cols = [&](size_t i) { return std::min(psvd_[i].m, psvd_[i].n); };
+    std::stable_sort(sel.begin(), sel.end(), [&](size_t a, size_t b) { return cols(a) > cols(b); });
+    const size_t T = sel.size();
+    std::vector<SvdEigDev> tasks(T);
+    double units = 0;
+    for (size_t i = 0; i < T; i++) {
+        SvdDev& t = psvd_[sel[i]];
+        SvdEigDev& d = tasks[i];
+        const int64_t mx = std::max(t.m, t.n), kx = std::min(t.m, t.n);
+        d.mx = int32_t(mx);
+        d.kx = int32_t(kx);
+        double* cur = t.work;
+        auto take = [&](int64_t n) {
+            double* p = cur;
+            cur += n;
+            return p;
+        };
+        d.xt = take(mx * kx);
+        d.xt2 = take(mx * kx);
+        d.b = take(kx * kx);
+        d.z = take(kx * kx);
+        d.s = take(kx * kx);
+        d.vt = take(kx * kx);
+        d.tb = take(256 * svd_eig_blocks(kx));
+        d.de = take(2 * kx);
+        d.e = take(kx);
+        d.tau = take(kx);
+        d.sig = take(kx);
+        d.order = reinterpret_cast<int32_t*>(take((kx + 1) / 2));
+        d.flags = reinterpret_cast<int32_t*>(take(2));
+        if (cur != t.work + svd_doubles(t.m, t.n)) throw Error("internal: svd scratch layout");
+        t.done = d.flags;
+        d.t = t;
+        units += psvd_cost_[sel[i]];
+    }
+    const size_t toff = put(tasks);
+    auto stage = [&](int st, int variant, size_t first, const std::vector<TileDev>* list, int64_t num) {
+        Cmd c;
+        c.kind = SVD_EIG;
+        c.stage = st;
+        c.rpt = variant;
+        c.tasks = toff + first * sizeof(SvdEigDev);
+        c.prefix = list ? put(*list) : 0;
+        c.count = c.nwg = num;
+        cmds_.push_back(c);
+    };
+    // tasks are sorted by columns: the ranges with lo < columns <= hi
+    auto range = [&](int lo, int hi) {
+        size_t a = 0, b = 0;
+        while (a < T && tasks[a].kx > hi) a++;
+        b = a;
+        while (b < T && tasks[b].kx > lo) b++;
+        return std::pair<size_t, size_t>(a, b);
+    };
+    // one unit per `width` columns of tasks [a, b), numbered from `base`
+    auto list = [&](int width, size_t a, size_t b, size_t base) {
+        std::vector<TileDev> l;
+        for (size_t i = a; i < b; i++)
+            for (int j = 0; j * width < tasks[i].kx; j++) l.push_back(TileDev{int32_t(i - base), j, 0, 0});
+        return l;
+    };
+    // a product per task in the double kernels, whatever the batch's type
+    auto product = [&](auto fill) {
+        std::vector<GemmDev> g(T);
+        std::vector<TileDev> tiles[2];
+        for (size_t i = 0; i < T; i++) {
+            g[i].alpha = 1.0;
+            fill(tasks[i], g[i]);
+            const int v = std::max(g[i].m, g[i].n) <= 48 ? 0 : 1, w = GEMM_TILE_OF[v];
+            for (int x = 0; x * w < g[i].m; x++)
+                for (int y = 0; y * w < g[i].n; y++) tiles[v].push_back(TileDev{int32_t(i), x, y, 0});
+        }
+        const size_t goff = put(g);
+        for (int v = 0; v < 2; v++) {
+            if (tiles[v].empty()) continue;
+            Cmd c;
+            c.kind = GEMM;
+            c.stage = 0;
+            c.tasks = goff;
+            c.prefix = put(tiles[v]);
+            c.count = int64_t(T);
+            c.nwg = int64_t(tiles[v].size());
+            c.rpt = v;
+            c.dt = 0;
+            cmds_.push_back(c);
+        }
+    };
+    auto set = [](GemmDev& g, const double* a, int ta, int lda, const double* b, int tb, int ldb, double* c, int m, int n,
+                  int k) {
+        g.a = a;
+        g.ta = ta;
+        g.lda = lda;
+        g.b = b;
+        g.tb = tb;
+        g.ldb = ldb;
+        g.c = c;
+        g.ldc = n;
+        g.m = m;
+        g.n = n;
+        g.k = k;
+    };
+    const int64_t num = int64_t(T);
+    const size_t first_cmd = cmds_.size();
+    stage(SVD_EIG_LOAD, 0, 0, nullptr, num);
+    cmds_[first_cmd].units = units;
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.xt, 0, d.mx, d.xt, 1, d.mx, d.b, d.kx, d.kx, d.mx); });
+    static const int tri_hi[4] = {64, 128, 192, SVD_EIG_MAX_COLS};
+    for (int v = 3; v >= 0; v--) {
+        const auto [a, b] = range(v ? tri_hi[v - 1] : 0, tri_hi[v]);
+        if (b > a) stage(SVD_EIG_TRIDIAG, v, a, nullptr, int64_t(b - a));
+    }
+    const auto l16 = list(16, 0, T, 0), l64 = list(64, 0, T, 0), l32 = list(32, 0, T, 0);
+    stage(SVD_EIG_TFACTOR, 0, 0, &l16, int64_t(l16.size()));
+    stage(SVD_EIG_VECTORS, 0, 0, &l64, int64_t(l64.size()));
+    static const int back_hi[5] = {64, 128, 192, 320, SVD_EIG_MAX_COLS};
+    for (int v = 4; v >= 0; v--) {
+        const auto [a, b] = range(v ? back_hi[v - 1] : 0, back_hi[v]);
+        if (b <= a) continue;
+        const auto l = list(64, a, b, 0);
+        stage(SVD_EIG_BACK, v, 0, &l, int64_t(l.size()));
+    }
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.z, 1, d.kx, d.z, 0, d.kx, d.s, d.kx, d.kx, d.kx); });
+    stage(SVD_EIG_POLISH, 0, 0, nullptr, num);
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.s, 0, d.kx, d.z, 1, d.kx, d.vt, d.kx, d.kx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.vt, 0, d.kx, d.xt, 0, d.mx, d.xt2, d.kx, d.mx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.xt2, 0, d.mx, d.xt2, 1, d.mx, d.b, d.kx, d.kx, d.mx); });
+    stage(SVD_EIG_REFINE, 0, 0, nullptr, num);
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.b, 1, d.kx, d.xt2, 0, d.mx, d.xt, d.kx, d.mx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.b, 1, d.kx, d.vt, 0, d.kx, d.z, d.kx, d.kx, d.kx); });
+    stage(SVD_EIG_ORDER, 0, 0, nullptr, num);
+    stage(SVD_EIG_WRITE, 0, 0, &l32, int64_t(l32.size()));
+}
+
+void Batch::flush_svd() {
+    flush_svd_eig();
+    flush_decomp(SVD, psvd_, psvd_cost_, SVD_LDS_MAX, svd_lds_doubles);
+}
 
 void Batch::run(hipStream_t st) {
     flush_diag();
@@ -453,6 +597,10 @@ void Batch::run(hipStream_t st) {
             case QR:
                 launch_qr(reinterpret_cast<const QrDev*>(base + c.tasks), c.count, c.lds, c.rpt, dtype_, st);
                 break;
+            case SVD_EIG:
+                launch_svd_eig(c.stage, c.rpt, reinterpret_cast<const SvdEigDev*>(base + c.tasks),
+                               reinterpret_cast<const TileDev*>(base + c.prefix), c.count, dtype_, st);
+                break;
             case SVD:
                 launch_svd(reinterpret_cast<const SvdDev*>(base + c.tasks), c.count, c.lds, c.rpt, dtype_, st);
                 break;
@@ -461,6 +609,7 @@ void Batch::run(hipStream_t st) {
             check_hip(hipEventRecord(eb, st), "timer record");
             int k = int(c.kind);
             if (c.kind == QR && c.rpt == 1) k = KernelTimer::QR_BLOCKED;
+            if (c.stage >= 0) k = KernelTimer::SVD_EIG;
             if (c.kind == SVD && c.rpt == 8) k = KernelTimer::SVD_REG8;
             if (c.kind == SVD && c.rpt == 16) k = KernelTimer::SVD_REG16;
             if (c.kind == SVD && c.rpt == 24) k = KernelTimer::SVD_REG24;

@@ -60,7 +60,7 @@ class Staging {
 struct KernelTimer {
     // one entry per kernel (variant) so that launch averages compare with a
     // kernel trace: QR / SVD are the LDS and unblocked-global kernels
-    enum { PERM, FILL, GEMM, QR, SVD, DIAG, QR_BLOCKED, SVD_REG8, SVD_REG16, SVD_REG24, NKIND };
+    enum { PERM, FILL, GEMM, QR, SVD, DIAG, QR_BLOCKED, SVD_REG8, SVD_REG16, SVD_REG24, SVD_EIG, NKIND };
     struct Acc {
         double ms = 0, units = 0, launches = 0;
     } acc[NKIND];
@@ -136,7 +136,7 @@ class Batch {
     void set_fast_svd(bool on) { fast_svd_ = on; }
 
    private:
-    enum Kind { PERM, FILL, GEMM, QR, SVD, DIAG };
+    enum Kind { PERM, FILL, GEMM, QR, SVD, DIAG, SVD_EIG };
     struct Cmd {
         Kind kind;
         size_t tasks, prefix;  // blob offsets (prefix: GEMM tiles, permute / fill units)
@@ -146,13 +146,15 @@ class Batch {
         int rpt = 0;       // register tile of the large-block SVD kernel
         int dt = -1;       // element type / GEMM precision override (-1: batch dtype)
         int conv = 0;      // permute conversion (1: f64 -> f32, 2: f32 -> f64)
+        int stage = -1;    // stage of the eigenvector SVD (its products too: their time counts there)
     };
     template<typename D>
     void flush_decomp(Kind kind, std::vector<D>& tasks, std::vector<double>& cost, int64_t lds_max,
-                      int64_t (*doubles)(int64_t, int64_t));
+                      int64_t (*doubles)(int64_t, int64_t));  // doubles: the kernels' working set in LDS
     KernelTimer* timer_ = nullptr;
     Staging* staging_ = nullptr;
-    double pend_units_[6] = {0, 0, 0, 0, 0, 0};
+    double pend_units_[7] = {0, 0, 0, 0, 0, 0, 0};
+    void flush_svd_eig();
     template<typename T>
     size_t put(const std::vector<T>& v);
     void flush_flat(Kind kind, std::vector<PermDev>& pd, std::vector<FillDev>& fd);

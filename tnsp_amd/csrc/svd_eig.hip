@@ -1,0 +1,773 @@
+// Singular value decomposition of sector blocks through the eigenvectors of
+// their Gram matrix, with one exact refinement.
+//
+// X holds the kx = min(m, n) columns of the block (M or M^T) scaled by a power
+// of two, as in the Jacobi kernels.  The path
+//   B = X^T X                      (grouped GEMM)
+//   B = Q T Q^T                    (Householder tridiagonalisation)
+//   T Z = Z diag(lambda)           (bisection, twisted factorisations)
+//   V = Q Z, V <- V (3 - V^T V)/2  (block reflectors, one Newton-Schulz step)
+//   X' = X V, G = X'^T X'          (grouped GEMMs)
+//   X'' = X' (I + E), V'' = V (I + E),  E_ij = G_ij / (G_jj - G_ii)
+// leaves columns that are orthogonal to the tolerance of the Jacobi sweeps:
+// squaring costs X' some of its orthogonality (cosines up to eps s1^2 /
+// (si sj)), and I + E removes these cosines to first order, all pairs at once.
+// What it does not remove is below kx c^2 + e c + e^2 for cosines up to c and
+// row sums of |E| up to e; a block is taken only if both are at most
+// EIG_SMALL = 1e-8, which keeps that below half the sweeps' tolerance.  Any
+// other block (close singular values, rank deficiency, entries that are not
+// finite) is left to the Jacobi kernels, which run after this path and skip
+// the blocks marked done.  On 231 blocks of 40 to 190 columns of the 8x8 D=8
+// PEPS the cosines before the refinement were 1.4e-13 in the median and
+// 1.6e-8 at most, and 4e-16 at most after it.
+//
+// One-sided Jacobi does 10 to 14 sweeps of kx^2 / 2 rotations of length mx;
+// this path does about 14 kx^3 multiply-adds, most of them on the matrix
+// cores in launches that spread a block over many workgroups.  Times of both
+// stand at the routing rule (svd_eig_fits).
+#include "device.hpp"
+#include "kernels.hpp"
+
+#include <algorithm>
+#include <stdexcept>
+#include <string>
+
+namespace tns {
+
+namespace {
+
+// data written by an earlier kernel and read at uniform addresses: scalar loads
+typedef const __attribute__((address_space(4))) double* cptr;
+
+constexpr double EIG_SMALL = 1e-8;
+// row sums of |V^T V - 1| above which one Newton-Schulz step (which squares
+// the defect) does not reach rounding
+constexpr double EIG_DEFECT = 1e-7;
+
+inline void check(hipError_t e, const char* what) {
+    if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// ------------------------------------------------------------------- load
+// X (kx rows of mx, the columns of X one after the other) from the block,
+// scaled so that its largest entry lies in [1, 2).  32 x 32 tiles through LDS
+// where the block is stored the other way round, so that both sides coalesce.
+template<typename T>
+__global__ __launch_bounds__(1024) void eig_load_kernel(const SvdEigDev* __restrict__ tasks) {
+    const SvdEigDev tk = tasks[blockIdx.x];
+    __shared__ double wmax[16];
+    __shared__ double tile[32][33];
+    const gptr<const T> in = to_global(static_cast<const T*>(tk.t.in));
+    const gptr<double> xt = to_global(tk.xt);
+    const int tid = threadIdx.x, mx = tk.mx, kx = tk.kx;
+    double amax = 0.0;
+    bool fine = true;
+    for (int e = tid; e < mx * kx; e += 1024) {
+        const double x = fabs(double(in[e]));
+        fine = fine && x <= 1.79e308;
+        amax = fmax(amax, x);
+    }
+    amax = wave_max(amax);
+    if (tid % WAVE == 0) wmax[tid / WAVE] = amax;
+    fine = __syncthreads_and(fine);
+    for (int w = 0; w < 16; w++) amax = fmax(amax, wmax[w]);
+    const int ex = jacobi_scale_exponent(amax);
+    const double scl = ldexp(1.0, -ex);
+    if (tid == 0) {
+        tk.flags[0] = 0;                              // done
+        tk.flags[1] = (fine && amax > 0.0) ? 0 : 1;  // not for this path
+        tk.flags[2] = ex;
+    }
+    if (tk.t.m < tk.t.n) {
+        // M^T: row c of the block is column c of X
+        for (int e = tid; e < mx * kx; e += 1024) xt[e] = double(in[e]) * scl;
+        return;
+    }
+    const int ti = tid / 32, tj = tid % 32;
+    for (int r0 = 0; r0 < mx; r0 += 32) {
+        for (int c0 = 0; c0 < kx; c0 += 32) {
+            const int r = r0 + ti, c = c0 + tj;
+            if (r < mx && c < kx) tile[ti][tj] = double(in[r * kx + c]) * scl;
+            __syncthreads();
+            if (c0 + ti < kx && r0 + tj < mx) xt[(c0 + ti) * mx + r0 + tj] = tile[tj][ti];
+            __syncthreads();
+        }
+    }
+}
+
+// -------------------------------------------------------- tridiagonal form
+// What both versions write per step j: the diagonal, the off-diagonal entry
+// below it and its square (floored, so that the Sturm recurrence never meets
+// a split matrix), and the reflector v (zero up to j, one at j + 1) as row j
+// of `b`.
+struct TriOut {
+    gptr<double> de, e, tau;
+    double floor2;
+    __device__ void step(int j, int n, double d, double beta, double t) const {
+        de[2 * j] = d;
+        if (j == 0) de[1] = 0.0;
+        tau[j] = t;
+        if (j + 1 < n) {
+            e[j] = beta;
+            de[2 * j + 3] = fmax(beta * beta, floor2);
+        }
+    }
+};
+
+// Matrix in registers: thread (ti, tj) of TI x 16 holds rows ti + TI a and
+// columns tj + 16 b, a < A, b < BC.  Per column two barriers: row j (column j
+// by symmetry) goes to LDS, every wave forms the reflector from it; then
+// p = tau B v by partial rows and a sum over the 16 lanes of a row group, and
+// the rank-two update.  Bound by LDS reads of v and p (3 BC + 2 A values per
+// thread and step) and the chain of two barriers, one square root and one
+// division per step; a block of rows or columns already reduced is skipped.
+template<int TI, int A, int BC>
+__global__ __launch_bounds__(TI * 16) void eig_tridiag_kernel(const SvdEigDev* __restrict__ tasks) {
+    constexpr int N = TI * A > 16 * BC ? TI * A : 16 * BC, NW = TI * 16 / WAVE;
+    __shared__ double xs[2][N], ps[2][N], wtr[NW];
+    const SvdEigDev tk = tasks[blockIdx.x];
+    const int n = tk.kx, tid = threadIdx.x, lane = tid % WAVE, ti = tid / 16, tj = tid % 16;
+    if (n > TI * A || n > 16 * BC || tk.flags[1]) return;  // uniform over the workgroup
+    const gptr<double> B = to_global(tk.b);
+    double rb[A][BC];
+    double trace = 0.0;
+#pragma unroll
+    for (int a = 0; a < A; a++)
+#pragma unroll
+        for (int b = 0; b < BC; b++) {
+            const int r = ti + TI * a, c = tj + 16 * b;
+            rb[a][b] = (r < n && c < n) ? B[r * n + c] : 0.0;
+            if (r == c) trace += rb[a][b];
+        }
+    for (int i = tid; i < 2 * N; i += TI * 16) (&ps[0][0])[i] = 0.0;
+    trace = wave_sum(trace);
+    if (lane == 0) wtr[tid / WAVE] = trace;
+    __syncthreads();
+    trace = 0.0;
+    for (int w = 0; w < NW; w++) trace += wtr[w];
+    const TriOut out{to_global(tk.de), to_global(tk.e), to_global(tk.tau), 1e-40 * trace * trace};
+    for (int j = 0; j < n; j++) {
+        double* x = xs[j & 1];
+        double* p = ps[j & 1];
+#pragma unroll
+        for (int a = 0; a < A; a++)
+            if (j / TI == a && ti == j % TI) {
+#pragma unroll
+                for (int b = 0; b < BC; b++) x[tj + 16 * b] = rb[a][b];
+            }
+        __syncthreads();
+        double alpha = 0.0, sigma = 0.0;
+        if (j + 1 < n) {
+            alpha = x[j + 1];
+            double s = 0.0;
+            for (int i = j + 2 + lane; i < n; i += WAVE) s += x[i] * x[i];
+            sigma = wave_sum(s);
+        }
+        double tau, beta;
+        householder(alpha, sigma, tau, beta);
+        const double scale = tau != 0.0 ? 1.0 / (alpha - beta) : 0.0;
+        if (tid == 0) out.step(j, n, x[j], beta, tau);
+        if (tid < n) B[j * n + tid] = tid <= j ? 0.0 : (tid == j + 1 ? 1.0 : x[tid] * scale);
+        // the next step writes the other buffer, and the one after it waits
+        // for every wave to have left this step
+        if (tau == 0.0) continue;
+        double vc[BC];
+#pragma unroll
+        for (int b = 0; b < BC; b++) {
+            const int c = tj + 16 * b;
+            vc[b] = c <= j ? 0.0 : (c == j + 1 ? 1.0 : x[c] * scale);
+        }
+#pragma unroll
+        for (int a = 0; a < A; a++) {
+            if (TI * a + TI - 1 <= j) continue;
+            double s = 0.0;
+#pragma unroll
+            for (int b = 0; b < BC; b++)
+                if (16 * b + 15 > j) s += rb[a][b] * vc[b];
+            s = row_sum16(s);
+            if (tj == 0) p[ti + TI * a] = tau * s;
+        }
+        __syncthreads();
+        double s = 0.0;
+        for (int i = j + 1 + lane; i < n; i += WAVE) s += p[i] * (i == j + 1 ? 1.0 : x[i] * scale);
+        const double K = 0.5 * tau * wave_sum(s);
+        double wc[BC];
+#pragma unroll
+        for (int b = 0; b < BC; b++) {
+            const int c = tj + 16 * b;
+            wc[b] = c <= j ? 0.0 : p[c] - K * vc[b];
+        }
+#pragma unroll
+        for (int a = 0; a < A; a++) {
+            if (TI * a + TI - 1 <= j) continue;
+            const int r = ti + TI * a;
+            const double vr = r <= j ? 0.0 : (r == j + 1 ? 1.0 : x[r] * scale);
+            const double wr = r <= j ? 0.0 : p[r] - K * vr;
+#pragma unroll
+            for (int b = 0; b < BC; b++)
+                if (16 * b + 15 > j) rb[a][b] -= vr * wc[b] + wr * vc[b];
+        }
+    }
+}
+
+// Matrix in global memory (more columns than the registers hold): one pass
+// over the trailing matrix per step, which applies the previous step's
+// rank-two update, stores the result and multiplies it by the new reflector.
+// One wave per row, lane l holds columns l + 64 t.  Bound by those passes
+// (kx^3 16 / 3 bytes through the XCD's L2 by one workgroup).
+constexpr int TRI_GLB_T = (SVD_EIG_MAX_COLS + WAVE - 1) / WAVE;
+__global__ __launch_bounds__(1024) void eig_tridiag_glb_kernel(const SvdEigDev* __restrict__ tasks) {
+    __shared__ double xs[SVD_EIG_MAX_COLS], vs[SVD_EIG_MAX_COLS], ws[SVD_EIG_MAX_COLS], ps[SVD_EIG_MAX_COLS], red[16];
+    const SvdEigDev tk = tasks[blockIdx.x];
+    const int n = tk.kx, tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    if (n > SVD_EIG_MAX_COLS || tk.flags[1]) return;
+    // the trailing matrix is updated in place in `s`, the reflectors go to `b`
+    const gptr<double> B = to_global(tk.s), R = to_global(tk.b);
+    double trace = 0.0;
+    for (int r = wave; r < n; r += 16)
+        for (int c = lane; c < n; c += WAVE) {
+            const double v = R[r * n + c];
+            B[r * n + c] = v;
+            if (r == c) trace += v;
+        }
+    for (int i = tid; i < n; i += 1024) vs[i] = ws[i] = 0.0;
+    trace = wave_sum(trace);
+    if (lane == 0) red[wave] = trace;
+    __syncthreads();
+    trace = 0.0;
+    for (int w = 0; w < 16; w++) trace += red[w];
+    const TriOut out{to_global(tk.de), to_global(tk.e), to_global(tk.tau), 1e-40 * trace * trace};
+    for (int j = 0; j < n; j++) {
+        if (tid >= j && tid < n) xs[tid] = B[j * n + tid] - vs[j] * ws[tid] - ws[j] * vs[tid];
+        __syncthreads();
+        double alpha = 0.0, sigma = 0.0;
+        if (j + 1 < n) {
+            alpha = xs[j + 1];
+            double s = 0.0;
+            for (int i = j + 2 + lane; i < n; i += WAVE) s += xs[i] * xs[i];
+            sigma = wave_sum(s);
+        }
+        double tau, beta;
+        householder(alpha, sigma, tau, beta);
+        const double scale = tau != 0.0 ? 1.0 / (alpha - beta) : 0.0;
+        if (tid == 0) out.step(j, n, xs[j], beta, tau);
+        if (tid < n) R[j * n + tid] = tid <= j ? 0.0 : (tid == j + 1 ? 1.0 : xs[tid] * scale);
+        // v, w of the previous step and the new v at this lane's columns
+        double ov[TRI_GLB_T], ow[TRI_GLB_T], nv[TRI_GLB_T];
+#pragma unroll
+        for (int t = 0; t < TRI_GLB_T; t++) {
+            const int c = lane + WAVE * t;
+            const bool in = c < n && c > j;
+            ov[t] = in ? vs[c] : 0.0;
+            ow[t] = in ? ws[c] : 0.0;
+            nv[t] = in ? (c == j + 1 ? 1.0 : xs[c] * scale) : 0.0;
+        }
+        for (int r = j + 1 + wave; r < n; r += 16) {
+            const double vr = vs[r], wr = ws[r];
+            double s = 0.0;
+#pragma unroll
+            for (int t = 0; t < TRI_GLB_T; t++) {
+                if (WAVE * t >= n || WAVE * t + WAVE - 1 <= j) continue;
+                const int c = lane + WAVE * t;
+                if (c < n && c > j) {
+                    const double v = B[r * n + c] - vr * ow[t] - wr * ov[t];
+                    B[r * n + c] = v;
+                    s += v * nv[t];
+                }
+            }
+            s = wave_sum(s);
+            if (lane == 0) ps[r] = tau * s;
+        }
+        __syncthreads();
+        double s = 0.0;
+        for (int i = j + 1 + lane; i < n; i += WAVE) s += ps[i] * (i == j + 1 ? 1.0 : xs[i] * scale);
+        const double K = 0.5 * tau * wave_sum(s);
+        // every wave has read the old v, w (before the barrier above) and the
+        // sums above read ps and xs only
+        for (int i = tid; i < n; i += 1024) {
+            const double v = i <= j ? 0.0 : (i == j + 1 ? 1.0 : xs[i] * scale);
+            vs[i] = v;
+            ws[i] = i <= j ? 0.0 : ps[i] - K * v;
+        }
+        __syncthreads();
+    }
+}
+
+// T (16 x 16, upper) of the block reflectors of 16 consecutive columns,
+// H = I - V T V^T (forward, columnwise): the Gram matrix of the reflectors on
+// the fp64 MFMA, then the recurrence, one lane per row.  One wave per block.
+__global__ __launch_bounds__(64) void eig_tfactor_kernel(const SvdEigDev* __restrict__ tasks,
+                                                        const TileDev* __restrict__ units) {
+    __shared__ double Gm[16][17], Tm[16][17];
+    const SvdEigDev tk = tasks[units[blockIdx.x].task];
+    const int blk = units[blockIdx.x].tm, n = tk.kx, lane = threadIdx.x, lm = lane % 16, lk = lane / 16;
+    if (tk.flags[1]) return;
+    const gptr<const double> R = to_global(tk.b);
+    const int j = 16 * blk + lm;
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int r0 = 16 * blk; r0 < n; r0 += 4) {
+        const int r = r0 + lk;
+        const double v = (j < n && r < n) ? R[j * n + r] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, v, acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) Gm[lk + 4 * i][lm] = acc[i];
+    __syncthreads();
+    if (lane < 16) {
+        for (int i = 0; i < 16; i++) {
+            const int col = 16 * blk + i;
+            const double ti = col < n ? tk.tau[col] : 0.0;
+            double v = 0.0;
+            if (i == lane) {
+                v = ti;
+            } else if (i > lane) {
+                double s = 0.0;
+                for (int l = lane; l < i; l++) s += Tm[lane][l] * Gm[l][i];
+                v = -ti * s;
+            }
+            Tm[lane][i] = v;
+        }
+    }
+    __syncthreads();
+    const gptr<double> out = to_global(tk.tb) + 256 * blk;
+#pragma unroll
+    for (int i = 0; i < 4; i++) out[(lk + 4 * i) * 16 + lm] = Tm[lk + 4 * i][lm];
+}
+
+// ------------------------------------------------ eigenvalues and -vectors
+// Number of eigenvalues of T below x: sign changes of the leading minors,
+// rescaled every four steps.
+__device__ inline int sturm_count(cptr de, int n, double x) {
+    double p0 = 1.0, p1 = de[0] - x;
+    bool neg = p1 < 0.0;
+    int c = neg;
+    int i = 1;
+    auto step = [&](int q) __attribute__((always_inline)) {
+        const double p2 = (de[2 * q] - x) * p1 - de[2 * q + 1] * p0;
+        const bool ng = p2 < 0.0;
+        c += ng != neg;
+        neg = ng;
+        p0 = p1;
+        p1 = p2;
+    };
+    for (; i + 4 <= n; i += 4) {
+        step(i);
+        step(i + 1);
+        step(i + 2);
+        step(i + 3);
+        const int e = __builtin_amdgcn_frexp_exp(fmax(fabs(p0), fabs(p1)));
+        p0 = __builtin_amdgcn_ldexp(p0, -e);
+        p1 = __builtin_amdgcn_ldexp(p1, -e);
+    }
+    for (; i < n; i++) step(i);
+    return c;
+}
+
+// 64 eigenvalues and eigenvectors of T per workgroup, one per lane.
+// Eigenvalues: each step splits the intervals in five, one Sturm count per
+// wave (24 steps, 5^24 > 2^55).  Vectors: the twisted factorisation of
+// T - lambda (forward by wave 0, backward by wave 1 at the same time), the
+// twist where its pivot is smallest, and the two back substitutions.  Every
+// lane runs a serial chain of kx steps, so the time is their latency; the
+// factors pass through global memory, lanes side by side.
+// Eigenvectors of close eigenvalues come out less orthogonal; the caller
+// measures and refines them.
+__global__ __launch_bounds__(256) void eig_vectors_kernel(const SvdEigDev* __restrict__ tasks,
+                                                         const TileDev* __restrict__ units) {
+    __shared__ int cnt[4][64], gi[4][64];
+    __shared__ double gm[4][64];
+    const SvdEigDev tk = tasks[units[blockIdx.x].task];
+    const int n = tk.kx, lane = threadIdx.x % WAVE, w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / WAVE);
+    if (tk.flags[1]) return;
+    const int k = 64 * units[blockIdx.x].tm + lane, kk = min(k, n - 1);
+    const cptr de = (cptr)(tk.de), ee = (cptr)(tk.e);
+    double lo = 0.0, hi = 0.0;
+    {
+        double a = -1e308, b = -1e308;
+        for (int i = lane; i < n; i += WAVE) {
+            const double r = (i > 0 ? fabs(tk.e[i - 1]) : 0.0) + (i + 1 < n ? fabs(tk.e[i]) : 0.0);
+            a = fmax(a, tk.de[2 * i] + r);
+            b = fmax(b, r - tk.de[2 * i]);
+        }
+        hi = wave_max(a);
+        lo = -wave_max(b);
+        const double pad = 1e-14 * fmax(fabs(lo), fabs(hi));
+        hi += pad;
+        lo -= pad;
+    }
+    const double pivmin = 1e-32 * (hi - lo);
+    for (int it = 0; it < 24; it++) {
+        const double h = (hi - lo) * 0.2;
+        cnt[w][lane] = sturm_count(de, n, lo + h * (w + 1));
+        __syncthreads();
+        const double base = lo;
+        double nlo = lo, nhi = hi;
+#pragma unroll
+        for (int s = 3; s >= 0; s--)
+            if (cnt[s][lane] > kk) nhi = base + h * (s + 1);
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+            if (cnt[s][lane] <= kk) nlo = base + h * (s + 1);
+        lo = nlo;
+        hi = nhi;
+        __syncthreads();
+    }
+    const double lam = 0.5 * (lo + hi);
+    const gptr<double> Lp = to_global(tk.s), Lm = to_global(tk.vt), Z = to_global(tk.z);
+    auto inv = [&](double q) __attribute__((always_inline)) {
+        return refined_rcp(fabs(q) < pivmin ? copysign(pivmin, q) : q);
+    };
+    if (w == 0) {
+        double q = de[0] - lam;
+        for (int i = 0; i + 1 < n; i++) {
+            const double l = ee[i] * inv(q);
+            if (k < n) Lp[i * n + k] = l;
+            q = de[2 * i + 2] - lam - ee[i] * l;
+        }
+    } else if (w == 1) {
+        double q = de[2 * n - 2] - lam;
+        for (int i = n - 2; i >= 0; i--) {
+            const double l = ee[i] * inv(q);
+            if (k < n) Lm[(i + 1) * n + k] = l;
+            q = de[2 * i] - lam - ee[i] * l;
+        }
+    }
+    __syncthreads();
+    {
+        double best = 1e308;
+        int at = n * w / 4;
+        for (int i = n * w / 4; i < n * (w + 1) / 4; i++) {
+            double g = de[2 * i] - lam;
+            if (k < n) {
+                if (i > 0) g -= ee[i - 1] * Lp[(i - 1) * n + k];
+                if (i + 1 < n) g -= ee[i] * Lm[(i + 1) * n + k];
+            }
+            if (fabs(g) < best) {
+                best = fabs(g);
+                at = i;
+            }
+        }
+        gm[w][lane] = best;
+        gi[w][lane] = at;
+    }
+    __syncthreads();
+    int r = gi[0][lane];
+    {
+        double best = gm[0][lane];
+#pragma unroll
+        for (int v = 1; v < 4; v++)
+            if (gm[v][lane] < best) {
+                best = gm[v][lane];
+                r = gi[v][lane];
+            }
+    }
+    __syncthreads();
+    double ss = 0.0;
+    if (w == 0 && k < n) {
+        double z = 1.0;
+        Z[r * n + k] = 1.0;
+#pragma unroll 4
+        for (int i = n - 2; i >= 0; i--) {
+            const double l = Lp[i * n + k];
+            if (i < r) {
+                z = -l * z;
+                ss += z * z;
+                Z[i * n + k] = z;
+            }
+        }
+    } else if (w == 1 && k < n) {
+        double z = 1.0;
+#pragma unroll 4
+        for (int i = 1; i < n; i++) {
+            const double l = Lm[i * n + k];
+            if (i > r) {
+                z = -l * z;
+                ss += z * z;
+                Z[i * n + k] = z;
+            }
+        }
+    }
+    gm[w][lane] = ss;
+    __syncthreads();
+    const double f = refined_rsqrt(1.0 + gm[0][lane] + gm[1][lane]);
+    if (k < n)
+        for (int i = w; i < n; i += 4) Z[i * n + k] *= f;
+}
+
+// V = Q Z: the block reflectors, last first, applied to strips of 16 columns
+// of Z, one strip per wave, in registers.  A strip's row tile t, register i,
+// lane l holds row 16 t + 4 i + l / 16, column l % 16: the accumulator layout
+// of the fp64 MFMA is also its B operand layout for the four rows of step i,
+// so W = V^T Z and T W feed the next product without moving.  V's rows sit in
+// LDS with a stride of 17, which both operand reads cross without conflicts.
+template<int TILES>
+__global__ __launch_bounds__(256) void eig_back_kernel(const SvdEigDev* __restrict__ tasks,
+                                                      const TileDev* __restrict__ units) {
+    extern __shared__ double lds[];
+    const SvdEigDev tk = tasks[units[blockIdx.x].task];
+    const int n = tk.kx, tid = threadIdx.x, lane = tid % WAVE, lm = lane % 16, lk = lane / 16;
+    if (n > 16 * TILES || tk.flags[1]) return;
+    double* Vs = lds;                      // 16 TILES rows of stride 17
+    double* Ts = lds + 16 * TILES * 17;    // 16 x 17
+    const int c = 64 * units[blockIdx.x].tm + 16 * (tid / WAVE) + lm;
+    const gptr<double> Z = to_global(tk.z);
+    const gptr<const double> R = to_global(tk.b), Tb = to_global(tk.tb);
+    d4 z[TILES];
+#pragma unroll
+    for (int t = 0; t < TILES; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = 16 * t + 4 * i + lk;
+            z[t][i] = (r < n && c < n) ? Z[r * n + c] : 0.0;
+        }
+    for (int blk = (n - 1) / 16; blk >= 0; blk--) {
+        __syncthreads();
+        for (int e = tid; e < 16 * 16 * TILES; e += 256) {
+            const int jj = e / (16 * TILES), i = e % (16 * TILES), j = 16 * blk + jj;
+            Vs[i * 17 + jj] = (j < n && i < n && i > j) ? R[j * n + i] : 0.0;
+        }
+        Ts[(tid / 16) * 17 + tid % 16] = Tb[256 * blk + tid];
+        __syncthreads();
+        d4 wv = {0.0, 0.0, 0.0, 0.0}, wv2 = wv;
+#pragma unroll
+        for (int t = 0; t < TILES; t++) {
+            if (t < blk || 16 * t >= n) continue;
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+                wv = __builtin_amdgcn_mfma_f64_16x16x4f64(Vs[(16 * t + 4 * i + lk) * 17 + lm], z[t][i], wv, 0, 0, 0);
+                wv2 = __builtin_amdgcn_mfma_f64_16x16x4f64(Vs[(16 * t + 4 * i + 4 + lk) * 17 + lm], z[t][i + 1], wv2, 0,
+                                                           0, 0);
+            }
+        }
+        wv += wv2;
+        d4 tw = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            tw = __builtin_amdgcn_mfma_f64_16x16x4f64(Ts[lm * 17 + 4 * i + lk], wv[i], tw, 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < TILES; t++) {
+            if (t < blk || 16 * t >= n) continue;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                z[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-Vs[(16 * t + lm) * 17 + 4 * i + lk], tw[i], z[t], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < TILES; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int r = 16 * t + 4 * i + lk;
+            if (r < n && c < n) Z[r * n + c] = z[t][i];
+        }
+}
+
+// --------------------------------------------------- checks and corrections
+// s <- (3 - s) / 2 for s = V^T V, after measuring its distance from one
+__global__ __launch_bounds__(1024) void eig_polish_kernel(const SvdEigDev* __restrict__ tasks) {
+    const SvdEigDev tk = tasks[blockIdx.x];
+    const int n = tk.kx, lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    if (tk.flags[1]) return;
+    const gptr<double> S = to_global(tk.s);
+    bool fine = true;
+    for (int r = wave; r < n; r += 16) {
+        double sum = 0.0;
+        for (int c = lane; c < n; c += WAVE) {
+            const double v = S[r * n + c], one = r == c ? 1.0 : 0.0;
+            sum += fabs(v - one);
+            S[r * n + c] = 1.5 * one - 0.5 * v;
+        }
+        fine = fine && wave_sum(sum) <= EIG_DEFECT;  // false for NaN
+    }
+    if (!__syncthreads_and(fine) && threadIdx.x == 0) tk.flags[1] = 1;
+}
+
+// b <- I + E from b = G = X'^T X', with the pair rules of the Jacobi sweeps
+// (cosines at most tol are left alone), after the checks that decide whether
+// the block is this path's
+__global__ __launch_bounds__(1024) void eig_refine_kernel(const SvdEigDev* __restrict__ tasks) {
+    __shared__ double d[SVD_EIG_MAX_COLS], root[SVD_EIG_MAX_COLS], red[16];
+    const SvdEigDev tk = tasks[blockIdx.x];
+    const int n = tk.kx, tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    if (n > SVD_EIG_MAX_COLS || tk.flags[1]) return;
+    const gptr<double> G = to_global(tk.b);
+    double fro = 0.0;
+    for (int i = tid; i < n; i += 1024) {
+        const double v = G[i * n + i];
+        d[i] = v;
+        root[i] = sqrt(v);
+        fro += v;
+    }
+    fro = wave_sum(fro);
+    if (lane == 0) red[wave] = fro;
+    __syncthreads();
+    fro = 0.0;
+    for (int w = 0; w < 16; w++) fro += red[w];
+    const double live = fmax(JACOBI_QUIET, JACOBI_DEAD2 * fro);
+    const double tol = fmax(1e-15, 2.220446049250313e-16 * tk.mx);
+    bool fine = true;
+    for (int r = wave; r < n; r += 16) {
+        const double dr = d[r], rr = root[r];
+        double sum = 0.0;
+        for (int c = lane; c < n; c += WAVE) {
+            const double g = G[r * n + c], scale = rr * root[c];
+            double e = 1.0;
+            if (c != r) {
+                e = 0.0;
+                if (!(fabs(g) <= tol * scale)) {
+                    e = g / (d[c] - dr);
+                    fine = fine && fabs(g) <= EIG_SMALL * scale;
+                }
+                sum += fabs(e);
+            }
+            G[r * n + c] = e;
+        }
+        fine = fine && wave_sum(sum) <= EIG_SMALL && dr > live;
+    }
+    if (!__syncthreads_and(fine) && tid == 0) tk.flags[1] = 1;
+}
+
+// Singular values (column norms), their descending order (ties by column)
+// and the mark that takes the block from the Jacobi kernels
+__global__ __launch_bounds__(256) void eig_order_kernel(const SvdEigDev* __restrict__ tasks) {
+    __shared__ double sg[SVD_EIG_MAX_COLS];
+    const SvdEigDev tk = tasks[blockIdx.x];
+    const int n = tk.kx, mx = tk.mx, tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    if (n > SVD_EIG_MAX_COLS || tk.flags[1]) return;
+    const gptr<const double> X = to_global(tk.xt);
+    bool fine = true;
+    for (int c = wave; c < n; c += 4) {
+        double s = 0.0;
+        for (int r = lane; r < mx; r += WAVE) s += X[c * mx + r] * X[c * mx + r];
+        s = wave_sum(s);
+        fine = fine && s > 0.0 && s < 1e300;
+        if (lane == 0) sg[c] = sqrt(s);
+    }
+    if (!__syncthreads_and(fine)) return;
+    for (int c = tid; c < n; c += 256) {
+        const double sc = sg[c];
+        int rank = 0;
+        for (int q = 0; q < n; q++) rank += (sg[q] > sc) || (sg[q] == sc && q < c);
+        tk.order[rank] = c;
+        tk.sig[rank] = sc;
+        tk.t.s[rank] = ldexp(sc, tk.flags[2]);
+    }
+    if (tid == 0) tk.flags[0] = 1;
+}
+
+// U and V^T of the block from the columns of X and V in rank order, 32 ranks
+// per workgroup; the factor stored column by column goes through LDS tiles.
+template<typename T>
+__global__ __launch_bounds__(256) void eig_write_kernel(const SvdEigDev* __restrict__ tasks,
+                                                       const TileDev* __restrict__ units) {
+    __shared__ double tile[32][33];
+    const SvdEigDev tk = tasks[units[blockIdx.x].task];
+    if (!tk.flags[0]) return;
+    const int n = tk.kx, r0 = 32 * units[blockIdx.x].tm, tx = threadIdx.x % 32, ty = threadIdx.x / 32;
+    const bool trans = tk.t.m < tk.t.n;
+    const gptr<const double> X = to_global(tk.xt), V = to_global(tk.z), sig = to_global(tk.sig);
+    const gptr<const int32_t> order = to_global(tk.order);
+    const gptr<T> U = to_global(static_cast<T*>(tk.t.u)), Vo = to_global(static_cast<T*>(tk.t.v));
+    // rows: the columns of X (m < n) or V, as rows of V^T; cols: the others,
+    // as columns of U
+    const gptr<const double> rows = trans ? X : V, cols = trans ? V : X;
+    const int rl = trans ? tk.mx : n, cl = trans ? n : tk.mx;
+    for (int q = ty; q < 32; q += 8) {
+        const int rank = r0 + q;
+        if (rank >= n) break;
+        const double f = trans ? 1.0 / sig[rank] : 1.0;
+        const gptr<const double> p = rows + int64_t(order[rank]) * rl;
+        for (int i = tx; i < rl; i += 32) Vo[int64_t(rank) * rl + i] = T(p[i] * f);
+    }
+    for (int i0 = 0; i0 < cl; i0 += 32) {
+        for (int q = ty; q < 32; q += 8) {
+            const int rank = r0 + q;
+            if (rank < n && i0 + tx < cl)
+                tile[q][tx] = cols[int64_t(order[rank]) * cl + i0 + tx] * (trans ? 1.0 : 1.0 / sig[rank]);
+        }
+        __syncthreads();
+        for (int q = ty; q < 32; q += 8)
+            if (i0 + q < cl && r0 + tx < n) U[int64_t(i0 + q) * n + r0 + tx] = T(tile[tx][q]);
+        __syncthreads();
+    }
+}
+
+}  // namespace
+
+namespace {
+template<int TILES>
+void launch_back(const SvdEigDev* tasks, const TileDev* units, dim3 grid, hipStream_t st) {
+    constexpr int lds = (16 * TILES * 17 + 16 * 17) * int(sizeof(double));
+    // once per kernel and process: the static's initialisation is thread-safe
+    static const bool allowed = [] {
+        if (lds > 64 * 1024)
+            check(hipFuncSetAttribute(reinterpret_cast<const void*>(eig_back_kernel<TILES>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, lds),
+                  "dynamic LDS attribute");
+        return true;
+    }();
+    (void)allowed;
+    hipLaunchKernelGGL(eig_back_kernel<TILES>, grid, dim3(256), size_t(lds), st, tasks, units);
+}
+}  // namespace
+
+void launch_svd_eig(int stage, int variant, const SvdEigDev* tasks, const TileDev* units, int64_t num, int dtype,
+                    hipStream_t st) {
+    if (num <= 0) return;
+    const dim3 grid(static_cast<unsigned>(num));
+    switch (stage) {
+        case SVD_EIG_LOAD:
+            if (dtype == 0)
+                hipLaunchKernelGGL(eig_load_kernel<double>, grid, dim3(1024), 0, st, tasks);
+            else
+                hipLaunchKernelGGL(eig_load_kernel<float>, grid, dim3(1024), 0, st, tasks);
+            break;
+        case SVD_EIG_TRIDIAG:
+            if (variant == 0)
+                hipLaunchKernelGGL((eig_tridiag_kernel<16, 4, 4>), grid, dim3(256), 0, st, tasks);
+            else if (variant == 1)
+                hipLaunchKernelGGL((eig_tridiag_kernel<32, 4, 8>), grid, dim3(512), 0, st, tasks);
+            else if (variant == 2)
+                hipLaunchKernelGGL((eig_tridiag_kernel<48, 4, 12>), grid, dim3(768), 0, st, tasks);
+            else
+                hipLaunchKernelGGL(eig_tridiag_glb_kernel, grid, dim3(1024), 0, st, tasks);
+            break;
+        case SVD_EIG_TFACTOR:
+            hipLaunchKernelGGL(eig_tfactor_kernel, grid, dim3(64), 0, st, tasks, units);
+            break;
+        case SVD_EIG_VECTORS:
+            hipLaunchKernelGGL(eig_vectors_kernel, grid, dim3(256), 0, st, tasks, units);
+            break;
+        case SVD_EIG_BACK:
+            if (variant == 0)
+                launch_back<4>(tasks, units, grid, st);
+            else if (variant == 1)
+                launch_back<8>(tasks, units, grid, st);
+            else if (variant == 2)
+                launch_back<12>(tasks, units, grid, st);
+            else if (variant == 3)
+                launch_back<20>(tasks, units, grid, st);
+            else
+                launch_back<SVD_EIG_MAX_COLS / 16>(tasks, units, grid, st);
+            break;
+        case SVD_EIG_POLISH:
+            hipLaunchKernelGGL(eig_polish_kernel, grid, dim3(1024), 0, st, tasks);
+            break;
+        case SVD_EIG_REFINE:
+            hipLaunchKernelGGL(eig_refine_kernel, grid, dim3(1024), 0, st, tasks);
+            break;
+        case SVD_EIG_ORDER:
+            hipLaunchKernelGGL(eig_order_kernel, grid, dim3(256), 0, st, tasks);
+            break;
+        case SVD_EIG_WRITE:
+            if (dtype == 0)
+                hipLaunchKernelGGL(eig_write_kernel<double>, grid, dim3(256), 0, st, tasks, units);
+            else
+                hipLaunchKernelGGL(eig_write_kernel<float>, grid, dim3(256), 0, st, tasks, units);
+            break;
+        default:
+            throw std::runtime_error("svd: unknown stage");
+    }
+    check(hipGetLastError(), "svd eigenvector stage launch");
+}
+
+}  // namespace tns
