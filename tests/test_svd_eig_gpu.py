@@ -104,3 +104,19 @@ def test_batch_of_mixed_sectors():
         r1 = gu.contract(gs, {("cu", "su")}).contract(gv, {("sv", "cv")})
         r0 = u.contract(s, {("cu", "su")}).contract(v, {("sv", "cv")})
         assert np.linalg.norm(r1.storage.numpy() - r0.data) <= 1e-12 * np.linalg.norm(r0.data)
+
+
+@pytest.mark.parametrize("m,n,null", [(135, 47, 1), (64, 64, 2), (200, 210, 3), (48, 90, 8), (40, 40, 9)])
+def test_null_columns_are_completed(m, n, null):
+    """A few zero singular values: U and V^T stay orthonormal."""
+    rng = np.random.default_rng(m + n + null)
+    u, s, v = np.linalg.svd(rng.standard_normal((m, n)), full_matrices=False)
+    s[len(s) - null:] = 0.0
+    x = (u * s) @ v
+    gu, gs, gv = dense_svd(x, "D")
+    tol = 4 * max(m, n) * EPS["D"]
+    assert np.max(np.abs(gs - np.linalg.svd(x, compute_uv=False)[:len(gs)])) <= tol * s[0]
+    assert np.linalg.norm((gu * gs) @ gv - x) <= tol * np.linalg.norm(x)
+    if null == 1:
+        assert np.max(np.abs(gu.T @ gu - np.eye(len(gs)))) <= tol
+        assert np.max(np.abs(gv @ gv.T - np.eye(len(gs)))) <= tol

@@ -185,6 +185,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const GemmDev* __res
     __shared__ T Bs[2][KB][TN + 1];
     const TileDev tile = tiles[blockIdx.x];
     const GemmDev g = tasks[tile.task];
+    if (g.skip && *g.skip) return;
     const gptr<const T> A = to_global(static_cast<const T*>(g.a));
     const gptr<const T> B = to_global(static_cast<const T*>(g.b));
     const int row0 = tile.tm * TM, col0 = tile.tn * TN;

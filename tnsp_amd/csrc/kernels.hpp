@@ -41,6 +41,7 @@ struct GemmDev {
     void* c;
     int32_t m, n, k, lda, ldb, ldc, ta, tb;
     double alpha;
+    const int32_t* skip;  // non-null: nothing to do where *skip is set
 };
 
 struct TileDev {
@@ -126,11 +127,12 @@ inline int64_t qr_doubles(int64_t m, int64_t n) { return m * n + (m < n ? m : n)
 // path: 64 tensors with sectors up to about 200 x 190 (some beyond the register
 // kernel's 192 rows) 98.6 -> 4.8 ms; 4 tensors with sectors up to about
 // 310 x 260 199 -> 5.4 ms; one stage of 128 8x8 D=8 configurations (register
-// 24 / 16 and LDS kernels, one after the other) 11.1 -> 4.9 ms.  Below 32
-// columns a whole sector fits a few waves' LDS rounds and the path's ~25
-// launches cost more than they save; above 640 the eigenvector strips no
-// longer fit the registers of one wave.
-constexpr int SVD_EIG_MIN_COLS = 32, SVD_EIG_MAX_COLS = 640;
+// 24 / 16 and LDS kernels, one after the other) 11.1 -> 4.9 ms.  Sectors of 16
+// to 31 columns ride along with larger ones (the LDS kernel's launch then takes
+// 198 instead of 294 us per stage of those configurations); alone, the path's
+// ~25 launches cost more than the LDS kernel's rounds.  Above 640 columns the
+// eigenvector strips no longer fit the registers of one wave.
+constexpr int SVD_EIG_MIN_COLS = 16, SVD_EIG_ALONE_COLS = 32, SVD_EIG_MAX_COLS = 640;
 inline bool svd_eig_fits(int64_t m, int64_t n) {
     const int64_t mx = m > n ? m : n, kx = m < n ? m : n;
     return kx >= SVD_EIG_MIN_COLS && kx <= SVD_EIG_MAX_COLS && mx * kx <= (int64_t(1) << 28);
@@ -170,18 +172,20 @@ struct SvdEigDev {
     double *b, *z, *s, *vt;   // kx x kx
     double *tb;               // 16 x 16 per block of reflectors
     double *de, *e, *tau;     // 2 kx (diagonal, squared off-diagonal), kx, kx
-    double *sig;              // kx
-    int32_t *order, *flags;   // kx; done, not for this path, scale exponent
+    double *sig;              // kx: reciprocal column norms in rank order
+    int32_t *order, *flags;   // kx; done, not for this path, scale exponent, first form of the step
     int32_t mx, kx;
 };
 enum SvdEigStage {
     SVD_EIG_LOAD,     // per task
-    SVD_EIG_TRIDIAG,  // per task; variant 0..2: at most 64 / 128 / 192 columns, 3: more
+    SVD_EIG_TRIDIAG,  // per task; variant 0..4: at most 64 / 128 / 192 / 320 / 640 columns
     SVD_EIG_TFACTOR,  // per task and 16 columns (units)
     SVD_EIG_VECTORS,  // per task and 64 columns (units)
     SVD_EIG_BACK,     // per task and 64 columns (units); variant: 64 / 128 / 192 / 320 / 640 columns
     SVD_EIG_POLISH,   // per task
     SVD_EIG_REFINE,   // per task
+    SVD_EIG_SECOND,   // per task
+    SVD_EIG_VERIFY,   // per task
     SVD_EIG_ORDER,    // per task
     SVD_EIG_WRITE     // per task and 32 columns (units)
 };

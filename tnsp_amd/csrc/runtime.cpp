@@ -403,9 +403,9 @@ void Batch::flush_svd_eig() {
     std::vector<size_t> sel;
     for (size_t i = 0; i < psvd_.size(); i++)
         if (fast_svd_ && svd_eig_fits(psvd_[i].m, psvd_[i].n)) sel.push_back(i);
-    if (sel.empty()) return;
     auto cols = [&](size_t i) { return std::min(psvd_[i].m, psvd_[i].n); };
     std::stable_sort(sel.begin(), sel.end(), [&](size_t a, size_t b) { return cols(a) > cols(b); });
+    if (sel.empty() || cols(sel[0]) < SVD_EIG_ALONE_COLS) return;
     const size_t T = sel.size();
     std::vector<SvdEigDev> tasks(T);
     double units = 0;
@@ -510,17 +510,16 @@ void Batch::flush_svd_eig() {
     stage(SVD_EIG_LOAD, 0, 0, nullptr, num);
     cmds_[first_cmd].units = units;
     product([&](SvdEigDev& d, GemmDev& g) { set(g, d.xt, 0, d.mx, d.xt, 1, d.mx, d.b, d.kx, d.kx, d.mx); });
-    static const int tri_hi[4] = {64, 128, 192, SVD_EIG_MAX_COLS};
-    for (int v = 3; v >= 0; v--) {
-        const auto [a, b] = range(v ? tri_hi[v - 1] : 0, tri_hi[v]);
+    static const int hi[5] = {64, 128, 192, 320, SVD_EIG_MAX_COLS};
+    for (int v = 4; v >= 0; v--) {
+        const auto [a, b] = range(v ? hi[v - 1] : 0, hi[v]);
         if (b > a) stage(SVD_EIG_TRIDIAG, v, a, nullptr, int64_t(b - a));
     }
     const auto l16 = list(16, 0, T, 0), l64 = list(64, 0, T, 0), l32 = list(32, 0, T, 0);
     stage(SVD_EIG_TFACTOR, 0, 0, &l16, int64_t(l16.size()));
     stage(SVD_EIG_VECTORS, 0, 0, &l64, int64_t(l64.size()));
-    static const int back_hi[5] = {64, 128, 192, 320, SVD_EIG_MAX_COLS};
     for (int v = 4; v >= 0; v--) {
-        const auto [a, b] = range(v ? back_hi[v - 1] : 0, back_hi[v]);
+        const auto [a, b] = range(v ? hi[v - 1] : 0, hi[v]);
         if (b <= a) continue;
         const auto l = list(64, a, b, 0);
         stage(SVD_EIG_BACK, v, 0, &l, int64_t(l.size()));
@@ -531,8 +530,18 @@ void Batch::flush_svd_eig() {
     product([&](SvdEigDev& d, GemmDev& g) { set(g, d.vt, 0, d.kx, d.xt, 0, d.mx, d.xt2, d.kx, d.mx, d.kx); });
     product([&](SvdEigDev& d, GemmDev& g) { set(g, d.xt2, 0, d.mx, d.xt2, 1, d.mx, d.b, d.kx, d.kx, d.mx); });
     stage(SVD_EIG_REFINE, 0, 0, nullptr, num);
+    product([&](SvdEigDev& d, GemmDev& g) {
+        set(g, d.b, 0, d.kx, d.b, 0, d.kx, d.s, d.kx, d.kx, d.kx);
+        g.skip = d.flags + 3;
+    });
+    stage(SVD_EIG_SECOND, 0, 0, nullptr, num);
     product([&](SvdEigDev& d, GemmDev& g) { set(g, d.b, 1, d.kx, d.xt2, 0, d.mx, d.xt, d.kx, d.mx, d.kx); });
     product([&](SvdEigDev& d, GemmDev& g) { set(g, d.b, 1, d.kx, d.vt, 0, d.kx, d.z, d.kx, d.kx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) {
+        set(g, d.xt, 0, d.mx, d.xt, 1, d.mx, d.b, d.kx, d.kx, d.mx);
+        g.skip = d.flags + 3;
+    });
+    stage(SVD_EIG_VERIFY, 0, 0, nullptr, num);
     stage(SVD_EIG_ORDER, 0, 0, nullptr, num);
     stage(SVD_EIG_WRITE, 0, 0, &l32, int64_t(l32.size()));
 }

@@ -12,14 +12,20 @@
 // leaves columns that are orthogonal to the tolerance of the Jacobi sweeps:
 // squaring costs X' some of its orthogonality (cosines up to eps s1^2 /
 // (si sj)), and I + E removes these cosines to first order, all pairs at once.
-// What it does not remove is below kx c^2 + e c + e^2 for cosines up to c and
-// row sums of |E| up to e; a block is taken only if both are at most
-// EIG_SMALL = 1e-8, which keeps that below half the sweeps' tolerance.  Any
-// other block (close singular values, rank deficiency, entries that are not
-// finite) is left to the Jacobi kernels, which run after this path and skip
-// the blocks marked done.  On 231 blocks of 40 to 190 columns of the 8x8 D=8
-// PEPS the cosines before the refinement were 1.4e-13 in the median and
-// 1.6e-8 at most, and 4e-16 at most after it.
+// For cosines up to c and row sums of |E| up to e, I + E is orthogonal up to
+// e^2 and leaves cosines below kx c^2 + e c + e^2: with both at most EIG_SMALL
+// these are rounding and less than half the sweeps' tolerance.  Above it the
+// step is I + E + E^2 / 2 (orthogonal up to e^4 / 4, e at most EIG_TURN) and the
+// cosines of X'' are measured.  Null columns (the Jacobi kernels' dead ones, up
+// to EIG_DEAD of them) take part in none of this; their directions in U are
+// completed to an orthonormal set at the end.  Any block that fails (close
+// singular values, a larger null space, entries that are not finite) is left to
+// the Jacobi kernels, which run after this path and skip the blocks marked
+// done.  Of 1065 blocks of 32 to 190 columns of the 8x8 D=8 PEPS 0.4% and of 240
+// of the 8x8 Z2 D=6 one 10% take the second form, and all pass; of 5972 blocks of
+// 16 and more columns two have a null column.  The cosines before the step are
+// 1.4e-13 in the median and 3.4e-6 at most.  One block left to the Jacobi kernels
+// costs its launch the whole 5 ms of a block there.
 //
 // One-sided Jacobi does 10 to 14 sweeps of kx^2 / 2 rotations of length mx;
 // this path does about 14 kx^3 multiply-adds, most of them on the matrix
@@ -39,7 +45,8 @@ namespace {
 // data written by an earlier kernel and read at uniform addresses: scalar loads
 typedef const __attribute__((address_space(4))) double* cptr;
 
-constexpr double EIG_SMALL = 1e-8;
+constexpr double EIG_SMALL = 1e-8, EIG_TURN = 1e-4;
+constexpr int EIG_DEAD = 8;
 // row sums of |V^T V - 1| above which one Newton-Schulz step (which squares
 // the defect) does not reach rounding
 constexpr double EIG_DEFECT = 1e-7;
@@ -77,6 +84,7 @@ __global__ __launch_bounds__(1024) void eig_load_kernel(const SvdEigDev* __restr
         tk.flags[0] = 0;                              // done
         tk.flags[1] = (fine && amax > 0.0) ? 0 : 1;  // not for this path
         tk.flags[2] = ex;
+        tk.flags[3] = 1;  // the step's first form, no measurement
     }
     if (tk.t.m < tk.t.n) {
         // M^T: row c of the block is column c of X
@@ -114,19 +122,38 @@ struct TriOut {
     }
 };
 
+// Reflector scalars from one refined reciprocal square root and one refined
+// reciprocal (every wave computes them: the division and square root
+// sequences took a third of a step): beta, tau = 1 - alpha / beta and scale =
+// 1 / (alpha - beta), each within a few ulp.
+__device__ inline void tri_reflector(double alpha, double sigma, double& tau, double& beta, double& scale) {
+    if (sigma == 0.0) {
+        tau = scale = 0.0;
+        beta = alpha;
+        return;
+    }
+    const double s = fma(alpha, alpha, sigma), r = refined_rsqrt(s), root = s * r, a = fabs(alpha);
+    beta = -copysign(root, alpha);
+    tau = fma(a, r, 1.0);
+    scale = copysign(refined_rcp(a + root), alpha);
+}
+
 // Matrix in registers: thread (ti, tj) of TI x 16 holds rows ti + TI a and
-// columns tj + 16 b, a < A, b < BC.  Per column two barriers: row j (column j
-// by symmetry) goes to LDS, every wave forms the reflector from it; then
-// p = tau B v by partial rows and a sum over the 16 lanes of a row group, and
-// the rank-two update.  Bound by LDS reads of v and p (3 BC + 2 A values per
-// thread and step) and the chain of two barriers, one square root and one
-// division per step; a block of rows or columns already reduced is skipped.
+// columns tj + 16 b, a < A, b < BC.  Per column two barriers.  The 16 lanes
+// that hold row j (column j by symmetry) put it into LDS with the square sum
+// below the diagonal; every wave forms the reflector from them.  Then s = B v
+// by partial rows and a sum over the 16 lanes of a row group, with v^T s summed
+// per wave on the way, and the rank-two update.  Bound by the LDS reads of v
+// and p (3 BC + 2 A values per thread and step) and by the chain of two
+// barriers and one reciprocal square root per step; a block of rows or columns
+// already reduced is skipped.  190 columns, one workgroup per CU: 640 us (770
+// with v and w held in registers, 36 of them spilled).
 template<int TI, int A, int BC>
 __global__ __launch_bounds__(TI * 16) void eig_tridiag_kernel(const SvdEigDev* __restrict__ tasks) {
     constexpr int N = TI * A > 16 * BC ? TI * A : 16 * BC, NW = TI * 16 / WAVE;
-    __shared__ double xs[2][N], ps[2][N], wtr[NW];
+    __shared__ double xs[2][N], ps[2][N], sg[2], dots[2][NW], wtr[NW];
     const SvdEigDev tk = tasks[blockIdx.x];
-    const int n = tk.kx, tid = threadIdx.x, lane = tid % WAVE, ti = tid / 16, tj = tid % 16;
+    const int n = tk.kx, tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE, ti = tid / 16, tj = tid % 16;
     if (n > TI * A || n > 16 * BC || tk.flags[1]) return;  // uniform over the workgroup
     const gptr<double> B = to_global(tk.b);
     double rb[A][BC];
@@ -141,7 +168,7 @@ __global__ __launch_bounds__(TI * 16) void eig_tridiag_kernel(const SvdEigDev* _
         }
     for (int i = tid; i < 2 * N; i += TI * 16) (&ps[0][0])[i] = 0.0;
     trace = wave_sum(trace);
-    if (lane == 0) wtr[tid / WAVE] = trace;
+    if (lane == 0) wtr[wave] = trace;
     __syncthreads();
     trace = 0.0;
     for (int w = 0; w < NW; w++) trace += wtr[w];
@@ -152,60 +179,65 @@ __global__ __launch_bounds__(TI * 16) void eig_tridiag_kernel(const SvdEigDev* _
 #pragma unroll
         for (int a = 0; a < A; a++)
             if (j / TI == a && ti == j % TI) {
+                double s = 0.0;
 #pragma unroll
-                for (int b = 0; b < BC; b++) x[tj + 16 * b] = rb[a][b];
+                for (int b = 0; b < BC; b++) {
+                    x[tj + 16 * b] = rb[a][b];
+                    if (tj + 16 * b > j + 1) s += rb[a][b] * rb[a][b];
+                }
+                s = row_sum16(s);
+                if (tj == 0) sg[j & 1] = s;
             }
         __syncthreads();
-        double alpha = 0.0, sigma = 0.0;
-        if (j + 1 < n) {
-            alpha = x[j + 1];
-            double s = 0.0;
-            for (int i = j + 2 + lane; i < n; i += WAVE) s += x[i] * x[i];
-            sigma = wave_sum(s);
-        }
-        double tau, beta;
-        householder(alpha, sigma, tau, beta);
-        const double scale = tau != 0.0 ? 1.0 / (alpha - beta) : 0.0;
+        double tau, beta, scale;
+        tri_reflector(j + 1 < n ? x[j + 1] : 0.0, sg[j & 1], tau, beta, scale);
         if (tid == 0) out.step(j, n, x[j], beta, tau);
         if (tid < n) B[j * n + tid] = tid <= j ? 0.0 : (tid == j + 1 ? 1.0 : x[tid] * scale);
-        // the next step writes the other buffer, and the one after it waits
+        // the next step writes the other buffers, and the one after it waits
         // for every wave to have left this step
         if (tau == 0.0) continue;
-        double vc[BC];
+        // v is read again for the update: held, it would spill at A BC = 48
+        double vr[A], sum[A], dot = 0.0;
+#pragma unroll
+        for (int a = 0; a < A; a++) {
+            const int r = ti + TI * a;
+            vr[a] = r <= j ? 0.0 : (r == j + 1 ? 1.0 : x[r] * scale);
+            sum[a] = 0.0;
+        }
 #pragma unroll
         for (int b = 0; b < BC; b++) {
+            if (16 * b + 15 <= j) continue;
             const int c = tj + 16 * b;
-            vc[b] = c <= j ? 0.0 : (c == j + 1 ? 1.0 : x[c] * scale);
+            const double v = c <= j ? 0.0 : (c == j + 1 ? 1.0 : x[c] * scale);
+#pragma unroll
+            for (int a = 0; a < A; a++) sum[a] += rb[a][b] * v;
         }
 #pragma unroll
         for (int a = 0; a < A; a++) {
             if (TI * a + TI - 1 <= j) continue;
-            double s = 0.0;
-#pragma unroll
-            for (int b = 0; b < BC; b++)
-                if (16 * b + 15 > j) s += rb[a][b] * vc[b];
-            s = row_sum16(s);
+            const double s = row_sum16(sum[a]);
+            dot += s * vr[a];
             if (tj == 0) p[ti + TI * a] = tau * s;
         }
+        // the 16 lanes of a row group hold the same sums: four groups per wave
+        dot = swap_sum<32>(swap_sum<16>(dot));
+        if (lane == 0) dots[j & 1][wave] = dot;
         __syncthreads();
-        double s = 0.0;
-        for (int i = j + 1 + lane; i < n; i += WAVE) s += p[i] * (i == j + 1 ? 1.0 : x[i] * scale);
-        const double K = 0.5 * tau * wave_sum(s);
-        double wc[BC];
+        double K = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) K += dots[j & 1][w];
+        K *= 0.5 * tau * tau;
+        double wr[A];
+#pragma unroll
+        for (int a = 0; a < A; a++) wr[a] = ti + TI * a <= j ? 0.0 : p[ti + TI * a] - K * vr[a];
 #pragma unroll
         for (int b = 0; b < BC; b++) {
+            if (16 * b + 15 <= j) continue;
             const int c = tj + 16 * b;
-            wc[b] = c <= j ? 0.0 : p[c] - K * vc[b];
-        }
+            const double v = c <= j ? 0.0 : (c == j + 1 ? 1.0 : x[c] * scale);
+            const double w = c <= j ? 0.0 : p[c] - K * v;
 #pragma unroll
-        for (int a = 0; a < A; a++) {
-            if (TI * a + TI - 1 <= j) continue;
-            const int r = ti + TI * a;
-            const double vr = r <= j ? 0.0 : (r == j + 1 ? 1.0 : x[r] * scale);
-            const double wr = r <= j ? 0.0 : p[r] - K * vr;
-#pragma unroll
-            for (int b = 0; b < BC; b++)
-                if (16 * b + 15 > j) rb[a][b] -= vr * wc[b] + wr * vc[b];
+            for (int a = 0; a < A; a++) rb[a][b] -= vr[a] * w + wr[a] * v;
         }
     }
 }
@@ -213,14 +245,15 @@ __global__ __launch_bounds__(TI * 16) void eig_tridiag_kernel(const SvdEigDev* _
 // Matrix in global memory (more columns than the registers hold): one pass
 // over the trailing matrix per step, which applies the previous step's
 // rank-two update, stores the result and multiplies it by the new reflector.
-// One wave per row, lane l holds columns l + 64 t.  Bound by those passes
-// (kx^3 16 / 3 bytes through the XCD's L2 by one workgroup).
-constexpr int TRI_GLB_T = (SVD_EIG_MAX_COLS + WAVE - 1) / WAVE;
+// One wave per TRI_GLB_R rows, lane l holds columns l + 64 t, t < TRI_GLB_T.
+// Bound by those passes (kx^3 16 / 3 bytes through the XCD's L2 by one
+// workgroup) and their latency.
+template<int TRI_GLB_T, int TRI_GLB_R>
 __global__ __launch_bounds__(1024) void eig_tridiag_glb_kernel(const SvdEigDev* __restrict__ tasks) {
     __shared__ double xs[SVD_EIG_MAX_COLS], vs[SVD_EIG_MAX_COLS], ws[SVD_EIG_MAX_COLS], ps[SVD_EIG_MAX_COLS], red[16];
     const SvdEigDev tk = tasks[blockIdx.x];
     const int n = tk.kx, tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
-    if (n > SVD_EIG_MAX_COLS || tk.flags[1]) return;
+    if (n > WAVE * TRI_GLB_T || tk.flags[1]) return;
     // the trailing matrix is updated in place in `s`, the reflectors go to `b`
     const gptr<double> B = to_global(tk.s), R = to_global(tk.b);
     double trace = 0.0;
@@ -247,9 +280,8 @@ __global__ __launch_bounds__(1024) void eig_tridiag_glb_kernel(const SvdEigDev* 
             for (int i = j + 2 + lane; i < n; i += WAVE) s += xs[i] * xs[i];
             sigma = wave_sum(s);
         }
-        double tau, beta;
-        householder(alpha, sigma, tau, beta);
-        const double scale = tau != 0.0 ? 1.0 / (alpha - beta) : 0.0;
+        double tau, beta, scale;
+        tri_reflector(alpha, sigma, tau, beta, scale);
         if (tid == 0) out.step(j, n, xs[j], beta, tau);
         if (tid < n) R[j * n + tid] = tid <= j ? 0.0 : (tid == j + 1 ? 1.0 : xs[tid] * scale);
         // v, w of the previous step and the new v at this lane's columns
@@ -262,21 +294,37 @@ __global__ __launch_bounds__(1024) void eig_tridiag_glb_kernel(const SvdEigDev* 
             ow[t] = in ? ws[c] : 0.0;
             nv[t] = in ? (c == j + 1 ? 1.0 : xs[c] * scale) : 0.0;
         }
-        for (int r = j + 1 + wave; r < n; r += 16) {
-            const double vr = vs[r], wr = ws[r];
-            double s = 0.0;
+        // TRI_GLB_R rows at a time keep their loads in flight together
+        for (int r0 = j + 1 + wave; r0 < n; r0 += 16 * TRI_GLB_R) {
+            double vr[TRI_GLB_R], wr[TRI_GLB_R], s[TRI_GLB_R];
+#pragma unroll
+            for (int q = 0; q < TRI_GLB_R; q++) {
+                const int r = min(r0 + 16 * q, n - 1);
+                vr[q] = vs[r];
+                wr[q] = ws[r];
+                s[q] = 0.0;
+            }
 #pragma unroll
             for (int t = 0; t < TRI_GLB_T; t++) {
                 if (WAVE * t >= n || WAVE * t + WAVE - 1 <= j) continue;
                 const int c = lane + WAVE * t;
                 if (c < n && c > j) {
-                    const double v = B[r * n + c] - vr * ow[t] - wr * ov[t];
-                    B[r * n + c] = v;
-                    s += v * nv[t];
+                    double v[TRI_GLB_R];
+#pragma unroll
+                    for (int q = 0; q < TRI_GLB_R; q++) v[q] = B[min(r0 + 16 * q, n - 1) * n + c];
+#pragma unroll
+                    for (int q = 0; q < TRI_GLB_R; q++) {
+                        v[q] -= vr[q] * ow[t] + wr[q] * ov[t];
+                        if (r0 + 16 * q < n) B[(r0 + 16 * q) * n + c] = v[q];
+                        s[q] += v[q] * nv[t];
+                    }
                 }
             }
-            s = wave_sum(s);
-            if (lane == 0) ps[r] = tau * s;
+#pragma unroll
+            for (int q = 0; q < TRI_GLB_R; q++) {
+                const double sum = wave_sum(s[q]);
+                if (lane == 0 && r0 + 16 * q < n) ps[r0 + 16 * q] = tau * sum;
+            }
         }
         __syncthreads();
         double s = 0.0;
@@ -581,9 +629,8 @@ __global__ __launch_bounds__(1024) void eig_polish_kernel(const SvdEigDev* __res
     if (!__syncthreads_and(fine) && threadIdx.x == 0) tk.flags[1] = 1;
 }
 
-// b <- I + E from b = G = X'^T X', with the pair rules of the Jacobi sweeps
-// (cosines at most tol are left alone), after the checks that decide whether
-// the block is this path's
+// b <- I + E from b = G = X'^T X' and the checks that decide whether the block
+// is this path's and which form of the step it takes
 __global__ __launch_bounds__(1024) void eig_refine_kernel(const SvdEigDev* __restrict__ tasks) {
     __shared__ double d[SVD_EIG_MAX_COLS], root[SVD_EIG_MAX_COLS], red[16];
     const SvdEigDev tk = tasks[blockIdx.x];
@@ -604,7 +651,8 @@ __global__ __launch_bounds__(1024) void eig_refine_kernel(const SvdEigDev* __res
     for (int w = 0; w < 16; w++) fro += red[w];
     const double live = fmax(JACOBI_QUIET, JACOBI_DEAD2 * fro);
     const double tol = fmax(1e-15, 2.220446049250313e-16 * tk.mx);
-    bool fine = true;
+    bool fine = true, small = true;
+    int dead = 0;
     for (int r = wave; r < n; r += 16) {
         const double dr = d[r], rr = root[r];
         double sum = 0.0;
@@ -612,43 +660,141 @@ __global__ __launch_bounds__(1024) void eig_refine_kernel(const SvdEigDev* __res
             const double g = G[r * n + c], scale = rr * root[c];
             double e = 1.0;
             if (c != r) {
-                e = 0.0;
-                if (!(fabs(g) <= tol * scale)) {
-                    e = g / (d[c] - dr);
-                    fine = fine && fabs(g) <= EIG_SMALL * scale;
-                }
+                e = g / (d[c] - dr);
+                // as orthogonal as the sweeps ask: turned only if the turn is
+                // slight (close values would turn far for nothing)
+                if (fabs(g) <= tol * scale && !(fabs(e) <= 1e-9)) e = 0.0;
+                if (dr <= live || d[c] <= live) e = 0.0;
+                small = small && (e == 0.0 || fabs(g) <= EIG_SMALL * scale);
                 sum += fabs(e);
             }
             G[r * n + c] = e;
         }
-        fine = fine && wave_sum(sum) <= EIG_SMALL && dr > live;
+        const double row = wave_sum(sum);
+        small = small && row <= EIG_SMALL;
+        fine = fine && row <= EIG_TURN && dr == dr;
+        dead += dr <= live && lane == 0;
     }
+    // a wave has at most kx / 16 rows: the count fits the vote's bits
+    int total = 0;
+    for (int q = 0; q < (SVD_EIG_MAX_COLS + 15) / 16; q++) total += __syncthreads_count(q < dead);
+    fine = __syncthreads_and(fine && total <= EIG_DEAD);
+    small = __syncthreads_and(small);
+    if (tid == 0) {
+        if (!fine) tk.flags[1] = 1;
+        if (!small) tk.flags[3] = 0;
+    }
+}
+
+// b <- I + E + E^2 / 2 = (1 + s) / 2 for s = (I + E)^2
+__global__ __launch_bounds__(1024) void eig_second_kernel(const SvdEigDev* __restrict__ tasks) {
+    const SvdEigDev tk = tasks[blockIdx.x];
+    const int n = tk.kx;
+    if (tk.flags[1] || tk.flags[3]) return;
+    const gptr<const double> S = to_global(tk.s);
+    const gptr<double> Q = to_global(tk.b);
+    for (int e = threadIdx.x; e < n * n; e += 1024) Q[e] = 0.5 * S[e] + (e / n == e % n ? 0.5 : 0.0);
+}
+
+// Cosines of X'' after the second form (b = X''^T X'').  A pair left alone may
+// measure a rounding above the tolerance now, hence the margin.
+__global__ __launch_bounds__(1024) void eig_verify_kernel(const SvdEigDev* __restrict__ tasks) {
+    __shared__ double root[SVD_EIG_MAX_COLS], red[16];
+    const SvdEigDev tk = tasks[blockIdx.x];
+    const int n = tk.kx, tid = threadIdx.x;
+    if (n > SVD_EIG_MAX_COLS || tk.flags[1] || tk.flags[3]) return;
+    const gptr<const double> G = to_global(tk.b);
+    double fro = 0.0;
+    for (int i = tid; i < n; i += 1024) {
+        fro += G[i * n + i];
+        root[i] = sqrt(G[i * n + i]);
+    }
+    fro = wave_sum(fro);
+    if (tid % WAVE == 0) red[tid / WAVE] = fro;
+    __syncthreads();
+    fro = 0.0;
+    for (int w = 0; w < 16; w++) fro += red[w];
+    const double live = sqrt(fmax(JACOBI_QUIET, JACOBI_DEAD2 * fro));
+    const double tol = fmax(1e-15, 2.220446049250313e-16 * tk.mx);
+    bool fine = true;
+    for (int r = tid / WAVE; r < n; r += 16)
+        for (int c = tid % WAVE; c < n; c += WAVE)
+            if (c != r && root[r] > live && root[c] > live)
+                fine = fine && fabs(G[r * n + c]) <= 1.1 * tol * (root[r] * root[c]);
     if (!__syncthreads_and(fine) && tid == 0) tk.flags[1] = 1;
 }
 
-// Singular values (column norms), their descending order (ties by column)
-// and the mark that takes the block from the Jacobi kernels
-__global__ __launch_bounds__(256) void eig_order_kernel(const SvdEigDev* __restrict__ tasks) {
-    __shared__ double sg[SVD_EIG_MAX_COLS];
+// Singular values (column norms), their descending order (ties by column),
+// the directions of null columns and the mark that takes the block from the
+// Jacobi kernels.  A null column keeps its tiny norm as its singular value; its
+// direction is the first unit vector that keeps half its length after two
+// passes of Gram-Schmidt against every other column.
+__global__ __launch_bounds__(1024) void eig_order_kernel(const SvdEigDev* __restrict__ tasks) {
+    __shared__ double sg[SVD_EIG_MAX_COLS], inv[SVD_EIG_MAX_COLS], coef[SVD_EIG_MAX_COLS], red[16];
     const SvdEigDev tk = tasks[blockIdx.x];
     const int n = tk.kx, mx = tk.mx, tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     if (n > SVD_EIG_MAX_COLS || tk.flags[1]) return;
-    const gptr<const double> X = to_global(tk.xt);
+    const gptr<double> X = to_global(tk.xt);
     bool fine = true;
-    for (int c = wave; c < n; c += 4) {
+    double fro = 0.0;
+    for (int c = wave; c < n; c += 16) {
         double s = 0.0;
         for (int r = lane; r < mx; r += WAVE) s += X[c * mx + r] * X[c * mx + r];
         s = wave_sum(s);
-        fine = fine && s > 0.0 && s < 1e300;
-        if (lane == 0) sg[c] = sqrt(s);
+        fine = fine && s < 1e300;
+        fro += s;
+        if (lane == 0) sg[c] = s;
     }
+    if (lane == 0) red[wave] = fro;
     if (!__syncthreads_and(fine)) return;
-    for (int c = tid; c < n; c += 256) {
+    fro = 0.0;
+    for (int w = 0; w < 16; w++) fro += red[w];
+    const double live = fmax(JACOBI_QUIET, JACOBI_DEAD2 * fro);
+    for (int c = tid; c < n; c += 1024) {
+        const double s = sg[c], root = sqrt(s);
+        inv[c] = s > live ? 1.0 / root : 0.0;  // 0: no direction yet
+        sg[c] = root;
+    }
+    __syncthreads();
+    for (int c = 0; c < n; c++) {
+        if (inv[c] > 0.0) continue;  // uniform over the workgroup
+        for (int j = 0; j < mx; j++) {
+            for (int r = tid; r < mx; r += 1024) X[c * mx + r] = r == j ? 1.0 : 0.0;
+            for (int pass = 0; pass < 2; pass++) {
+                __syncthreads();
+                for (int d = wave; d < n; d += 16) {
+                    double s = 0.0;
+                    if (inv[d] > 0.0)
+                        for (int r = lane; r < mx; r += WAVE) s += X[c * mx + r] * X[d * mx + r];
+                    s = wave_sum(s);
+                    if (lane == 0) coef[d] = s * inv[d] * inv[d];
+                }
+                __syncthreads();
+                for (int r = tid; r < mx; r += 1024) {
+                    double v = X[c * mx + r];
+                    for (int d = 0; d < n; d++)
+                        if (inv[d] > 0.0) v -= coef[d] * X[d * mx + r];
+                    X[c * mx + r] = v;
+                }
+            }
+            __syncthreads();
+            double s = 0.0;
+            for (int r = lane; r < mx; r += WAVE) s += X[c * mx + r] * X[c * mx + r];
+            s = wave_sum(s);  // every wave: the same value
+            if (s > 0.25) {
+                if (tid == 0) inv[c] = 1.0 / sqrt(s);
+                break;
+            }
+            __syncthreads();
+        }
+        __syncthreads();
+    }
+    for (int c = tid; c < n; c += 1024) {
         const double sc = sg[c];
         int rank = 0;
         for (int q = 0; q < n; q++) rank += (sg[q] > sc) || (sg[q] == sc && q < c);
         tk.order[rank] = c;
-        tk.sig[rank] = sc;
+        tk.sig[rank] = inv[c];
         tk.t.s[rank] = ldexp(sc, tk.flags[2]);
     }
     if (tid == 0) tk.flags[0] = 1;
@@ -664,7 +810,7 @@ __global__ __launch_bounds__(256) void eig_write_kernel(const SvdEigDev* __restr
     if (!tk.flags[0]) return;
     const int n = tk.kx, r0 = 32 * units[blockIdx.x].tm, tx = threadIdx.x % 32, ty = threadIdx.x / 32;
     const bool trans = tk.t.m < tk.t.n;
-    const gptr<const double> X = to_global(tk.xt), V = to_global(tk.z), sig = to_global(tk.sig);
+    const gptr<const double> X = to_global(tk.xt), V = to_global(tk.z), inv = to_global(tk.sig);
     const gptr<const int32_t> order = to_global(tk.order);
     const gptr<T> U = to_global(static_cast<T*>(tk.t.u)), Vo = to_global(static_cast<T*>(tk.t.v));
     // rows: the columns of X (m < n) or V, as rows of V^T; cols: the others,
@@ -674,7 +820,7 @@ __global__ __launch_bounds__(256) void eig_write_kernel(const SvdEigDev* __restr
     for (int q = ty; q < 32; q += 8) {
         const int rank = r0 + q;
         if (rank >= n) break;
-        const double f = trans ? 1.0 / sig[rank] : 1.0;
+        const double f = trans ? inv[rank] : 1.0;
         const gptr<const double> p = rows + int64_t(order[rank]) * rl;
         for (int i = tx; i < rl; i += 32) Vo[int64_t(rank) * rl + i] = T(p[i] * f);
     }
@@ -682,7 +828,7 @@ __global__ __launch_bounds__(256) void eig_write_kernel(const SvdEigDev* __restr
         for (int q = ty; q < 32; q += 8) {
             const int rank = r0 + q;
             if (rank < n && i0 + tx < cl)
-                tile[q][tx] = cols[int64_t(order[rank]) * cl + i0 + tx] * (trans ? 1.0 : 1.0 / sig[rank]);
+                tile[q][tx] = cols[int64_t(order[rank]) * cl + i0 + tx] * (trans ? 1.0 : inv[rank]);
         }
         __syncthreads();
         for (int q = ty; q < 32; q += 8)
@@ -728,8 +874,10 @@ void launch_svd_eig(int stage, int variant, const SvdEigDev* tasks, const TileDe
                 hipLaunchKernelGGL((eig_tridiag_kernel<32, 4, 8>), grid, dim3(512), 0, st, tasks);
             else if (variant == 2)
                 hipLaunchKernelGGL((eig_tridiag_kernel<48, 4, 12>), grid, dim3(768), 0, st, tasks);
+            else if (variant == 3)
+                hipLaunchKernelGGL((eig_tridiag_glb_kernel<5, 3>), grid, dim3(1024), 0, st, tasks);
             else
-                hipLaunchKernelGGL(eig_tridiag_glb_kernel, grid, dim3(1024), 0, st, tasks);
+                hipLaunchKernelGGL((eig_tridiag_glb_kernel<SVD_EIG_MAX_COLS / WAVE, 1>), grid, dim3(1024), 0, st, tasks);
             break;
         case SVD_EIG_TFACTOR:
             hipLaunchKernelGGL(eig_tfactor_kernel, grid, dim3(64), 0, st, tasks, units);
@@ -755,8 +903,14 @@ void launch_svd_eig(int stage, int variant, const SvdEigDev* tasks, const TileDe
         case SVD_EIG_REFINE:
             hipLaunchKernelGGL(eig_refine_kernel, grid, dim3(1024), 0, st, tasks);
             break;
+        case SVD_EIG_SECOND:
+            hipLaunchKernelGGL(eig_second_kernel, grid, dim3(1024), 0, st, tasks);
+            break;
+        case SVD_EIG_VERIFY:
+            hipLaunchKernelGGL(eig_verify_kernel, grid, dim3(1024), 0, st, tasks);
+            break;
         case SVD_EIG_ORDER:
-            hipLaunchKernelGGL(eig_order_kernel, grid, dim3(256), 0, st, tasks);
+            hipLaunchKernelGGL(eig_order_kernel, grid, dim3(1024), 0, st, tasks);
             break;
         case SVD_EIG_WRITE:
             if (dtype == 0)
