@@ -888,8 +888,7 @@ void plan_svd_factor(const Shape& t, const std::vector<int32_t>& free_u, int32_t
     p.args_v.new_names = res_v;
 }
 
-void plan_svd_truncate(SvdPlan& p, const double* svals, int64_t remain_cut, double relative_cut) {
-    const Kind& k = kind_by_id(p.kind_id);
+std::vector<int64_t> svd_remain(const SvdPlan& p, const double* svals, int64_t remain_cut, double relative_cut) {
     const int ns = int(p.s_sym.size());
     int64_t total_dim = 0;
     double smax = 0;
@@ -906,14 +905,14 @@ void plan_svd_truncate(SvdPlan& p, const double* svals, int64_t remain_cut, doub
     }
     const double threshold = relative_cut > 0 ? relative_cut * smax : 0.0;
     const int64_t rc = (remain_cut < 0 || remain_cut > total_dim) ? total_dim : remain_cut;
-    p.remain.assign(ns, 0);
+    std::vector<int64_t> remain(ns, 0);
     // svd.hpp:454-472: repeatedly keep the largest next value across sectors
     for (int64_t it = 0; it < rc; it++) {
         int best = -1;
         double bv = 0;
         for (int i = 0; i < ns; i++) {
-            if (p.remain[i] != p.s_k[i]) {
-                double v = svals[p.s_off[i] + p.remain[i]];
+            if (remain[i] != p.s_k[i]) {
+                double v = svals[p.s_off[i] + remain[i]];
                 if (v > bv) {
                     bv = v;
                     best = i;
@@ -921,10 +920,21 @@ void plan_svd_truncate(SvdPlan& p, const double* svals, int64_t remain_cut, doub
             }
         }
         if (best >= 0 && bv > threshold)
-            p.remain[best]++;
+            remain[best]++;
         else
             break;
     }
+    return remain;
+}
+
+void plan_svd_truncate(SvdPlan& p, const double* svals, int64_t remain_cut, double relative_cut) {
+    plan_svd_finish(p, svd_remain(p, svals, remain_cut, relative_cut));
+}
+
+void plan_svd_finish(SvdPlan& p, std::vector<int64_t> remain) {
+    const Kind& k = kind_by_id(p.kind_id);
+    const int ns = int(p.s_sym.size());
+    p.remain = std::move(remain);
     CutSpec cut_u{p.cu, {}}, cut_v{p.cv, {}};
     for (int i = 0; i < ns; i++) {
         cut_u.dims.push_back({p.s_sym[i], p.remain[i]});

@@ -12,7 +12,10 @@
 //   qr        TAT/include/TAT/implement/qr.hpp:310-508
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
+#include <cstring>
+#include <initializer_list>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -62,8 +65,88 @@ struct Segment {
     int64_t d = 0;
 };
 
+// A vector with room for N elements inside.  The planners build and drop
+// thousands of edges per configuration, most of them of one to three segments
+// (a site's physical legs stay on its tensor with one segment each): as
+// std::vector, malloc and free were 60% of the planning time, most of it waiting
+// for arena locks when one thread freed what another had allocated.
+template<typename T, int N>
+class SmallVec {
+   public:
+    SmallVec() = default;
+    SmallVec(std::initializer_list<T> l) { assign(l.begin(), l.end()); }
+    SmallVec(const SmallVec& o) { assign(o.begin(), o.end()); }
+    SmallVec(SmallVec&& o) noexcept { take(o); }
+    ~SmallVec() {
+        if (data_ != inline_()) delete[] data_;
+    }
+    SmallVec& operator=(const SmallVec& o) {
+        if (this != &o) assign(o.begin(), o.end());
+        return *this;
+    }
+    SmallVec& operator=(SmallVec&& o) noexcept {
+        if (this != &o) {
+            if (data_ != inline_()) delete[] data_;
+            take(o);
+        }
+        return *this;
+    }
+    size_t size() const { return size_; }
+    bool empty() const { return size_ == 0; }
+    T* data() { return data_; }
+    const T* data() const { return data_; }
+    T* begin() { return data_; }
+    T* end() { return data_ + size_; }
+    const T* begin() const { return data_; }
+    const T* end() const { return data_ + size_; }
+    T& operator[](size_t i) { return data_[i]; }
+    const T& operator[](size_t i) const { return data_[i]; }
+    T& back() { return data_[size_ - 1]; }
+    void clear() { size_ = 0; }
+    void reserve(size_t n) {
+        if (n <= cap_) return;
+        T* p = new T[n];
+        std::copy(data_, data_ + size_, p);
+        if (data_ != inline_()) delete[] data_;
+        data_ = p;
+        cap_ = n;
+    }
+    void push_back(const T& v) {
+        const T copy = v;  // v may live in this vector
+        if (size_ == cap_) reserve(2 * cap_);
+        data_[size_++] = copy;
+    }
+    // [first, last) is not part of this vector
+    void assign(const T* first, const T* last) {
+        size_ = 0;
+        reserve(size_t(last - first));
+        std::copy(first, last, data_);
+        size_ = size_t(last - first);
+    }
+
+   private:
+    T* inline_() { return room_; }
+    void take(SmallVec& o) {
+        size_ = o.size_;
+        if (o.data_ != o.inline_()) {
+            data_ = o.data_;
+            cap_ = o.cap_;
+            o.data_ = o.inline_();
+            o.cap_ = N;
+        } else {
+            data_ = inline_();
+            cap_ = N;
+            std::copy(o.data_, o.data_ + o.size_, data_);
+        }
+        o.size_ = 0;
+    }
+    T room_[N];
+    T* data_ = room_;
+    size_t size_ = 0, cap_ = N;
+};
+
 struct Edge {
-    std::vector<Segment> segs;
+    SmallVec<Segment, 4> segs;
     bool arrow = false;
     int find(const Sym& q) const {
         for (size_t i = 0; i < segs.size(); i++)
@@ -224,6 +307,9 @@ void plan_svd_factor(const Shape& t, const std::vector<int32_t>& free_u, int32_t
                      SvdPlan& p);
 // remain_cut < 0: no count limit; relative_cut <= 0: none
 void plan_svd_truncate(SvdPlan& p, const double* svals, int64_t remain_cut, double relative_cut);
+// its two halves: how many values each sector keeps, and the plan for that
+std::vector<int64_t> svd_remain(const SvdPlan& p, const double* svals, int64_t remain_cut, double relative_cut);
+void plan_svd_finish(SvdPlan& p, std::vector<int64_t> remain);
 
 // ------------------------------------------------------------------ qr
 // Buffers: 0 = input, 1 = merged, 2 = t1, 3 = t2, 4 = Q out, 5 = R out

@@ -21,7 +21,7 @@ double now() {
 
 // ------------------------------------------------------------------ pool
 Pool::Pool(int n) {
-    for (int i = 1; i < n; i++) workers_.emplace_back([this, i] { work(i); });
+    for (int i = 1; i < n; i++) workers_.emplace_back([this] { work(); });
 }
 
 Pool::~Pool() {
@@ -33,29 +33,36 @@ Pool::~Pool() {
     for (auto& t : workers_) t.join();
 }
 
-void Pool::work(int id) {
-    int seen = 0;
+void Pool::work() {
+    int64_t seen = 0;
     while (true) {
         const std::function<void(int64_t, int64_t)>* fn;
-        int64_t n;
+        int64_t n, step;
         {
             std::unique_lock<std::mutex> lk(mu_);
-            cv_.wait(lk, [&] { return stop_ || generation_ != seen; });
+            cv_.wait(lk, [&] { return stop_ || (fn_ && generation_ != seen); });
             if (stop_) return;
             seen = generation_;
             fn = fn_;
             n = n_;
+            step = step_;
+            active_++;
         }
-        const int T = size();
-        const int64_t b = n * id / T, e = n * (id + 1) / T;
-        if (b < e) (*fn)(b, e);
+        take(*fn, n, step);
         {
             std::lock_guard<std::mutex> g(mu_);
-            if (--pending_ == 0) done_cv_.notify_all();
+            if (--active_ == 0) done_cv_.notify_all();
         }
     }
 }
 
+void Pool::take(const std::function<void(int64_t, int64_t)>& fn, int64_t n, int64_t step) {
+    for (int64_t b = next_.fetch_add(step); b < n; b = next_.fetch_add(step)) fn(b, std::min(n, b + step));
+}
+
+// The items are taken in small runs by whoever is awake: a worker that wakes
+// late (tens of microseconds, as long as planning a dozen items) delays
+// nobody, and the caller only waits for runs already taken.
 void Pool::parallel_for(int64_t n, const std::function<void(int64_t, int64_t)>& fn) {
     if (n <= 0) return;
     // waking the workers costs more than planning a few items
@@ -73,19 +80,21 @@ void Pool::parallel_for(int64_t n, const std::function<void(int64_t, int64_t)>& 
             if (!err) err = std::current_exception();
         }
     };
+    const int64_t step = std::max<int64_t>(1, n / (4 * size()));
     {
         std::lock_guard<std::mutex> g(mu_);
         fn_ = &guarded;
         n_ = n;
-        pending_ = int(workers_.size());
+        step_ = step;
+        next_ = 0;
         generation_++;
     }
     cv_.notify_all();
-    const int T = size();
-    guarded(0, n / T);
+    take(guarded, n, step);
     {
         std::unique_lock<std::mutex> lk(mu_);
-        done_cv_.wait(lk, [&] { return pending_ == 0; });
+        fn_ = nullptr;  // nobody joins any more
+        done_cv_.wait(lk, [&] { return active_ == 0; });
     }
     if (err) std::rethrow_exception(err);
 }
@@ -114,13 +123,82 @@ void DevArena::release() {
     cap = used = 0;
 }
 
+// ------------------------------------------------------------------ shapes
+namespace {
+size_t shape_hash(const Shape& s) {
+    size_t h = size_t(s.kind_id);
+    auto mix = [&](uint64_t v) { h = (h ^ v) * 0x9E3779B97F4A7C15ull + (h >> 29); };
+    for (int32_t n : s.names) mix(uint32_t(n));
+    for (const Edge& e : s.edges) {
+        mix(e.segs.size() * 2 + (e.arrow ? 1 : 0));
+        for (const Segment& g : e.segs) {
+            mix((uint64_t(uint32_t(g.q.v[0])) << 32) | uint32_t(g.q.v[1]));
+            mix(uint64_t(g.d));
+        }
+    }
+    return h;
+}
+
+bool same_shape(const Shape& a, const Shape& b) {
+    if (a.kind_id != b.kind_id || a.names != b.names || a.edges.size() != b.edges.size()) return false;
+    for (size_t i = 0; i < a.edges.size(); i++)
+        if (!same_edge(a.edges[i], b.edges[i])) return false;
+    return true;
+}
+
+// Numbers the distinct keys of the n items in order of appearance: item i has
+// key id[i], number q stands for item first[q].
+template<typename Key, typename Hash, typename F>
+void group(int64_t n, const F& key, std::vector<int32_t>& id, std::vector<int64_t>& first) {
+    std::unordered_map<Key, int32_t, Hash> seen;
+    seen.reserve(size_t(n));
+    id.resize(size_t(n));
+    first.clear();
+    for (int64_t i = 0; i < n; i++) {
+        const auto at = seen.emplace(key(i), int32_t(first.size()));
+        if (at.second) first.push_back(i);
+        id[size_t(i)] = at.first->second;
+    }
+}
+
+using ShapePair = std::pair<const Shape*, const Shape*>;
+struct ShapePairHash {
+    size_t operator()(const ShapePair& p) const {
+        return std::hash<const Shape*>()(p.first) * 31 + std::hash<const Shape*>()(p.second);
+    }
+};
+using Remain = std::pair<int32_t, std::vector<int64_t>>;  // factor plan, kept values per sector
+struct RemainHash {
+    size_t operator()(const Remain& r) const {
+        size_t h = size_t(r.first);
+        for (int64_t v : r.second) h = (h ^ size_t(v)) * 0x9E3779B97F4A7C15ull;
+        return h;
+    }
+};
+
+template<typename P>
+void at_least(std::vector<P>& v, size_t n) {
+    if (v.size() < n) v.resize(n);
+}
+}  // namespace
+
+const Shape* ShapeStore::intern(Shape&& s) {
+    const size_t h = shape_hash(s);
+    const auto range = by_hash_.equal_range(h);
+    for (auto it = range.first; it != range.second; ++it)
+        if (same_shape(*it->second, s)) return it->second;
+    shapes_.push_back(std::make_unique<Shape>(std::move(s)));
+    by_hash_.emplace(h, shapes_.back().get());
+    return shapes_.back().get();
+}
+
 // ------------------------------------------------------------------ engine
 enum NameIdx { N_P0, N_T, N_U, N_D, N_L, N_R, N_L1, N_L2, N_L3, N_R1, N_R2, N_P, N_Q, N_FIRST_SITE };
 
 Engine::Engine(int kind, int L1, int L2, const std::vector<Shape>& sites, const std::vector<const void*>& site_data,
                int dtype, const std::vector<int32_t>& names, int threads)
     : kind_(kind), L1_(L1), L2_(L2), dtype_(dtype), es_(dtype == 0 ? 8 : 4), sites_(sites), site_data_(site_data),
-      names_(names), pool_(std::max(1, threads)) {
+      names_(names), batch_(dtype), pool_(std::max(1, threads)) {
     if (int(sites.size()) != L1 * L2 || int(site_data.size()) != L1 * L2) throw Error("engine: wrong number of sites");
     if (int(names.size()) != N_FIRST_SITE + L1 * L2) throw Error("engine: wrong number of name ids");
     const int p0 = sites_[0].index_of(names_[N_P0]);
@@ -133,7 +211,13 @@ Engine::~Engine() {
 }
 
 void Engine::trim() {
-    // the working arenas regrow on the next evaluation; the projected sites stay
+    // the working arenas and plans regrow on the next evaluation; the
+    // projected sites stay
+    cplans_.clear();
+    qplans_.clear();
+    splans_.clear();
+    tplans_.clear();
+    batch_ = Batch(dtype_);
     for (int i = 0; i < NARENA; i++)
         if (i != A_PERSIST) arenas_[i].release();
 }
@@ -152,11 +236,18 @@ void Engine::run_batch(Batch& b, hipStream_t st) {
 }
 
 void Engine::rename(std::vector<Slot*>& t, const std::vector<std::pair<int32_t, int32_t>>& m) {
+    std::unordered_map<const Shape*, const Shape*> done;
     for (auto* s : t) {
-        for (auto& [o, n] : m) {
-            const int i = s->sh.index_of(o);
-            if (i >= 0) s->sh.names[i] = n;
+        auto [at, fresh] = done.emplace(s->sh, nullptr);
+        if (fresh) {
+            Shape r = *s->sh;
+            for (auto& [o, n] : m) {
+                const int i = r.index_of(o);
+                if (i >= 0) r.names[i] = n;
+            }
+            at->second = store_->intern(std::move(r));
         }
+        s->sh = at->second;
     }
 }
 
@@ -172,11 +263,16 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
                       const std::vector<std::pair<int32_t, int32_t>>& pairs, std::vector<Slot*>& out, int oa,
                       hipStream_t st) {
     const int64_t B = int64_t(a.size());
-    const auto pr = present_pairs(a[0]->sh, b[0]->sh, pairs);
-    std::vector<ContractPlan> plans(B);
+    const auto pr = present_pairs(*a[0]->sh, *b[0]->sh, pairs);
     double t0 = now();
-    pool_.parallel_for(B, [&](int64_t s, int64_t e) {
-        for (int64_t i = s; i < e; i++) plan_contract(a[i]->sh, b[i]->sh, pr, plans[i]);
+    std::vector<int32_t> id;
+    std::vector<int64_t> first;
+    group<ShapePair, ShapePairHash>(B, [&](int64_t i) { return ShapePair(a[i]->sh, b[i]->sh); }, id, first);
+    const int64_t U = int64_t(first.size());
+    auto& plans = cplans_;
+    at_least(plans, size_t(U));
+    pool_.parallel_for(U, [&](int64_t s, int64_t e) {
+        for (int64_t u = s; u < e; u++) plan_contract(*a[first[u]]->sh, *b[first[u]]->sh, pr, plans[u]);
     });
     stats_.plan_s += now() - t0;
     // allocation
@@ -189,11 +285,11 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
     const int64_t eg = lowp ? 4 : es_;
     std::vector<int64_t> ta(B), tb(B), tp(B), to(B);
     for (int64_t i = 0; i < B; i++) {
-        ta[i] = int64_t(arenas_[A_TEMP].alloc(size_t(plans[i].ma.size * eg)));
-        tb[i] = int64_t(arenas_[A_TEMP].alloc(size_t(plans[i].mb.size * eg)));
-        tp[i] = int64_t(arenas_[A_TEMP].alloc(size_t(plans[i].prod.size * eg)));
-        to[i] = int64_t(arenas_[oa].alloc(size_t(plans[i].result.size * es_)));
-        stats_.gemm_flops += double(plans[i].flops);
+        ta[i] = int64_t(arenas_[A_TEMP].alloc(size_t(plans[id[i]].ma.size * eg)));
+        tb[i] = int64_t(arenas_[A_TEMP].alloc(size_t(plans[id[i]].mb.size * eg)));
+        tp[i] = int64_t(arenas_[A_TEMP].alloc(size_t(plans[id[i]].prod.size * eg)));
+        to[i] = int64_t(arenas_[oa].alloc(size_t(plans[id[i]].result.size * es_)));
+        stats_.gemm_flops += double(plans[id[i]].flops);
     }
     grow_all(st);
     t0 = now();
@@ -204,13 +300,13 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
         char* Tp = arenas_[A_TEMP].base;
         for (int64_t i = 0; i < B; i++) {
             void* bufs[6] = {ptr(*a[i]), ptr(*b[i]), Tp + ta[i], Tp + tb[i], Tp + tp[i], nullptr};
-            prep.perm(plans[i].perm_a, bufs, es_);
-            prep.perm(plans[i].perm_b, bufs, es_);
+            prep.perm(plans[id[i]].perm_a, bufs, es_);
+            prep.perm(plans[id[i]].perm_b, bufs, es_);
         }
         prep.flush_perm();
         for (int64_t i = 0; i < B; i++) {
             void* bufs[6] = {nullptr, nullptr, Tp + ta[i], Tp + tb[i], Tp + tp[i], nullptr};
-            prep.fill(plans[i].fills, bufs, es_);
+            prep.fill(plans[id[i]].fills, bufs, es_);
         }
         prep.flush_fill();
         run_batch(prep, st);
@@ -228,7 +324,7 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
                     for (int64_t i = 0; i < B; i++) {
                         void* bufs[6] = {nullptr, nullptr, Tp + ta[i], Tp + tb[i], Tp + tp[i], nullptr};
                         std::vector<GemmTask> sel;
-                        for (auto& t : plans[i].gemms)
+                        for (auto& t : plans[id[i]].gemms)
                             if (Batch::gemm_class(t.m, t.n) == c) sel.push_back(t);
                         g.gemm(sel, bufs, es_);
                     }
@@ -245,18 +341,19 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
             }
         }
     }
-    Batch bt(dtype_);
+    Batch& bt = batch_;
+    bt.reset();
     static const int bf16_table[3] = {0, 0, 0};
     bt.set_gemm_table(gemm_prec_ >= 2 ? bf16_table : gemm_table_);
     char* T = arenas_[A_TEMP].base;
     for (int64_t i = 0; i < B; i++) {
         void* bufs[6] = {ptr(*a[i]), ptr(*b[i]), T + ta[i], T + tb[i], T + tp[i], arenas_[oa].base + to[i]};
         if (lowp) {
-            bt.perm_cvt(plans[i].perm_a, bufs, es_, eg);
-            bt.perm_cvt(plans[i].perm_b, bufs, es_, eg);
+            bt.perm_cvt(plans[id[i]].perm_a, bufs, es_, eg);
+            bt.perm_cvt(plans[id[i]].perm_b, bufs, es_, eg);
         } else {
-            bt.perm(plans[i].perm_a, bufs, es_);
-            bt.perm(plans[i].perm_b, bufs, es_);
+            bt.perm(plans[id[i]].perm_a, bufs, es_);
+            bt.perm(plans[id[i]].perm_b, bufs, es_);
         }
     }
     if (lowp)
@@ -265,7 +362,7 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
         bt.flush_perm();
     for (int64_t i = 0; i < B; i++) {
         void* bufs[6] = {nullptr, nullptr, T + ta[i], T + tb[i], T + tp[i], nullptr};
-        bt.fill(plans[i].fills, bufs, eg);
+        bt.fill(plans[id[i]].fills, bufs, eg);
     }
     if (lowp)
         bt.flush_fill_as(1);
@@ -273,7 +370,7 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
         bt.flush_fill();
     for (int64_t i = 0; i < B; i++) {
         void* bufs[6] = {nullptr, nullptr, T + ta[i], T + tb[i], T + tp[i], nullptr};
-        bt.gemm(plans[i].gemms, bufs, eg);
+        bt.gemm(plans[id[i]].gemms, bufs, eg);
     }
     if (lowp)
         bt.flush_gemm_as(gemm_prec_);
@@ -282,9 +379,9 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
     for (int64_t i = 0; i < B; i++) {
         void* bufs[6] = {nullptr, nullptr, T + ta[i], T + tb[i], T + tp[i], arenas_[oa].base + to[i]};
         if (lowp)
-            bt.perm_cvt(plans[i].perm_out, bufs, eg, es_);
+            bt.perm_cvt(plans[id[i]].perm_out, bufs, eg, es_);
         else
-            bt.perm(plans[i].perm_out, bufs, es_);
+            bt.perm(plans[id[i]].perm_out, bufs, es_);
     }
     if (lowp)
         bt.flush_perm_cvt(2);
@@ -293,8 +390,10 @@ void Engine::contract(std::vector<Slot*>& a, std::vector<Slot*>& b,
     stats_.bind_s += now() - t0;
     stats_.launches += 4;
     run_batch(bt, st);
+    std::vector<const Shape*> res(static_cast<size_t>(U));
+    for (int64_t u = 0; u < U; u++) res[u] = store_->intern(std::move(plans[u].result));
     for (int64_t i = 0; i < B; i++) {
-        out[i]->sh = std::move(plans[i].result);
+        out[i]->sh = res[id[i]];
         out[i]->arena = oa;
         out[i]->off = to[i];
     }
@@ -305,11 +404,16 @@ void Engine::qr(std::vector<Slot*>& t, const std::vector<int32_t>& free_names, i
     const int64_t B = int64_t(t.size());
     std::vector<int32_t> fr;
     for (auto n : free_names)
-        if (t[0]->sh.index_of(n) >= 0) fr.push_back(n);
-    std::vector<QrPlan> plans(B);
+        if (t[0]->sh->index_of(n) >= 0) fr.push_back(n);
     double t0 = now();
-    pool_.parallel_for(B, [&](int64_t s, int64_t e) {
-        for (int64_t i = s; i < e; i++) plan_qr(t[i]->sh, 'r', fr, cq, cr, plans[i]);
+    std::vector<int32_t> id;
+    std::vector<int64_t> first;
+    group<const Shape*, std::hash<const Shape*>>(B, [&](int64_t i) { return t[i]->sh; }, id, first);
+    const int64_t U = int64_t(first.size());
+    auto& plans = qplans_;
+    at_least(plans, size_t(U));
+    pool_.parallel_for(U, [&](int64_t s, int64_t e) {
+        for (int64_t u = s; u < e; u++) plan_qr(*t[first[u]]->sh, 'r', fr, cq, cr, plans[u]);
     });
     stats_.plan_s += now() - t0;
     arenas_[A_TEMP].reset();
@@ -317,7 +421,7 @@ void Engine::qr(std::vector<Slot*>& t, const std::vector<int32_t>& free_names, i
     keep_[oa] = arenas_[oa].used;
     std::vector<int64_t> tm(B), t1(B), t2(B), ts(B), oq(B), orr(B);
     for (int64_t i = 0; i < B; i++) {
-        const QrPlan& p = plans[i];
+        const QrPlan& p = plans[id[i]];
         tm[i] = int64_t(arenas_[A_TEMP].alloc(size_t(p.merged.size * es_)));
         t1[i] = int64_t(arenas_[A_TEMP].alloc(size_t(p.t1.size * es_)));
         t2[i] = int64_t(arenas_[A_TEMP].alloc(size_t(p.t2.size * es_)));
@@ -330,33 +434,39 @@ void Engine::qr(std::vector<Slot*>& t, const std::vector<int32_t>& free_names, i
     }
     grow_all(st);
     t0 = now();
-    Batch bt(dtype_);
+    Batch& bt = batch_;
+    bt.reset();
     char* T = arenas_[A_TEMP].base;
     char* O = arenas_[oa].base;
     for (int64_t i = 0; i < B; i++) {
         void* bufs[6] = {ptr(*t[i]), T + tm[i], T + t1[i], T + t2[i], O + oq[i], O + orr[i]};
-        bt.perm(plans[i].perm_in, bufs, es_);
+        bt.perm(plans[id[i]].perm_in, bufs, es_);
     }
     bt.flush_perm();
     for (int64_t i = 0; i < B; i++) {
         void* bufs[6] = {ptr(*t[i]), T + tm[i], T + t1[i], T + t2[i], O + oq[i], O + orr[i]};
-        bt.qr(plans[i].qrs, bufs, es_, reinterpret_cast<double*>(T + ts[i]));
+        bt.qr(plans[id[i]].qrs, bufs, es_, reinterpret_cast<double*>(T + ts[i]));
     }
     bt.flush_qr();
     for (int64_t i = 0; i < B; i++) {
         void* bufs[6] = {ptr(*t[i]), T + tm[i], T + t1[i], T + t2[i], O + oq[i], O + orr[i]};
-        bt.perm(plans[i].perm_1, bufs, es_);
-        bt.perm(plans[i].perm_2, bufs, es_);
+        bt.perm(plans[id[i]].perm_1, bufs, es_);
+        bt.perm(plans[id[i]].perm_2, bufs, es_);
     }
     bt.flush_perm();
     stats_.bind_s += now() - t0;
     stats_.launches += 3;
     run_batch(bt, st);
+    std::vector<const Shape*> rq(static_cast<size_t>(U)), rr(static_cast<size_t>(U));
+    for (int64_t u = 0; u < U; u++) {
+        rq[u] = store_->intern(std::move(plans[u].q));
+        rr[u] = store_->intern(std::move(plans[u].r));
+    }
     for (int64_t i = 0; i < B; i++) {
-        q[i]->sh = std::move(plans[i].q);
+        q[i]->sh = rq[id[i]];
         q[i]->arena = oa;
         q[i]->off = oq[i];
-        r[i]->sh = std::move(plans[i].r);
+        r[i]->sh = rr[id[i]];
         r[i]->arena = oa;
         r[i]->off = orr[i];
     }
@@ -366,10 +476,15 @@ void Engine::svd(std::vector<Slot*>& t, const std::vector<int32_t>& free_u, int3
                  int32_t sv, std::vector<Slot*>& u, std::vector<Slot*>& s, std::vector<Slot*>& v, int oa,
                  hipStream_t st) {
     const int64_t B = int64_t(t.size());
-    std::vector<SvdPlan> plans(B);
     double t0 = now();
-    pool_.parallel_for(B, [&](int64_t b, int64_t e) {
-        for (int64_t i = b; i < e; i++) plan_svd_factor(t[i]->sh, free_u, cu, cv, su, sv, plans[i]);
+    std::vector<int32_t> fid;
+    std::vector<int64_t> ffirst;
+    group<const Shape*, std::hash<const Shape*>>(B, [&](int64_t i) { return t[i]->sh; }, fid, ffirst);
+    const int64_t F = int64_t(ffirst.size());
+    auto& fplans = splans_;
+    at_least(fplans, size_t(F));
+    pool_.parallel_for(F, [&](int64_t b, int64_t e) {
+        for (int64_t q = b; q < e; q++) plan_svd_factor(*t[ffirst[q]]->sh, free_u, cu, cv, su, sv, fplans[q]);
     });
     stats_.plan_s += now() - t0;
     arenas_[A_TEMP].reset();
@@ -378,7 +493,7 @@ void Engine::svd(std::vector<Slot*>& t, const std::vector<int32_t>& free_u, int3
     keep_[oa] = arenas_[oa].used;
     std::vector<int64_t> tm(B), t1(B), t2(B), ts(B), sv_off(B);
     for (int64_t i = 0; i < B; i++) {
-        const SvdPlan& p = plans[i];
+        const SvdPlan& p = fplans[fid[i]];
         tm[i] = int64_t(arenas_[A_TEMP].alloc(size_t(p.merged.size * es_)));
         t1[i] = int64_t(arenas_[A_TEMP].alloc(size_t(p.t1.size * es_)));
         t2[i] = int64_t(arenas_[A_TEMP].alloc(size_t(p.t2.size * es_)));
@@ -393,18 +508,19 @@ void Engine::svd(std::vector<Slot*>& t, const std::vector<int32_t>& free_u, int3
     const size_t sv_bytes = arenas_[A_SVALS].used;
     grow_all(st);
     t0 = now();
-    Batch bt(dtype_);
+    Batch& bt = batch_;
+    bt.reset();
     bt.set_fast_svd(true);
     char* T = arenas_[A_TEMP].base;
     char* S = arenas_[A_SVALS].base;
     for (int64_t i = 0; i < B; i++) {
         void* bufs[5] = {ptr(*t[i]), T + tm[i], T + t1[i], T + t2[i], S + sv_off[i]};
-        bt.perm(plans[i].perm_in, bufs, es_);
+        bt.perm(fplans[fid[i]].perm_in, bufs, es_);
     }
     bt.flush_perm();
     for (int64_t i = 0; i < B; i++) {
         void* bufs[5] = {ptr(*t[i]), T + tm[i], T + t1[i], T + t2[i], S + sv_off[i]};
-        bt.svd(plans[i].svds, bufs, es_, reinterpret_cast<double*>(T + ts[i]));
+        bt.svd(fplans[fid[i]].svds, bufs, es_, reinterpret_cast<double*>(T + ts[i]));
     }
     bt.flush_svd();
     stats_.bind_s += now() - t0;
@@ -417,48 +533,69 @@ void Engine::svd(std::vector<Slot*>& t, const std::vector<int32_t>& free_u, int3
     stats_.sync_s += now() - t1s;
     if (profile_) timer_.collect();
     t0 = now();
+    // how many values each sector keeps is up to the item, the plan to that
+    std::vector<std::vector<int64_t>> remain(static_cast<size_t>(B));
     pool_.parallel_for(B, [&](int64_t b, int64_t e) {
         for (int64_t i = b; i < e; i++)
-            plan_svd_truncate(plans[i], svals_host_.data() + sv_off[i] / 8, remain_cut_, relative_cut_);
+            remain[i] = svd_remain(fplans[fid[i]], svals_host_.data() + sv_off[i] / 8, remain_cut_, relative_cut_);
+    });
+    std::vector<int32_t> id;
+    std::vector<int64_t> first;
+    group<Remain, RemainHash>(B, [&](int64_t i) { return Remain(fid[i], remain[i]); }, id, first);
+    const int64_t U = int64_t(first.size());
+    auto& plans = tplans_;
+    at_least(plans, size_t(U));
+    pool_.parallel_for(U, [&](int64_t b, int64_t e) {
+        for (int64_t q = b; q < e; q++) {
+            plans[q] = fplans[fid[first[q]]];
+            plan_svd_finish(plans[q], std::move(remain[first[q]]));
+        }
     });
     stats_.plan_s += now() - t0;
     std::vector<int64_t> ou(B), os(B), ov(B);
     for (int64_t i = 0; i < B; i++) {
-        ou[i] = int64_t(arenas_[oa].alloc(size_t(plans[i].u.size * es_)));
-        os[i] = int64_t(arenas_[oa].alloc(size_t(plans[i].s.size * es_)));
-        ov[i] = int64_t(arenas_[oa].alloc(size_t(plans[i].v.size * es_)));
+        ou[i] = int64_t(arenas_[oa].alloc(size_t(plans[id[i]].u.size * es_)));
+        os[i] = int64_t(arenas_[oa].alloc(size_t(plans[id[i]].s.size * es_)));
+        ov[i] = int64_t(arenas_[oa].alloc(size_t(plans[id[i]].v.size * es_)));
     }
     grow_all(st);
     t0 = now();
-    Batch b2(dtype_);
+    Batch& b2 = batch_;
+    b2.reset();
     char* O = arenas_[oa].base;
     for (int64_t i = 0; i < B; i++) {
         void* bufs[8] = {nullptr, T + tm[i], T + t1[i], T + t2[i], S + sv_off[i], O + ou[i], O + os[i], O + ov[i]};
-        b2.fill(plans[i].fills_s, bufs, es_);
+        b2.fill(plans[id[i]].fills_s, bufs, es_);
     }
     b2.flush_fill();
     for (int64_t i = 0; i < B; i++) {
         void* bufs[8] = {nullptr, T + tm[i], T + t1[i], T + t2[i], S + sv_off[i], O + ou[i], O + os[i], O + ov[i]};
-        b2.perm(plans[i].perm_u, bufs, es_);
-        b2.perm(plans[i].perm_v, bufs, es_);
+        b2.perm(plans[id[i]].perm_u, bufs, es_);
+        b2.perm(plans[id[i]].perm_v, bufs, es_);
     }
     b2.flush_perm();
     for (int64_t i = 0; i < B; i++) {
         void* bufs[8] = {nullptr, T + tm[i], T + t1[i], T + t2[i], S + sv_off[i], O + ou[i], O + os[i], O + ov[i]};
-        b2.diag(plans[i].diag_s, bufs, es_);
+        b2.diag(plans[id[i]].diag_s, bufs, es_);
     }
     b2.flush_diag();
     stats_.bind_s += now() - t0;
     stats_.launches += 3;
     run_batch(b2, st);
+    std::vector<const Shape*> ru(static_cast<size_t>(U)), rs(static_cast<size_t>(U)), rv(static_cast<size_t>(U));
+    for (int64_t q = 0; q < U; q++) {
+        ru[q] = store_->intern(std::move(plans[q].u));
+        rs[q] = store_->intern(std::move(plans[q].s));
+        rv[q] = store_->intern(std::move(plans[q].v));
+    }
     for (int64_t i = 0; i < B; i++) {
-        u[i]->sh = std::move(plans[i].u);
+        u[i]->sh = ru[id[i]];
         u[i]->arena = oa;
         u[i]->off = ou[i];
-        s[i]->sh = std::move(plans[i].s);
+        s[i]->sh = rs[id[i]];
         s[i]->arena = oa;
         s[i]->off = os[i];
-        v[i]->sh = std::move(plans[i].v);
+        v[i]->sh = rv[id[i]];
         v[i]->arena = oa;
         v[i]->off = ov[i];
     }
@@ -521,9 +658,11 @@ void Engine::project_sites(hipStream_t st) {
                   "shrinker upload");
         check_hip(hipStreamSynchronize(st), "shrinker sync");
     }
-    one_.sh = Shape();
-    one_.sh.kind_id = kind_;
-    one_.sh.finalize();
+    site_shapes_.clear();
+    Shape one;
+    one.kind_id = kind_;
+    one.finalize();
+    one_.sh = site_shapes_.intern(std::move(one));
     one_.arena = A_PERSIST;
     one_.off = one_off;
     // contract every site with each of its shrinkers in one batch; raw sites
@@ -531,8 +670,8 @@ void Engine::project_sites(hipStream_t st) {
     std::vector<Slot> a(shr.size()), b(shr.size()), o(shr.size());
     std::vector<Slot*> pa, pb, po;
     for (size_t i = 0; i < shr.size(); i++) {
-        a[i].sh = sites_[i / nphys_];
-        b[i].sh = shr[i];
+        a[i].sh = &sites_[i / nphys_];
+        b[i].sh = &shr[i];
         b[i].arena = A_PERSIST;
         b[i].off = soff[i];
         pa.push_back(&a[i]);
@@ -560,7 +699,9 @@ void Engine::project_sites(hipStream_t st) {
     const std::vector<std::pair<int32_t, int32_t>> pr{{names_[N_P0], names_[N_Q]}};
     const int prec = gemm_prec_;
     gemm_prec_ = 0;
+    store_ = &site_shapes_;
     contract(pa, pb, pr, po, A_PERSIST, st);
+    store_ = &chunk_shapes_;
     gemm_prec_ = prec;
     keep_[A_PERSIST] = arenas_[A_PERSIST].used;
     proj_.assign(o.begin(), o.end());
@@ -588,6 +729,7 @@ void Engine::evaluate_chunk(int64_t B, const int32_t* occ, double* psi, hipStrea
     const int64_t per = int64_t(L1_) * L2_;
     for (int64_t i = 0; i < B * per; i++)
         if (occ[i] < 0 || occ[i] >= nphys_) throw Error("occupation index out of range of the physical edge");
+    chunk_shapes_.clear();
     auto proj = [&](int64_t b, int l1, int l2) -> const Slot& {
         return proj_[size_t((l1 * L2_ + l2) * nphys_ + occ[b * per + l1 * L2_ + l2])];
     };
@@ -682,12 +824,13 @@ void Engine::evaluate_chunk(int64_t B, const int32_t* occ, double* psi, hipStrea
     keep_[A_TEMP] = 0;
     const int64_t goff = int64_t(arenas_[A_TEMP].alloc(size_t(B * es_)));
     grow_all(st);
-    Batch bt(dtype_);
+    Batch& bt = batch_;
+    bt.reset();
     char* G = arenas_[A_TEMP].base + goff;
     bt.fill_raw(G, B);
     bt.flush_fill();
     for (int64_t b = 0; b < B; b++) {
-        if (inl[b].sh.size != 1) continue;
+        if (inl[b].sh->size != 1) continue;
         PermTask t;
         t.rank = 1;
         t.n = 1;

@@ -9,10 +9,13 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <condition_variable>
 #include <functional>
+#include <memory>
 #include <mutex>
 #include <thread>
+#include <unordered_map>
 #include <vector>
 
 #include "core.hpp"
@@ -25,18 +28,19 @@ class Pool {
     explicit Pool(int n);
     ~Pool();
     int size() const { return int(workers_.size()) + 1; }
-    // fn(begin, end) over [0, n) in contiguous chunks, caller participates
+    // fn(begin, end) over [0, n) in contiguous runs, caller participates
     void parallel_for(int64_t n, const std::function<void(int64_t, int64_t)>& fn);
 
    private:
-    void work(int id);
+    void work();
+    void take(const std::function<void(int64_t, int64_t)>& fn, int64_t n, int64_t step);
     std::vector<std::thread> workers_;
     std::mutex mu_;
     std::condition_variable cv_, done_cv_;
     const std::function<void(int64_t, int64_t)>* fn_ = nullptr;
-    int64_t n_ = 0;
-    int generation_ = 0;
-    int pending_ = 0;
+    int64_t n_ = 0, step_ = 1, generation_ = 0;
+    std::atomic<int64_t> next_{0};
+    int active_ = 0;
     bool stop_ = false;
 };
 
@@ -57,8 +61,25 @@ struct DevArena {
     void release();
 };
 
+// Shapes of one chunk (or of the projected sites), each structure once: the
+// tensors of different configurations that have the same edges share one
+// Shape, so a batched op is planned once per distinct input structure and a
+// slot is a pointer.
+class ShapeStore {
+   public:
+    const Shape* intern(Shape&& s);
+    void clear() {
+        shapes_.clear();
+        by_hash_.clear();
+    }
+
+   private:
+    std::vector<std::unique_ptr<Shape>> shapes_;
+    std::unordered_multimap<size_t, const Shape*> by_hash_;
+};
+
 struct Slot {
-    Shape sh;
+    const Shape* sh = nullptr;
     int arena = -1;  // index into Engine::arenas_
     int64_t off = 0; // byte offset
 };
@@ -143,6 +164,14 @@ class Engine {
     std::vector<int32_t> names_;
     int nphys_ = 0;
     std::vector<Slot> proj_;  // [(l1*L2+l2)*nphys + p]
+    ShapeStore site_shapes_, chunk_shapes_;
+    ShapeStore* store_ = &chunk_shapes_;  // where an op's results go
+    // plans and launch records kept from op to op for their memory; their
+    // contents are rebuilt by every op
+    std::vector<ContractPlan> cplans_;
+    std::vector<QrPlan> qplans_;
+    std::vector<SvdPlan> splans_, tplans_;
+    Batch batch_;
     Slot one_;
     DevArena arenas_[NARENA];
     size_t keep_[NARENA] = {0, 0, 0, 0, 0};

@@ -29,8 +29,7 @@ struct PermDev {
 // l = ceil(log2 d), mul = floor(2^(31+l) / d) + 1 (< 2^32 for every d >= 1)
 // and sh = 31 + l, floor(x / d) = (x * mul) >> sh for all 0 <= x < 2^31.
 inline void perm_magic(uint32_t d, uint32_t* mul, int32_t* sh) {
-    int l = 0;
-    while ((uint64_t(1) << l) < d) l++;
+    const int l = d > 1 ? 32 - __builtin_clz(d - 1) : 0;
     *mul = uint32_t((uint64_t(1) << (31 + l)) / d + 1);
     *sh = 31 + l;
 }

@@ -131,7 +131,7 @@ PermDev bind_perm(const PermTask& t, void* const* bufs, int64_t es_src, int64_t 
     d.rank = t.rank;
     d.neg = t.neg;
     if (t.n >= (int64_t(1) << 31)) throw Error("permute task too large");
-    for (int i = 0; i < MAXR; i++) {
+    for (int i = 0; i < t.rank; i++) {
         d.dims[i] = t.dims[i];
         d.ss[i] = t.ss[i];
         d.ds[i] = t.ds[i];
