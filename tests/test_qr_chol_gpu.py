@@ -1,0 +1,95 @@
+"""The Cholesky path of the sector QR (tall blocks of 32 to 224 columns) at the
+edges of its tiles, and blocks it has to leave to the Householder kernels,
+against numpy's LAPACK, signs included.
+
+Tolerances: both factorisations are backward stable, Q orthogonal and A - Q R
+zero to c max(m, n) eps with c = 4; Q and R themselves differ between two such
+factorisations by that times the condition number of the block."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+EPS = {"D": 2.0 ** -52, "S": 2.0 ** -23}
+
+
+def dense_qr(x, dtype, lq):
+    from tnsp_amd import TAT
+
+    m, n = x.shape
+    t = getattr(TAT.No, dtype).Tensor(["a", "b"], [m, n])
+    t.storage = x.reshape(-1)
+    # the last edge decides between QR (it belongs to R) and LQ (to Q)
+    q, r = t.qr("r", {"a"} if lq else {"b"}, "Q", "R")
+    k = min(m, n)
+    if lq:
+        return (q.transpose(["b", "Q"]).storage.numpy().reshape(n, k).astype(np.float64),
+                r.transpose(["R", "a"]).storage.numpy().reshape(k, m).astype(np.float64))
+    return (q.transpose(["a", "Q"]).storage.numpy().reshape(m, k).astype(np.float64),
+            r.transpose(["R", "b"]).storage.numpy().reshape(k, n).astype(np.float64))
+
+
+def check(x, dtype, lq, same=True):
+    q, r = dense_qr(x, dtype, lq)
+    a = x.astype(np.float32).astype(np.float64) if dtype == "S" else x
+    a = a.T if lq else a
+    scale = np.max(np.abs(a)) or 1.0
+    a, r = a / scale, r / scale
+    tol = 4 * max(a.shape) * EPS[dtype]
+    assert np.max(np.abs(q.T @ q - np.eye(q.shape[1]))) <= tol
+    assert np.linalg.norm(q @ r - a) <= tol * np.linalg.norm(a)
+    assert np.all(np.tril(r, -1) == 0)
+    if same:
+        q0, r0 = np.linalg.qr(a)
+        tol *= np.linalg.cond(a)
+        assert np.linalg.norm(q - q0) <= tol * np.linalg.norm(q0)
+        assert np.linalg.norm(r - r0) <= tol * np.linalg.norm(r0)
+
+
+@pytest.mark.parametrize("lq", [False, True])
+@pytest.mark.parametrize("m,n", [(32, 32), (33, 32), (63, 63), (64, 64), (65, 64), (130, 65), (128, 128), (200, 129),
+                                 (192, 192), (1173, 176), (700, 192), (500, 193), (224, 224), (300, 225), (1500, 40), (100, 31)])
+def test_tall_blocks(m, n, lq):
+    x = np.random.default_rng(m * 1000 + n).standard_normal((m, n))
+    check(x.T.copy() if lq else x, "D", lq)
+
+
+@pytest.mark.parametrize("m,n", [(40, 33), (400, 129)])
+def test_float32_blocks(m, n):
+    check(np.random.default_rng(m).standard_normal((m, n)).astype(np.float32), "S", False)
+
+
+@pytest.mark.parametrize("n", [40, 150])
+@pytest.mark.parametrize("kind", ["triangular", "identity", "diagonal", "rank", "zero_column", "graded_columns",
+                                  "ill_conditioned", "tiny", "huge", "zero_rows"])
+def test_special_blocks(n, kind):
+    """Taken or left, the result is a QR; where Q and R are determined by the
+    block (full rank, well conditioned) they have the Householder signs."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n + 30, n))
+    same = True
+    if kind == "triangular":
+        x = np.triu(x)
+    elif kind == "identity":
+        x = np.eye(n + 30, n)
+    elif kind == "diagonal":
+        x = np.eye(n + 30, n) * rng.standard_normal(n)
+    elif kind == "rank":
+        x = x[:, :n // 2] @ rng.standard_normal((n // 2, n))
+        same = False
+    elif kind == "zero_column":
+        x[:, n // 2] = 0.0
+        same = False
+    elif kind == "graded_columns":
+        x = x * np.logspace(0, -6, n)
+    elif kind == "ill_conditioned":
+        u, s, v = np.linalg.svd(x, full_matrices=False)
+        x = (u * np.logspace(0, -9, n)) @ v
+    elif kind == "tiny":
+        x = x * 1e-200
+    elif kind == "huge":
+        x = x * 1e150
+    elif kind == "zero_rows":
+        x[n // 2:] = 0.0
+        same = False
+    check(x, "D", False, same)

@@ -181,11 +181,17 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const GemmDev* __res
                                                            const TileDev* __restrict__ tiles) {
     constexpr int NT = 64 * WR * WC, TM = 16 * WR * FM, TN = 16 * WC * FN;
     constexpr int LA = (TM * KB + NT - 1) / NT, LB = (KB * TN + NT - 1) / NT;
-    __shared__ T As[2][TM][KB + 1];
-    __shared__ T Bs[2][KB][TN + 1];
+    // row strides that spread an operand read (16 rows x 4 of A, 4 rows x 16 of
+    // B) evenly over the 64 banks: 18 doubles put the 16 rows of A 4 words
+    // apart, and a B stride of 32 words modulo 64 puts every other row on the
+    // other half (strides of KB + 1 and TN + 1 doubled up most reads of B)
+    constexpr int BP = TN % 32 == 0 ? 16 : 0;
+    __shared__ T As[2][TM][KB + 2];
+    __shared__ T Bs[2][KB][TN + BP];
     const TileDev tile = tiles[blockIdx.x];
-    const GemmDev g = tasks[tile.task];
+    GemmDev g = tasks[tile.task];
     if (g.skip && *g.skip) return;
+    if (tile.kmax) g.k = min(g.k, tile.kmax);
     const gptr<const T> A = to_global(static_cast<const T*>(g.a));
     const gptr<const T> B = to_global(static_cast<const T*>(g.b));
     const int row0 = tile.tm * TM, col0 = tile.tn * TN;
@@ -547,6 +553,7 @@ __global__ __launch_bounds__(QR_WG) void qr_kernel_lds(const QrDev* __restrict__
     __shared__ double red[QR_WG / WAVE];
     __shared__ double bc[1];
     const QrDev tk = tasks[blockIdx.x];
+    if (tk.done && *tk.done) return;
     const int mx = tk.lq ? tk.n : tk.m, nx = tk.lq ? tk.m : tk.n;
     qr_body<T>(tk, smem, smem + int64_t(mx) * nx, red, bc);
 }
@@ -556,6 +563,7 @@ __global__ __launch_bounds__(QR_WG) void qr_kernel_glb(const QrDev* __restrict__
     __shared__ double red[QR_WG / WAVE];
     __shared__ double bc[1];
     const QrDev tk = tasks[blockIdx.x];
+    if (tk.done && *tk.done) return;
     const int mx = tk.lq ? tk.n : tk.m, nx = tk.lq ? tk.m : tk.n;
     qr_body<T>(tk, tk.work, tk.work + int64_t(mx) * nx, red, bc);
 }
@@ -745,6 +753,7 @@ __global__ __launch_bounds__(QR_WG) void qr_kernel_blocked(const QrDev* __restri
     __shared__ double red[QR_WG / WAVE];
     __shared__ double bc[1];
     const QrDev tk = tasks[blockIdx.x];
+    if (tk.done && *tk.done) return;
     const int m = tk.m, n = tk.n, lq = tk.lq;
     const int mx = lq ? n : m, nx = lq ? m : n, k = mx < nx ? mx : nx;
     const int nbmax = qb_panel_width(mx);
