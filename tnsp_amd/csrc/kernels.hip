@@ -181,13 +181,8 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const GemmDev* __res
                                                            const TileDev* __restrict__ tiles) {
     constexpr int NT = 64 * WR * WC, TM = 16 * WR * FM, TN = 16 * WC * FN;
     constexpr int LA = (TM * KB + NT - 1) / NT, LB = (KB * TN + NT - 1) / NT;
-    // row strides that spread an operand read (16 rows x 4 of A, 4 rows x 16 of
-    // B) evenly over the 64 banks: 18 doubles put the 16 rows of A 4 words
-    // apart, and a B stride of 32 words modulo 64 puts every other row on the
-    // other half (strides of KB + 1 and TN + 1 doubled up most reads of B)
-    constexpr int BP = TN % 32 == 0 ? 16 : 0;
-    __shared__ T As[2][TM][KB + 2];
-    __shared__ T Bs[2][KB][TN + BP];
+    __shared__ T As[2][TM][KB + 1];
+    __shared__ T Bs[2][KB][TN + 1];
     const TileDev tile = tiles[blockIdx.x];
     GemmDev g = tasks[tile.task];
     if (g.skip && *g.skip) return;
