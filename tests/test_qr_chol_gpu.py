@@ -59,7 +59,7 @@ def test_float32_blocks(m, n):
     check(np.random.default_rng(m).standard_normal((m, n)).astype(np.float32), "S", False)
 
 
-@pytest.mark.parametrize("n", [40, 150])
+@pytest.mark.parametrize("n", [20, 40, 150])
 @pytest.mark.parametrize("kind", ["triangular", "identity", "diagonal", "rank", "zero_column", "graded_columns",
                                   "ill_conditioned", "tiny", "huge", "zero_rows"])
 def test_special_blocks(n, kind):

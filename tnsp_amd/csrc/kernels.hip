@@ -457,10 +457,19 @@ __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau,
     const T* in = static_cast<const T*>(tk.in);
     const int tid = threadIdx.x;
     const int G = qr_group_lanes(mx, nx), NG = QR_WG / G, g = tid / G, gl = tid % G;
+    double amax = 0;
     for (int64_t e = tid; e < int64_t(mx) * nx; e += QR_WG) {
         const int r = int(e % mx), c = int(e / mx);
-        X[e] = double(lq ? in[int64_t(c) * n + r] : in[int64_t(r) * n + c]);
+        const double x = double(lq ? in[int64_t(c) * n + r] : in[int64_t(r) * n + c]);
+        X[e] = x;
+        amax = fmax(amax, fabs(x));
     }
+    amax = block_max<QR_WG>(amax, red);
+    // blocks whose squares would vanish or overflow work on entries of order one
+    // (without it a block of 1e-200 looks like zero columns and gets no reflectors)
+    const int shift = amax > 0.0 && amax <= 1.79e308 && (amax < 1e-140 || amax > 1e140) ? -ilogb(amax) : 0;
+    if (shift)
+        for (int64_t e = tid; e < int64_t(mx) * nx; e += QR_WG) X[e] = ldexp(X[e], shift);
     __syncthreads();
     // squared norm below the diagonal of the column to reduce: a block sum
     // for column 0, then from the group that updates the next column
@@ -494,12 +503,12 @@ __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau,
     if (!lq) {
         for (int64_t e = tid; e < int64_t(k) * n; e += QR_WG) {
             const int r = int(e / n), c = int(e % n);
-            f2[e] = T(r <= c ? X[int64_t(c) * mx + r] : 0.0);
+            f2[e] = T(r <= c ? (shift ? ldexp(X[int64_t(c) * mx + r], -shift) : X[int64_t(c) * mx + r]) : 0.0);
         }
     } else {
         for (int64_t e = tid; e < int64_t(m) * k; e += QR_WG) {
             const int i = int(e / k), r = int(e % k);
-            f1[e] = T(r <= i ? X[int64_t(i) * mx + r] : 0.0);
+            f1[e] = T(r <= i ? (shift ? ldexp(X[int64_t(i) * mx + r], -shift) : X[int64_t(i) * mx + r]) : 0.0);
         }
     }
     __syncthreads();
