@@ -138,10 +138,10 @@ struct Layout {
 };
 int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
 
+int64_t qr_scratch(const QrTask& t) { return qr_doubles(t.m, t.n); }
 int64_t svd_scratch(const SvdTask& t) { return svd_doubles(t.m, t.n); }
 
-// plain_qr: QR scratch of the Householder kernels alone
-Layout layout_of(const tns_plan* p, int dtype, bool plain_qr = false) {
+Layout layout_of(const tns_plan* p, int dtype) {
     const int64_t es = dtype == 0 ? 8 : 4;
     Layout L;
     auto sizes = buffer_sizes(p);
@@ -172,7 +172,7 @@ Layout layout_of(const tns_plan* p, int dtype, bool plain_qr = false) {
             put(2, sizes[2] * es);
             put(3, sizes[3] * es);
             int64_t sc = 0;
-            for (auto& t : p->q.qrs) sc += plain_qr ? qr_plain_doubles(t.m, t.n) : qr_doubles(t.m, t.n, t.lq);
+            for (auto& t : p->q.qrs) sc += qr_scratch(t);
             L.scratch = L.total;
             L.total = align256(L.total + sc * 8);
             break;
@@ -419,22 +419,19 @@ int tns_plan_run(tns_plan* p, int dtype, const void* const* inputs, void* const*
 
 }  // extern "C"
 
-int64_t tns::plan_workspace_bytes(const tns_plan* p, int dtype, bool plain_qr) {
-    return layout_of(p, dtype, plain_qr).total;
-}
+int64_t tns::plan_workspace_bytes(const tns_plan* p, int dtype) { return layout_of(p, dtype).total; }
 
 bool tns::plan_is_svd(const tns_plan* p) { return p->type == tns_plan::SVD; }
 
 void tns::run_plan(tns_plan* p, int dtype, const void* const* inputs, void* const* outputs, void* workspace,
-                   hipStream_t stream, Staging* staging, bool plain_qr) {
+                   hipStream_t stream, Staging* staging) {
     {
         if (dtype != 0 && dtype != 1) throw Error("unsupported dtype");
         const int64_t es = dtype == 0 ? 8 : 4;
-        Layout L = layout_of(p, dtype, plain_qr);
+        Layout L = layout_of(p, dtype);
         char* ws = static_cast<char*>(workspace);
         if (L.total > 0 && !ws) throw Error("workspace required");
         Batch bt(dtype);
-        bt.set_plain_qr(plain_qr);
         if (staging) bt.set_staging(staging);
         switch (p->type) {
             case tns_plan::EDGEOP:

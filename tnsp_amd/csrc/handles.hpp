@@ -20,11 +20,11 @@ int set_error(const char* what);
 
 class Staging;
 // body of tns_plan_run; staging = nullptr uses the calling thread's own
-// (growable) task staging; plain_qr: workspace without the Cholesky QR's scratch
+// (growable) task staging
 void run_plan(tns_plan* p, int dtype, const void* const* inputs, void* const* outputs, void* workspace,
-              hipStream_t stream, Staging* staging, bool plain_qr = false);
+              hipStream_t stream, Staging* staging);
 // device workspace bytes tns_plan_run needs for the plan
-int64_t plan_workspace_bytes(const tns_plan* p, int dtype, bool plain_qr = false);
+int64_t plan_workspace_bytes(const tns_plan* p, int dtype);
 bool plan_is_svd(const tns_plan* p);
 }  // namespace tns
 

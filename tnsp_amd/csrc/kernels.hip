@@ -184,9 +184,8 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const GemmDev* __res
     __shared__ T As[2][TM][KB + 1];
     __shared__ T Bs[2][KB][TN + 1];
     const TileDev tile = tiles[blockIdx.x];
-    GemmDev g = tasks[tile.task];
+    const GemmDev g = tasks[tile.task];
     if (g.skip && *g.skip) return;
-    if (tile.kmax) g.k = min(g.k, tile.kmax);
     const gptr<const T> A = to_global(static_cast<const T*>(g.a));
     const gptr<const T> B = to_global(static_cast<const T*>(g.b));
     const int row0 = tile.tm * TM, col0 = tile.tn * TN;
@@ -557,7 +556,6 @@ __global__ __launch_bounds__(QR_WG) void qr_kernel_lds(const QrDev* __restrict__
     __shared__ double red[QR_WG / WAVE];
     __shared__ double bc[1];
     const QrDev tk = tasks[blockIdx.x];
-    if (tk.done && *tk.done) return;
     const int mx = tk.lq ? tk.n : tk.m, nx = tk.lq ? tk.m : tk.n;
     qr_body<T>(tk, smem, smem + int64_t(mx) * nx, red, bc);
 }
@@ -567,7 +565,6 @@ __global__ __launch_bounds__(QR_WG) void qr_kernel_glb(const QrDev* __restrict__
     __shared__ double red[QR_WG / WAVE];
     __shared__ double bc[1];
     const QrDev tk = tasks[blockIdx.x];
-    if (tk.done && *tk.done) return;
     const int mx = tk.lq ? tk.n : tk.m, nx = tk.lq ? tk.m : tk.n;
     qr_body<T>(tk, tk.work, tk.work + int64_t(mx) * nx, red, bc);
 }
@@ -757,7 +754,6 @@ __global__ __launch_bounds__(QR_WG) void qr_kernel_blocked(const QrDev* __restri
     __shared__ double red[QR_WG / WAVE];
     __shared__ double bc[1];
     const QrDev tk = tasks[blockIdx.x];
-    if (tk.done && *tk.done) return;
     const int m = tk.m, n = tk.n, lq = tk.lq;
     const int mx = lq ? n : m, nx = lq ? m : n, k = mx < nx ? mx : nx;
     const int nbmax = qb_panel_width(mx);

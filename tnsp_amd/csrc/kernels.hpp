@@ -44,8 +44,7 @@ struct GemmDev {
 };
 
 struct TileDev {
-    int32_t task, tm, tn;
-    int32_t kmax;  // GEMM: terms of the sum for this tile, 0 for all (triangular factors)
+    int32_t task, tm, tn, pad;
 };
 
 struct FillDev {
@@ -59,7 +58,6 @@ struct QrDev {
     void* f2;
     double* work;  // global scratch (mx*nx + k doubles) when not LDS-resident
     int32_t m, n, lq, pad;
-    const int32_t* done;  // non-null: nothing to do where *done is set (the Cholesky path took the sector)
 };
 
 struct SvdDev {
@@ -121,26 +119,8 @@ constexpr int SVD_WG = 256;
 constexpr int64_t LDS_CLASS[3] = {48 * 1024, 76 * 1024, 152 * 1024};
 constexpr int64_t QR_LDS_MAX = LDS_CLASS[2];
 constexpr int64_t SVD_LDS_MAX = LDS_CLASS[2];
-// Sectors that go through Cholesky factors first (qr_chol.hip): tall ones of
-// 32 to 224 columns (the eliminations hold nx x nx values in registers).
-// 48 tensors with sectors up to 1173 x 200: 6.4 -> 2.7 ms a pass (the Householder
-// kernels took 5.6 of it); one stage of 128 8x8 D=8 configurations: blocked
-// Householder 2.55 -> 0.87 ms (wide sectors stay there) and LDS Householder 0.99
-// -> 0.84 ms for 1.9 ms of this path, whose launches leave room for other lanes:
-// 256 amplitudes in four lanes 383 -> 367 ms.  Below 32 columns the LDS kernel's
-// chain is short.
-constexpr int QR_CHOL_MIN_COLS = 32, QR_CHOL_MAX_COLS = 224;
-inline bool qr_chol_fits(int64_t m, int64_t n, int lq) {
-    const int64_t mx = lq ? n : m, nx = lq ? m : n;
-    return nx <= mx && nx >= QR_CHOL_MIN_COLS && nx <= QR_CHOL_MAX_COLS && mx * nx <= (int64_t(1) << 28);
-}
-// scratch of a QR / LQ task beyond LDS: the block and its taus; the Cholesky
-// path's two column sets, four nx x nx matrices, the signs and the flags
-inline int64_t qr_plain_doubles(int64_t m, int64_t n) { return m * n + (m < n ? m : n); }
-inline int64_t qr_doubles(int64_t m, int64_t n, int lq) {
-    const int64_t nx = lq ? m : n;
-    return qr_chol_fits(m, n, lq) ? 2 * m * n + 4 * nx * nx + nx + 2 : qr_plain_doubles(m, n);
-}
+// scratch of a QR / LQ task beyond LDS: the block and its taus
+inline int64_t qr_doubles(int64_t m, int64_t n) { return m * n + (m < n ? m : n); }
 // Sectors that go through the eigenvectors of their Gram matrix first
 // (svd_eig.hip).  Whole SVD passes with the Jacobi kernels alone and with this
 // path: 64 tensors with sectors up to about 200 x 190 (some beyond the register
@@ -210,32 +190,6 @@ enum SvdEigStage {
 };
 void launch_svd_eig(int stage, int variant, const SvdEigDev* tasks, const TileDev* units, int64_t num, int dtype,
                     hipStream_t stream);
-
-// A sector on the Cholesky QR path (rows contiguous: row c of xt is column c)
-struct QrCholDev {
-    QrDev t;
-    double *xt, *q;              // nx x mx
-    double *b, *g, *r1, *r2;     // nx x nx
-    double* sign;                // nx
-    int32_t* flags;              // done, not for this path, scale exponent
-    int32_t mx, nx;
-};
-enum QrCholStage {
-    QR_CHOL_RANGE,   // per task
-    QR_CHOL_LOAD,    // per task and 32 columns (units)
-    QR_CHOL_FIRST,   // per task; variant 0..3: at most 64 / 128 / 192 / 224 columns
-    QR_CHOL_SECOND,  // likewise
-    QR_CHOL_SIGN,    // likewise
-    QR_CHOL_WRITE    // per task and 32 columns (units)
-};
-void launch_qr_chol(int stage, int variant, const QrCholDev* tasks, const TileDev* units, int64_t num, int dtype,
-                    hipStream_t stream);
-
-// Tasks up to which the eliminations of every size run as one launch of the
-// largest kernel needed: one workgroup per CU, so they all run at once and
-// the launch takes as long as its largest task, instead of one launch per size
-// class after the other.
-constexpr int64_t ONE_WAVE_TASKS = 256;
 
 // Copy n_i doubles from src_i to dst + off_i for every task, one workgroup
 // per task: gathers the singular values of a batch of decompositions into

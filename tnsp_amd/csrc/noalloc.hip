@@ -57,16 +57,14 @@ int tns_plan_run_noalloc(tns_plan* p, int dtype, const void* const* inputs, void
             throw tns::Error("noalloc: svd plans are not supported (tns_svd_factor writes into the caller's workspace)");
         // size checks come before any HIP call, so an oversized plan fails the
         // same way with or without a device
-        // a QR whose Cholesky path does not fit runs the Householder kernels
-        const bool plain_qr = tns::plan_workspace_bytes(p, dtype, false) > NOALLOC_WORKSPACE_BYTES;
-        const int64_t need = tns::plan_workspace_bytes(p, dtype, plain_qr);
+        const int64_t need = tns::plan_workspace_bytes(p, dtype);
         if (need > NOALLOC_WORKSPACE_BYTES)
             throw tns::Error("noalloc: the plan needs " + std::to_string(need) +
                              " bytes of workspace, more than the static maximum of " +
                              std::to_string(NOALLOC_WORKSPACE_BYTES) + " bytes; use tns_plan_run");
         unsigned char* base = scratch_on_current_device();
         tns::Staging staging(reinterpret_cast<char*>(base + NOALLOC_WORKSPACE_BYTES), size_t(NOALLOC_TASK_BYTES));
-        tns::run_plan(p, dtype, inputs, outputs, base, static_cast<hipStream_t>(stream), &staging, plain_qr);
+        tns::run_plan(p, dtype, inputs, outputs, base, static_cast<hipStream_t>(stream), &staging);
     })
 }
 

@@ -313,7 +313,7 @@ void Batch::qr(const std::vector<QrTask>& ts, void* const* bufs, int64_t es, dou
         q.m = t.m;
         q.n = t.n;
         q.lq = t.lq;
-        cur += plain_qr_ ? qr_plain_doubles(t.m, t.n) : qr_doubles(t.m, t.n, t.lq);
+        cur += qr_doubles(t.m, t.n);
         const double M = double(std::max(t.m, t.n)), N = double(std::min(t.m, t.n));
         const double fl = 4.0 * M * N * N - 4.0 * N * N * N / 3.0;
         pend_units_[QR] += fl;
@@ -373,93 +373,7 @@ void Batch::flush_decomp(Kind kind, std::vector<D>& tasks, std::vector<double>& 
     cost.clear();
 }
 
-// The Cholesky path over every sector it takes, by columns; the Householder
-// launches that follow skip what it finished.
-void Batch::flush_qr_chol() {
-    std::vector<size_t> sel;
-    for (size_t i = 0; i < pqr_.size(); i++)
-        if (!plain_qr_ && qr_chol_fits(pqr_[i].m, pqr_[i].n, pqr_[i].lq)) sel.push_back(i);
-    if (sel.empty()) return;
-    auto cols = [&](size_t i) { return std::min(pqr_[i].m, pqr_[i].n); };
-    std::stable_sort(sel.begin(), sel.end(), [&](size_t a, size_t b) { return cols(a) > cols(b); });
-    const size_t T = sel.size();
-    std::vector<QrCholDev> tasks(T);
-    std::vector<TileDev> l32;
-    double units = 0;
-    for (size_t i = 0; i < T; i++) {
-        QrDev& t = pqr_[sel[i]];
-        QrCholDev& d = tasks[i];
-        const int64_t mx = t.lq ? t.n : t.m, nx = t.lq ? t.m : t.n;
-        d.mx = int32_t(mx);
-        d.nx = int32_t(nx);
-        double* cur = t.work;
-        auto take = [&](int64_t n) {
-            double* p = cur;
-            cur += n;
-            return p;
-        };
-        d.xt = take(mx * nx);
-        d.q = take(mx * nx);
-        d.b = take(nx * nx);
-        d.g = take(nx * nx);
-        d.r1 = take(nx * nx);
-        d.r2 = take(nx * nx);
-        d.sign = take(nx);
-        d.flags = reinterpret_cast<int32_t*>(take(2));
-        if (cur != t.work + qr_doubles(t.m, t.n, t.lq)) throw Error("internal: qr scratch layout");
-        t.done = d.flags;
-        d.t = t;
-        units += pqr_cost_[sel[i]];
-        for (int j = 0; j * 32 < nx; j++) l32.push_back(TileDev{int32_t(i), j, 0, 0});
-    }
-    const size_t toff = put(tasks);
-    auto stage = [&](int st, int variant, size_t first, size_t units_at, int64_t num) {
-        Cmd c;
-        c.kind = QR_CHOL;
-        c.stage = st;
-        c.timed = KernelTimer::QR_CHOL;
-        c.rpt = variant;
-        c.tasks = toff + first * sizeof(QrCholDev);
-        c.prefix = units_at;
-        c.count = c.nwg = num;
-        cmds_.push_back(c);
-    };
-    auto sized = [&](int st) {
-        static const int hi[4] = {64, 128, 192, QR_CHOL_MAX_COLS};
-        size_t a = 0;
-        for (int v = 3; v >= 0; v--) {
-            size_t b = a;
-            const int lo = v && int64_t(T) > ONE_WAVE_TASKS ? hi[v - 1] : 0;
-            while (b < T && tasks[b].nx > lo && tasks[a].nx > (v ? hi[v - 1] : 0)) b++;
-            if (b > a) stage(st, v, a, 0, int64_t(b - a));
-            a = b;
-        }
-    };
-    auto product = [&](auto fill) {
-        std::vector<Product> ps(T);
-        for (size_t i = 0; i < T; i++) ps[i] = fill(tasks[i]);
-        this->product(ps, KernelTimer::QR_CHOL);
-    };
-    const size_t first_cmd = cmds_.size();
-    const size_t l32_at = put(l32);
-    stage(QR_CHOL_RANGE, 0, 0, 0, int64_t(T));
-    stage(QR_CHOL_LOAD, 0, 0, l32_at, int64_t(l32.size()));
-    cmds_[first_cmd].units = units;
-    product([](QrCholDev& d) { return Product{d.xt, d.xt, d.b, 0, d.mx, 1, d.mx, d.nx, d.nx, d.mx, nullptr, true, false}; });
-    sized(QR_CHOL_FIRST);
-    product([](QrCholDev& d) { return Product{d.g, d.xt, d.q, 0, d.nx, 0, d.mx, d.nx, d.mx, d.nx, nullptr, false, true}; });
-    product([](QrCholDev& d) { return Product{d.q, d.q, d.b, 0, d.mx, 1, d.mx, d.nx, d.nx, d.mx, nullptr, true, false}; });
-    sized(QR_CHOL_SECOND);
-    product([](QrCholDev& d) { return Product{d.g, d.q, d.xt, 0, d.nx, 0, d.mx, d.nx, d.mx, d.nx, nullptr, false, true}; });
-    product([](QrCholDev& d) { return Product{d.r2, d.r1, d.b, 0, d.nx, 0, d.nx, d.nx, d.nx, d.nx, nullptr, true, false}; });
-    sized(QR_CHOL_SIGN);
-    stage(QR_CHOL_WRITE, 0, 0, l32_at, int64_t(l32.size()));
-}
-
-void Batch::flush_qr() {
-    flush_qr_chol();
-    flush_decomp(QR, pqr_, pqr_cost_, QR_LDS_MAX, qr_plain_doubles);
-}
+void Batch::flush_qr() { flush_decomp(QR, pqr_, pqr_cost_, QR_LDS_MAX, qr_doubles); }
 
 void Batch::svd(const std::vector<SvdTask>& ts, void* const* bufs, int64_t es, double* scratch) {
     double* cur = scratch;
@@ -479,34 +393,6 @@ void Batch::svd(const std::vector<SvdTask>& ts, void* const* bufs, int64_t es, d
         pend_units_[SVD] += fl;
         psvd_.push_back(s);
         psvd_cost_.push_back(fl);
-    }
-}
-
-void Batch::product(const std::vector<Product>& ps, int timed) {
-    std::vector<GemmDev> g(ps.size());
-    std::vector<TileDev> tiles[2];
-    for (size_t i = 0; i < ps.size(); i++) {
-        const Product& p = ps[i];
-        g[i] = GemmDev{p.a, p.b, p.c, p.m, p.n, p.k, p.lda, p.ldb, p.n, p.ta, p.tb, 1.0, p.skip};
-        const int v = std::max(p.m, p.n) <= 48 ? 0 : 1, w = GEMM_TILE_OF[v];
-        for (int x = 0; x * w < p.m; x++)
-            for (int y = p.upper ? x : 0; y * w < p.n; y++)
-                tiles[v].push_back(TileDev{int32_t(i), x, y, p.lower_a ? (x + 1) * w : 0});
-    }
-    const size_t goff = put(g);
-    for (int v = 0; v < 2; v++) {
-        if (tiles[v].empty()) continue;
-        Cmd c;
-        c.kind = GEMM;
-        c.stage = 0;
-        c.timed = timed;
-        c.tasks = goff;
-        c.prefix = put(tiles[v]);
-        c.count = int64_t(ps.size());
-        c.nwg = int64_t(tiles[v].size());
-        c.rpt = v;
-        c.dt = 0;
-        cmds_.push_back(c);
     }
 }
 
@@ -558,7 +444,6 @@ void Batch::flush_svd_eig() {
         Cmd c;
         c.kind = SVD_EIG;
         c.stage = st;
-        c.timed = KernelTimer::SVD_EIG;
         c.rpt = variant;
         c.tasks = toff + first * sizeof(SvdEigDev);
         c.prefix = list ? put(*list) : 0;
@@ -580,28 +465,54 @@ void Batch::flush_svd_eig() {
             for (int j = 0; j * width < tasks[i].kx; j++) l.push_back(TileDev{int32_t(i - base), j, 0, 0});
         return l;
     };
-    auto set = [](Product& g, const double* a, int ta, int lda, const double* b, int tb, int ldb, double* c, int m, int n,
-                  int k) { g = Product{a, b, c, ta, lda, tb, ldb, m, n, k, nullptr}; };
+    // a product per task in the double kernels, whatever the batch's type
     auto product = [&](auto fill) {
-        std::vector<Product> ps(T);
-        for (size_t i = 0; i < T; i++) fill(tasks[i], ps[i]);
-        this->product(ps, KernelTimer::SVD_EIG);
+        std::vector<GemmDev> g(T);
+        std::vector<TileDev> tiles[2];
+        for (size_t i = 0; i < T; i++) {
+            g[i].alpha = 1.0;
+            fill(tasks[i], g[i]);
+            const int v = std::max(g[i].m, g[i].n) <= 48 ? 0 : 1, w = GEMM_TILE_OF[v];
+            for (int x = 0; x * w < g[i].m; x++)
+                for (int y = 0; y * w < g[i].n; y++) tiles[v].push_back(TileDev{int32_t(i), x, y, 0});
+        }
+        const size_t goff = put(g);
+        for (int v = 0; v < 2; v++) {
+            if (tiles[v].empty()) continue;
+            Cmd c;
+            c.kind = GEMM;
+            c.stage = 0;
+            c.tasks = goff;
+            c.prefix = put(tiles[v]);
+            c.count = int64_t(T);
+            c.nwg = int64_t(tiles[v].size());
+            c.rpt = v;
+            c.dt = 0;
+            cmds_.push_back(c);
+        }
+    };
+    auto set = [](GemmDev& g, const double* a, int ta, int lda, const double* b, int tb, int ldb, double* c, int m, int n,
+                  int k) {
+        g.a = a;
+        g.ta = ta;
+        g.lda = lda;
+        g.b = b;
+        g.tb = tb;
+        g.ldb = ldb;
+        g.c = c;
+        g.ldc = n;
+        g.m = m;
+        g.n = n;
+        g.k = k;
     };
     const int64_t num = int64_t(T);
     const size_t first_cmd = cmds_.size();
     stage(SVD_EIG_LOAD, 0, 0, nullptr, num);
     cmds_[first_cmd].units = units;
-    product([&](SvdEigDev& d, Product& g) { set(g, d.xt, 0, d.mx, d.xt, 1, d.mx, d.b, d.kx, d.kx, d.mx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.xt, 0, d.mx, d.xt, 1, d.mx, d.b, d.kx, d.kx, d.mx); });
     static const int hi[5] = {64, 128, 192, 320, SVD_EIG_MAX_COLS};
-    const bool one = range(0, 192).second - range(0, 192).first <= size_t(ONE_WAVE_TASKS);
     for (int v = 4; v >= 0; v--) {
-        auto [a, b] = range(v ? hi[v - 1] : 0, hi[v]);
-        if (one && v < 3) {
-            // the class of the largest of them takes them all
-            const auto all = range(0, 192);
-            if (b <= a || a != all.first) continue;
-            b = all.second;
-        }
+        const auto [a, b] = range(v ? hi[v - 1] : 0, hi[v]);
         if (b > a) stage(SVD_EIG_TRIDIAG, v, a, nullptr, int64_t(b - a));
     }
     const auto l16 = list(16, 0, T, 0), l64 = list(64, 0, T, 0), l32 = list(32, 0, T, 0);
@@ -613,20 +524,20 @@ void Batch::flush_svd_eig() {
         const auto l = list(64, a, b, 0);
         stage(SVD_EIG_BACK, v, 0, &l, int64_t(l.size()));
     }
-    product([&](SvdEigDev& d, Product& g) { set(g, d.z, 1, d.kx, d.z, 0, d.kx, d.s, d.kx, d.kx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.z, 1, d.kx, d.z, 0, d.kx, d.s, d.kx, d.kx, d.kx); });
     stage(SVD_EIG_POLISH, 0, 0, nullptr, num);
-    product([&](SvdEigDev& d, Product& g) { set(g, d.s, 0, d.kx, d.z, 1, d.kx, d.vt, d.kx, d.kx, d.kx); });
-    product([&](SvdEigDev& d, Product& g) { set(g, d.vt, 0, d.kx, d.xt, 0, d.mx, d.xt2, d.kx, d.mx, d.kx); });
-    product([&](SvdEigDev& d, Product& g) { set(g, d.xt2, 0, d.mx, d.xt2, 1, d.mx, d.b, d.kx, d.kx, d.mx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.s, 0, d.kx, d.z, 1, d.kx, d.vt, d.kx, d.kx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.vt, 0, d.kx, d.xt, 0, d.mx, d.xt2, d.kx, d.mx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.xt2, 0, d.mx, d.xt2, 1, d.mx, d.b, d.kx, d.kx, d.mx); });
     stage(SVD_EIG_REFINE, 0, 0, nullptr, num);
-    product([&](SvdEigDev& d, Product& g) {
+    product([&](SvdEigDev& d, GemmDev& g) {
         set(g, d.b, 0, d.kx, d.b, 0, d.kx, d.s, d.kx, d.kx, d.kx);
         g.skip = d.flags + 3;
     });
     stage(SVD_EIG_SECOND, 0, 0, nullptr, num);
-    product([&](SvdEigDev& d, Product& g) { set(g, d.b, 1, d.kx, d.xt2, 0, d.mx, d.xt, d.kx, d.mx, d.kx); });
-    product([&](SvdEigDev& d, Product& g) { set(g, d.b, 1, d.kx, d.vt, 0, d.kx, d.z, d.kx, d.kx, d.kx); });
-    product([&](SvdEigDev& d, Product& g) {
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.b, 1, d.kx, d.xt2, 0, d.mx, d.xt, d.kx, d.mx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) { set(g, d.b, 1, d.kx, d.vt, 0, d.kx, d.z, d.kx, d.kx, d.kx); });
+    product([&](SvdEigDev& d, GemmDev& g) {
         set(g, d.xt, 0, d.mx, d.xt, 1, d.mx, d.b, d.kx, d.kx, d.mx);
         g.skip = d.flags + 3;
     });
@@ -695,10 +606,6 @@ void Batch::run(hipStream_t st) {
             case QR:
                 launch_qr(reinterpret_cast<const QrDev*>(base + c.tasks), c.count, c.lds, c.rpt, dtype_, st);
                 break;
-            case QR_CHOL:
-                launch_qr_chol(c.stage, c.rpt, reinterpret_cast<const QrCholDev*>(base + c.tasks),
-                               reinterpret_cast<const TileDev*>(base + c.prefix), c.count, dtype_, st);
-                break;
             case SVD_EIG:
                 launch_svd_eig(c.stage, c.rpt, reinterpret_cast<const SvdEigDev*>(base + c.tasks),
                                reinterpret_cast<const TileDev*>(base + c.prefix), c.count, dtype_, st);
@@ -711,7 +618,7 @@ void Batch::run(hipStream_t st) {
             check_hip(hipEventRecord(eb, st), "timer record");
             int k = int(c.kind);
             if (c.kind == QR && c.rpt == 1) k = KernelTimer::QR_BLOCKED;
-            if (c.stage >= 0) k = c.timed;
+            if (c.stage >= 0) k = KernelTimer::SVD_EIG;
             if (c.kind == SVD && c.rpt == 8) k = KernelTimer::SVD_REG8;
             if (c.kind == SVD && c.rpt == 16) k = KernelTimer::SVD_REG16;
             if (c.kind == SVD && c.rpt == 24) k = KernelTimer::SVD_REG24;

@@ -60,7 +60,7 @@ class Staging {
 struct KernelTimer {
     // one entry per kernel (variant) so that launch averages compare with a
     // kernel trace: QR / SVD are the LDS and unblocked-global kernels
-    enum { PERM, FILL, GEMM, QR, SVD, DIAG, QR_BLOCKED, SVD_REG8, SVD_REG16, SVD_REG24, SVD_EIG, QR_CHOL, NKIND };
+    enum { PERM, FILL, GEMM, QR, SVD, DIAG, QR_BLOCKED, SVD_REG8, SVD_REG16, SVD_REG24, SVD_EIG, NKIND };
     struct Acc {
         double ms = 0, units = 0, launches = 0;
     } acc[NKIND];
@@ -131,14 +131,12 @@ class Batch {
     void reset();
     void set_timer(KernelTimer* t) { timer_ = t; }
     void set_staging(Staging* s) { staging_ = s; }
-    // QR scratch without room for the Cholesky path: Householder only
-    void set_plain_qr(bool on) { plain_qr_ = on; }
     // large SVD blocks may use the register-resident kernel, whose V is
     // recovered from U (no orthonormal completion for zero singular values)
     void set_fast_svd(bool on) { fast_svd_ = on; }
 
    private:
-    enum Kind { PERM, FILL, GEMM, QR, SVD, DIAG, SVD_EIG, QR_CHOL };
+    enum Kind { PERM, FILL, GEMM, QR, SVD, DIAG, SVD_EIG };
     struct Cmd {
         Kind kind;
         size_t tasks, prefix;  // blob offsets (prefix: GEMM tiles, permute / fill units)
@@ -148,27 +146,15 @@ class Batch {
         int rpt = 0;       // register tile of the large-block SVD kernel
         int dt = -1;       // element type / GEMM precision override (-1: batch dtype)
         int conv = 0;      // permute conversion (1: f64 -> f32, 2: f32 -> f64)
-        int stage = -1;    // stage of the eigenvector SVD or the Cholesky QR (their products too)
-        int timed = -1;    // KernelTimer kind of such a stage
+        int stage = -1;    // stage of the eigenvector SVD (its products too: their time counts there)
     };
     template<typename D>
     void flush_decomp(Kind kind, std::vector<D>& tasks, std::vector<double>& cost, int64_t lds_max,
                       int64_t (*doubles)(int64_t, int64_t));  // doubles: the kernels' working set in LDS
     KernelTimer* timer_ = nullptr;
     Staging* staging_ = nullptr;
-    double pend_units_[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    double pend_units_[7] = {0, 0, 0, 0, 0, 0, 0};
     void flush_svd_eig();
-    void flush_qr_chol();
-    // products of the staged paths: always double, one task per sector
-    struct Product {
-        const double *a, *b;
-        double* c;
-        int ta, lda, tb, ldb, m, n, k;
-        const int32_t* skip;
-        // the result's upper triangle only / a is lower triangular
-        bool upper = false, lower_a = false;
-    };
-    void product(const std::vector<Product>& ps, int timed);
     template<typename T>
     size_t put(const std::vector<T>& v);
     void flush_flat(Kind kind, std::vector<PermDev>& pd, std::vector<FillDev>& fd);
@@ -187,7 +173,7 @@ class Batch {
     std::vector<double> pqr_cost_, psvd_cost_;
     int64_t perm_elems_ = 0;
     double* scratch_cursor_ = nullptr;
-    bool fast_svd_ = false, plain_qr_ = false;
+    bool fast_svd_ = false;
 };
 
 }  // namespace tns

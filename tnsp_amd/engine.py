@@ -98,7 +98,7 @@ class AmplitudeEngine:
         return dict(zip(STAT_NAMES, list(vals)))
 
     KERNEL_KINDS = ["permute", "fill", "gemm", "qr", "svd", "diag", "qr_blocked", "svd_reg8", "svd_reg16", "svd_reg24",
-                    "svd_eig", "qr_chol"]
+                    "svd_eig"]
 
     def set_profile(self, on=True):
         _lib.check(_lib.lib().tns_engine_set_profile(self.handle, int(bool(on))))
