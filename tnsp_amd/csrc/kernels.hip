@@ -465,7 +465,8 @@ __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau,
     }
     amax = block_max<QR_WG>(amax, red);
     // blocks whose squares would vanish or overflow work on entries of order one
-    // (without it a block of 1e-200 looks like zero columns and gets no reflectors)
+    // (without it a block of 1e-200 looks like zero columns and gets no reflectors);
+    // 64 x 30, 2 blocks a call 124.5 -> 128.9 us (runs of one side differ by 4.7%)
     const int shift = amax > 0.0 && amax <= 1.79e308 && (amax < 1e-140 || amax > 1e140) ? -ilogb(amax) : 0;
     if (shift)
         for (int64_t e = tid; e < int64_t(mx) * nx; e += QR_WG) X[e] = ldexp(X[e], shift);
