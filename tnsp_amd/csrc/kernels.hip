@@ -1068,27 +1068,54 @@ __device__ __forceinline__ void svd_body(const SvdDev& tk, double* X, double* V,
         for (int c = 0; c < kx; c++) {
             if (sig[c] > 0.0) continue;
             double* xc = X + int64_t(c) * mx;
-            for (int j = 0; j < mx; j++) {
-                for (int r = gl; r < mx; r += G) xc[r] = (r == j) ? 1.0 : 0.0;
-                for (int pass = 0; pass < 2; pass++) {
+            // from the first unit vector that keeps half its length outside
+            // the other columns' span, or the one that keeps most (a square
+            // block with one null column: none may keep more than 1 / sqrt(mx))
+            double most = -1.0;
+            int at = 0;
+            for (int r0 = 0; r0 < mx && most <= 0.25; r0 += G) {
+                const int r = r0 + gl;
+                double left = -1.0;
+                if (r < mx) {
+                    left = 1.0;
                     for (int d = 0; d < kx; d++) {
                         if (d == c || (sig[d] <= 0.0 && d > c)) continue;
-                        const double* xd = X + int64_t(d) * mx;
-                        double dot = 0;
-                        for (int r = gl; r < mx; r += G) dot += xc[r] * xd[r];
-                        dot = group_sum(dot, G);
-                        for (int r = gl; r < mx; r += G) xc[r] -= dot * xd[r];
+                        const double q = X[int64_t(d) * mx + r];
+                        left -= q * q;
                     }
                 }
-                double nn = 0;
-                for (int r = gl; r < mx; r += G) nn += xc[r] * xc[r];
-                nn = group_sum(nn, G);
-                if (nn > 0.25) {
-                    const double inv = 1.0 / sqrt(nn);
-                    for (int r = gl; r < mx; r += G) xc[r] *= inv;
-                    break;
+                // the first above a quarter, else the largest
+                double top = left > 0.25 ? 4.0 - 0x1p-6 * gl : left;
+                int where = r;
+                for (int o = 1; o < G; o <<= 1) {
+                    const double other = __shfl_xor(top, o, WAVE);
+                    const int there = __shfl_xor(where, o, WAVE);
+                    if (other > top || (other == top && there < where)) {
+                        top = other;
+                        where = there;
+                    }
+                }
+                if (top > most) {
+                    most = top;
+                    at = where;
                 }
             }
+            for (int r = gl; r < mx; r += G) xc[r] = (r == at) ? 1.0 : 0.0;
+            for (int pass = 0; pass < 2; pass++) {
+                for (int d = 0; d < kx; d++) {
+                    if (d == c || (sig[d] <= 0.0 && d > c)) continue;
+                    const double* xd = X + int64_t(d) * mx;
+                    double dot = 0;
+                    for (int r = gl; r < mx; r += G) dot += xc[r] * xd[r];
+                    dot = group_sum(dot, G);
+                    for (int r = gl; r < mx; r += G) xc[r] -= dot * xd[r];
+                }
+            }
+            double nn = 0;
+            for (int r = gl; r < mx; r += G) nn += xc[r] * xc[r];
+            nn = group_sum(nn, G);
+            const double inv = 1.0 / sqrt(nn);
+            for (int r = gl; r < mx; r += G) xc[r] *= inv;
             // the completed column orthogonalises the later ones
             if (gl == 0) sig[c] = -sig[c];
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");

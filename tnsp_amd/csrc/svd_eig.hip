@@ -726,11 +726,14 @@ __global__ __launch_bounds__(1024) void eig_verify_kernel(const SvdEigDev* __res
 
 // Singular values (column norms), their descending order (ties by column),
 // the directions of null columns and the mark that takes the block from the
-// Jacobi kernels.  A null column keeps its tiny norm as its singular value; its
-// direction is the first unit vector that keeps half its length after two
-// passes of Gram-Schmidt against every other column.
+// Jacobi kernels.  A null column keeps its tiny norm as its singular value.  Its
+// direction starts from the first unit vector that keeps half its length
+// outside the other columns' span, or from the one that keeps most (in a
+// square block with one null column none may keep more than 1 / sqrt(mx)), and is
+// what two passes of Gram-Schmidt against every other column leave of it.
 __global__ __launch_bounds__(1024) void eig_order_kernel(const SvdEigDev* __restrict__ tasks) {
     __shared__ double sg[SVD_EIG_MAX_COLS], inv[SVD_EIG_MAX_COLS], coef[SVD_EIG_MAX_COLS], red[16];
+    __shared__ int pos[16];
     const SvdEigDev tk = tasks[blockIdx.x];
     const int n = tk.kx, mx = tk.mx, tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     if (n > SVD_EIG_MAX_COLS || tk.flags[1]) return;
@@ -758,35 +761,62 @@ __global__ __launch_bounds__(1024) void eig_order_kernel(const SvdEigDev* __rest
     __syncthreads();
     for (int c = 0; c < n; c++) {
         if (inv[c] > 0.0) continue;  // uniform over the workgroup
-        for (int j = 0; j < mx; j++) {
-            for (int r = tid; r < mx; r += 1024) X[c * mx + r] = r == j ? 1.0 : 0.0;
-            for (int pass = 0; pass < 2; pass++) {
-                __syncthreads();
-                for (int d = wave; d < n; d += 16) {
-                    double s = 0.0;
-                    if (inv[d] > 0.0)
-                        for (int r = lane; r < mx; r += WAVE) s += X[c * mx + r] * X[d * mx + r];
-                    s = wave_sum(s);
-                    if (lane == 0) coef[d] = s * inv[d] * inv[d];
-                }
-                __syncthreads();
-                for (int r = tid; r < mx; r += 1024) {
-                    double v = X[c * mx + r];
-                    for (int d = 0; d < n; d++)
-                        if (inv[d] > 0.0) v -= coef[d] * X[d * mx + r];
-                    X[c * mx + r] = v;
+        // squared length of each unit vector outside the span, 1024 at a time
+        double most = -1.0;
+        int at = 0;
+        for (int r0 = 0; r0 < mx && most <= 0.25; r0 += 1024) {
+            const int r = r0 + tid;
+            double left = -1.0;
+            if (r < mx) {
+                left = 1.0;
+                for (int d = 0; d < n; d++) {
+                    const double q = X[d * mx + r] * inv[d];
+                    left -= q * q;
                 }
             }
+            // the first above a quarter, else the largest
+            const double score = left > 0.25 ? 4.0 - 0x1p-10 * tid : left, top = wave_max(score);
+            const int lane_at = __builtin_ctzll(__ballot(score == top));
             __syncthreads();
-            double s = 0.0;
-            for (int r = lane; r < mx; r += WAVE) s += X[c * mx + r] * X[c * mx + r];
-            s = wave_sum(s);  // every wave: the same value
-            if (s > 0.25) {
-                if (tid == 0) inv[c] = 1.0 / sqrt(s);
-                break;
+            if (lane == 0) {
+                red[wave] = top;
+                pos[wave] = r0 + WAVE * wave + lane_at;
             }
             __syncthreads();
+            for (int w = 0; w < 16; w++)
+                if (red[w] > most) {
+                    most = red[w];
+                    at = pos[w];
+                }
         }
+        for (int r = tid; r < mx; r += 1024) X[c * mx + r] = r == at ? 1.0 : 0.0;
+        for (int pass = 0; pass < 2; pass++) {
+            __syncthreads();
+            for (int d = wave; d < n; d += 16) {
+                double s = 0.0;
+                if (inv[d] > 0.0)
+                    for (int r = lane; r < mx; r += WAVE) s += X[c * mx + r] * X[d * mx + r];
+                s = wave_sum(s);
+                if (lane == 0) coef[d] = s * inv[d] * inv[d];
+            }
+            __syncthreads();
+            for (int r = tid; r < mx; r += 1024) {
+                double v = X[c * mx + r];
+                for (int d = 0; d < n; d++)
+                    if (inv[d] > 0.0) v -= coef[d] * X[d * mx + r];
+                X[c * mx + r] = v;
+            }
+        }
+        __syncthreads();
+        double s = 0.0;
+        for (int r = lane; r < mx; r += WAVE) s += X[c * mx + r] * X[c * mx + r];
+        s = wave_sum(s);  // every wave: the same value
+        // at least 1 / kx keeps some unit vector; what did not is not for here
+        if (!(s > 1e-4)) {
+            if (tid == 0) tk.flags[1] = 1;
+            return;
+        }
+        if (tid == 0) inv[c] = 1.0 / sqrt(s);
         __syncthreads();
     }
     for (int c = tid; c < n; c += 1024) {
