@@ -207,6 +207,7 @@ int tns_conv3x3_forward(const float* x, const uint16_t* w, const float* bias, fl
                         int height, int width, int relu, void* stream);
 int tns_conv3x3_backward_data(const float* dy, const float* relu_y, const uint16_t* w, float* dx, int batch, int cin,
                               int cout, int height, int width, void* stream);
+/* bytes that suffice for the given batch and every smaller one */
 int tns_conv3x3_backward_weight_workspace(int batch, int cin, int cout, int64_t* bytes);
 int tns_conv3x3_backward_weight(const float* dy, const float* relu_y, const float* x, float* dw, float* dbias,
                                 int batch, int cin, int cout, int height, int width, void* workspace, void* stream);

@@ -85,3 +85,19 @@ def test_apply_hops_and_bond_hops_match_oracle():
         sel = flat[:, ia] != flat[:, ib]
         h = bond_hop(flat[sel], ia, ib, L2, horiz)
         assert mask[np.nonzero(sel)[0], h].all()
+
+
+def test_weight_gradient_workspace_serves_smaller_batches():
+    """A workspace of the largest batch is enough for every smaller one (the
+    run takes no size, so a program may keep it).  Chunks of samples: the
+    query of a batch is never below that of a smaller one."""
+    import ctypes
+
+    from tnsp_amd import _lib
+
+    ws = ctypes.c_int64()
+    last = 0
+    for batch in range(0, 2200):
+        _lib.check(_lib.lib().tns_conv3x3_backward_weight_workspace(batch, 32, 32, ctypes.byref(ws)))
+        assert ws.value >= last, batch
+        last = ws.value

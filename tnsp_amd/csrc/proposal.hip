@@ -435,11 +435,15 @@ namespace {
 // each at 32 channels) stay a small part of the traffic.  1024 samples of 32
 // channels, 8 x 8, all four layers with the reductions: 143 us with 2 samples
 // per workgroup, 165 us with 4, 296 us with 8.
-int conv_chunk(int B) { return std::max(1, (B + 511) / 512); }
+constexpr int CONV_CHUNKS_MAX = 512;
+int conv_chunk(int B) { return std::max(1, (B + CONV_CHUNKS_MAX - 1) / CONV_CHUNKS_MAX); }
 }  // namespace
 
+// Enough for every batch up to B, not only for B (513 samples make 257
+// workgroups of two, 512 make 512 of one): a caller may keep the workspace of
+// its largest batch.
 int64_t conv_bwd_weight_workspace(int B, int cin, int cout) {
-    const int chunks = B > 0 ? (B + conv_chunk(B) - 1) / conv_chunk(B) : 0;
+    const int chunks = std::max(0, std::min(B, CONV_CHUNKS_MAX));
     return int64_t(chunks) * (int64_t(cout) * cin * 9 + cout) * int64_t(sizeof(float));
 }
 
