@@ -137,3 +137,30 @@ def test_trim_keeps_psi():
     eng.trim()
     eng.trim()
     assert np.array_equal(first, again) and np.array_equal(eng.evaluate(configs[:3]), first[:3])
+
+
+def launches(eng):
+    return {k: v["launches"] for k, v in eng.kernel_stats().items()}
+
+
+def test_profiling_stops_when_switched_off():
+    """What runs while profiling is off is in no kernel statistics, also
+    after it is switched on again."""
+    from tnsp_amd import peps as ppeps
+    from tnsp_amd.engine import AmplitudeEngine
+
+    spec, storages, configs, _ = c2_case()
+    eng = AmplitudeEngine(ppeps.Lattice(spec, storages), chunk=8, lanes=1)
+    eng.evaluate(configs[:8])
+    eng.set_profile(True)
+    eng.evaluate(configs[:8])
+    eng.set_profile(False)
+    once = launches(eng)
+    assert sum(once.values()) > 0
+    eng.evaluate(configs[:8])
+    eng.evaluate(configs[:8])
+    assert launches(eng) == once
+    eng.set_profile(True)
+    eng.evaluate(configs[:8])
+    eng.set_profile(False)
+    assert launches(eng) == {k: 2 * v for k, v in once.items()}

@@ -229,7 +229,7 @@ void Engine::grow_all(hipStream_t st) {
 void Engine::run_batch(Batch& b, hipStream_t st) {
     const double t0 = now();
     stats_.perm_elems += double(b.perm_elements());
-    if (profile_) b.set_timer(&timer_);
+    b.set_timer(profile_ ? &timer_ : nullptr);  // the batch outlives the call
     b.set_staging(&staging_);
     b.run(st);
     stats_.exec_s += now() - t0;
