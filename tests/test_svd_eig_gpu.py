@@ -1,4 +1,4 @@
-"""The eigenvector path of the sector SVD (blocks of 32 to 640 columns) at the
+"""The eigenvector path of the sector SVD (blocks of 24 to 640 columns) at the
 edges of its tiles, and blocks it has to leave to the Jacobi kernels, against
 numpy's LAPACK.
 
@@ -139,3 +139,21 @@ def test_equal_columns_float32(n):
     x = np.random.default_rng(n).standard_normal((n, n)).astype(np.float32)
     x[:, 7] = x[:, 31]
     check_orthonormal(x, "S")
+
+
+@pytest.mark.parametrize("first", [(24, 24), (23, 31), (23, 23), (16, 31), (31, 20), (8, 9)])
+def test_sector_does_not_depend_on_its_company(first):
+    """A sector alone and beside a larger one that takes the eigenvector path:
+    the same bits."""
+    from tnsp_amd import TAT
+
+    m, n = first
+    x = np.random.default_rng(m + n).standard_normal((m, n))
+    alone = TAT.BoseU1.D.Tensor(["a", "b"], [[(0, m)], [(0, n)]])
+    pair = TAT.BoseU1.D.Tensor(["a", "b"], [[(0, m), (1, 70)], [(0, n), (-1, 64)]])
+    pair.storage = np.random.default_rng(1).standard_normal(pair.storage.size)
+    pair.blocks[[("a", 0), ("b", 0)]] = x
+    alone.blocks[[("a", 0), ("b", 0)]] = x
+    for one, two in zip(alone.svd({"a"}, "U", "V", "SU", "SV"), pair.svd({"a"}, "U", "V", "SU", "SV")):
+        key = [(name, 0) for name in one.names]
+        assert np.array_equal(one.blocks[key], two.blocks[key])

@@ -126,12 +126,17 @@ inline int64_t qr_doubles(int64_t m, int64_t n) { return m * n + (m < n ? m : n)
 // path: 64 tensors with sectors up to about 200 x 190 (some beyond the register
 // kernel's 192 rows) 98.6 -> 4.8 ms; 4 tensors with sectors up to about
 // 310 x 260 199 -> 5.4 ms; one stage of 128 8x8 D=8 configurations (register
-// 24 / 16 and LDS kernels, one after the other) 11.1 -> 4.9 ms.  Sectors of 16
-// to 31 columns ride along with larger ones (the LDS kernel's launch then takes
-// 198 instead of 294 us per stage of those configurations); alone, the path's
-// ~25 launches cost more than the LDS kernel's rounds.  Above 640 columns the
-// eigenvector strips no longer fit the registers of one wave.
-constexpr int SVD_EIG_MIN_COLS = 16, SVD_EIG_ALONE_COLS = 32, SVD_EIG_MAX_COLS = 640;
+// 24 / 16 and LDS kernels, one after the other) 11.1 -> 4.9 ms.  The lower line:
+// tensors of one sector, whole passes with the LDS Jacobi kernel against this
+// path, 1, 16 and 200 tensors a call: 31 x 30 599 / 1146 / 3118 against 415 /
+// 1005 / 3152 us, 140 x 28 567 / 1140 / 3193 against 433 / 1045 / 3047, 24 x 24
+// 483 / 1015 / 3029 against 360 / 996 / 3253 (runs of one side differ by 19% at
+// 200), 30 x 20 433 / 909 / 2792 against 360 / 1002 / 3205, 200 x 16 390 / 889 /
+// 2894 against 347 / 965 / 3149: below 24 columns many small sectors lose.  The
+// sector's size alone decides, so that its factors do not depend on what shares
+// its launch.  Above 640 columns the eigenvector strips no longer fit the
+// registers of one wave.
+constexpr int SVD_EIG_MIN_COLS = 24, SVD_EIG_MAX_COLS = 640;
 inline bool svd_eig_fits(int64_t m, int64_t n) {
     const int64_t mx = m > n ? m : n, kx = m < n ? m : n;
     return kx >= SVD_EIG_MIN_COLS && kx <= SVD_EIG_MAX_COLS && mx * kx <= (int64_t(1) << 28);

@@ -405,7 +405,7 @@ void Batch::flush_svd_eig() {
         if (fast_svd_ && svd_eig_fits(psvd_[i].m, psvd_[i].n)) sel.push_back(i);
     auto cols = [&](size_t i) { return std::min(psvd_[i].m, psvd_[i].n); };
     std::stable_sort(sel.begin(), sel.end(), [&](size_t a, size_t b) { return cols(a) > cols(b); });
-    if (sel.empty() || cols(sel[0]) < SVD_EIG_ALONE_COLS) return;
+    if (sel.empty()) return;
     const size_t T = sel.size();
     std::vector<SvdEigDev> tasks(T);
     double units = 0;
