@@ -753,13 +753,15 @@ __global__ __launch_bounds__(1024) void eig_order_kernel(const SvdEigDev* __rest
     fro = 0.0;
     for (int w = 0; w < 16; w++) fro += red[w];
     const double live = fmax(JACOBI_QUIET, JACOBI_DEAD2 * fro);
+    bool null = false;
     for (int c = tid; c < n; c += 1024) {
         const double s = sg[c], root = sqrt(s);
         inv[c] = s > live ? 1.0 / root : 0.0;  // 0: no direction yet
+        null = null || !(inv[c] > 0.0);
         sg[c] = root;
     }
-    __syncthreads();
-    for (int c = 0; c < n; c++) {
+    const int last = __syncthreads_or(null) ? n : 0;
+    for (int c = 0; c < last; c++) {
         if (inv[c] > 0.0) continue;  // uniform over the workgroup
         // squared length of each unit vector outside the span, 1024 at a time
         double most = -1.0;
