@@ -48,7 +48,7 @@ def check(x, dtype, lq, same=True):
 
 @pytest.mark.parametrize("n", [20, 40, 100])
 @pytest.mark.parametrize("kind", ["triangular", "identity", "diagonal", "rank", "zero_column", "graded_columns",
-                                  "ill_conditioned", "tiny", "huge", "zero_rows"])
+                                  "ill_conditioned", "tiny", "huge", "overflowing", "zero_rows"])
 def test_special_blocks(n, kind):
     """The result is a QR; where Q and R are determined by the
     block (full rank, well conditioned) they have the Householder signs."""
@@ -76,7 +76,28 @@ def test_special_blocks(n, kind):
         x = x * 1e-200
     elif kind == "huge":
         x = x * 1e150
+    elif kind == "overflowing":
+        x = x * 1e250
     elif kind == "zero_rows":
         x[n // 2:] = 0.0
         same = False
     check(x, "D", False, same)
+
+
+@pytest.mark.parametrize("lq", [False, True])
+def test_huge_block_keeps_its_tiny_columns(lq):
+    """Columns of 1e145 and of 1e-150 side by side: the squares of both are
+    finite, so the range scaling must not flush the small ones."""
+    x = np.random.default_rng(3).standard_normal((50, 20))
+    x[:, ::2] *= 1e145
+    x[:, 1::2] *= 1e-150
+    q, r = dense_qr(x.T if lq else x, "D", lq)
+    tol = 4 * 50 * EPS["D"]
+    assert np.max(np.abs(q.T @ q - np.eye(20))) <= tol
+    q0, r0 = np.linalg.qr(x)
+    # column by column: a column of R has the length of the block's
+    for c in range(20):
+        size = 1e145 if c % 2 == 0 else 1e-150
+        small = np.abs(r0[:, c]) <= 10 * size
+        assert np.all(small)
+        assert np.linalg.norm((q @ (r[:, c] / size)) - x[:, c] / size) <= tol * np.linalg.norm(x[:, c] / size)

@@ -165,18 +165,6 @@ __device__ inline double block_sum(double v, double* red) {
     return t;
 }
 
-template<int NT>
-__device__ inline double block_max(double v, double* red) {
-    v = wave_max(v);
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    __syncthreads();
-    if (lane == 0) red[wave] = v;
-    __syncthreads();
-    double t = red[0];
-    for (int w = 1; w < NT / WAVE; w++) t = fmax(t, red[w]);
-    return t;
-}
-
 // hardware reciprocal / reciprocal square root refined by two Newton steps
 __device__ inline double refined_rcp(double x) {
     double r = __builtin_amdgcn_rcp(x);

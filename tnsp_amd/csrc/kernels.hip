@@ -449,7 +449,10 @@ __device__ inline int qr_group_lanes(int rows, int cols) {
     return G;
 }
 
-template<typename T>
+// I: type of element indices.  32 bits where the block is in LDS: the passes that
+// load it and write R and Q divide once per element, and 64-bit divisions took
+// longer there than the range test.
+template<typename T, typename I>
 __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau, double* red, double* bc) {
     const int m = tk.m, n = tk.n, lq = tk.lq;
     const int mx = lq ? n : m, nx = lq ? m : n, k = mx < nx ? mx : nx;
@@ -457,30 +460,56 @@ __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau,
     const int tid = threadIdx.x;
     const int G = qr_group_lanes(mx, nx), NG = QR_WG / G, g = tid / G, gl = tid % G;
     double amax = 0;
-    for (int64_t e = tid; e < int64_t(mx) * nx; e += QR_WG) {
+    for (I e = tid; e < I(mx) * nx; e += QR_WG) {
         const int r = int(e % mx), c = int(e / mx);
-        const double x = double(lq ? in[int64_t(c) * n + r] : in[int64_t(r) * n + c]);
+        const double x = double(lq ? in[I(c) * n + r] : in[I(r) * n + c]);
         X[e] = x;
         amax = fmax(amax, fabs(x));
     }
-    amax = block_max<QR_WG>(amax, red);
-    // blocks whose squares would vanish or overflow work on entries of order one
-    // (without it a block of 1e-200 looks like zero columns and gets no reflectors);
-    // 64 x 30, 2 blocks a call 124.5 -> 128.9 us (runs of one side differ by 4.7%)
-    const int shift = amax > 0.0 && amax <= 1.79e308 && (amax < 1e-140 || amax > 1e140) ? -ilogb(amax) : 0;
-    if (shift)
-        for (int64_t e = tid; e < int64_t(mx) * nx; e += QR_WG) X[e] = ldexp(X[e], shift);
-    __syncthreads();
     // squared norm below the diagonal of the column to reduce: a block sum
-    // for column 0, then from the group that updates the next column
-    double sigma;
+    // for column 0, with the block's largest entry on the way, then from the
+    // group that updates the next column
+    double sigma = 0;
     {
+        double* big = red + QR_WG / WAVE;
+        const int lane = tid % WAVE, wave = tid / WAVE;
+        amax = wave_max(amax);
+        if (lane == 0) big[wave] = amax;
+        __syncthreads();
+        double s = 0;
+        for (int r = 1 + tid; r < mx; r += QR_WG) s += X[r] * X[r];
+        s = wave_sum(s);
+        if (lane == 0) red[wave] = s;
+        __syncthreads();
+        for (int w = 0; w < QR_WG / WAVE; w++) {
+            sigma += red[w];
+            amax = fmax(amax, big[w]);
+        }
+    }
+    // Blocks whose squares would vanish work on entries of order one (a block
+    // of 1e-200 looks like zero columns and gets no reflectors), blocks whose
+    // squared column norms could overflow on entries just below that, which
+    // spares their small columns.  Both are rare, and the test rides on column
+    // 0's barriers (two, without it three): launches of 69 blocks up to 140 x 138
+    // 392 us without and 389 us with it, 27 blocks 191 and 190, 96 small blocks
+    // 15.7 and 16.3.
+    int shift = 0;  // the same in every lane: the branches on it are scalar
+    if (amax > 0.0 && amax <= 1.79e308) {
+        if (amax < 1e-140)
+            shift = -ilogb(amax);
+        else if (!(amax * amax * mx <= 1e307))
+            shift = (1000 - ilogb(double(mx))) / 2 - ilogb(amax);
+    }
+    shift = __builtin_amdgcn_readfirstlane(shift);
+    if (shift) {
+        for (I e = tid; e < I(mx) * nx; e += QR_WG) X[e] = ldexp(X[e], shift);
+        __syncthreads();
         double s = 0;
         for (int r = 1 + tid; r < mx; r += QR_WG) s += X[r] * X[r];
         sigma = block_sum<QR_WG>(s, red);
     }
     for (int j = 0; j < k; j++) {
-        double* cj = X + int64_t(j) * mx;
+        double* cj = X + I(j) * mx;
         double tj, beta;
         householder(cj[j], sigma, tj, beta);
         if (tj != 0.0) {
@@ -500,24 +529,31 @@ __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau,
     T* f1 = static_cast<T*>(tk.f1);
     T* f2 = static_cast<T*>(tk.f2);
     // R (k x nx, upper trapezoid)
+    if (shift) {
+        for (I e = tid; e < I(k) * nx; e += QR_WG) {
+            const int r = int(e % k), c = int(e / k);
+            if (r <= c) X[I(c) * mx + r] = ldexp(X[I(c) * mx + r], -shift);
+        }
+        __syncthreads();
+    }
     if (!lq) {
-        for (int64_t e = tid; e < int64_t(k) * n; e += QR_WG) {
+        for (I e = tid; e < I(k) * n; e += QR_WG) {
             const int r = int(e / n), c = int(e % n);
-            f2[e] = T(r <= c ? (shift ? ldexp(X[int64_t(c) * mx + r], -shift) : X[int64_t(c) * mx + r]) : 0.0);
+            f2[e] = T(r <= c ? X[I(c) * mx + r] : 0.0);
         }
     } else {
-        for (int64_t e = tid; e < int64_t(m) * k; e += QR_WG) {
+        for (I e = tid; e < I(m) * k; e += QR_WG) {
             const int i = int(e / k), r = int(e % k);
-            f1[e] = T(r <= i ? (shift ? ldexp(X[int64_t(i) * mx + r], -shift) : X[int64_t(i) * mx + r]) : 0.0);
+            f1[e] = T(r <= i ? X[I(i) * mx + r] : 0.0);
         }
     }
     __syncthreads();
     for (int j = k - 1; j >= 0; j--) {
         const double tj = tau[j];
-        const double* v = X + int64_t(j) * mx;
+        const double* v = X + I(j) * mx;
         if (tj != 0.0) {
             for (int c = j + 1 + g; c < k; c += NG) {
-                double* qc = X + int64_t(c) * mx;
+                double* qc = X + I(c) * mx;
                 double d = 0;
                 for (int r = j + 1 + gl; r < mx; r += G) d += v[r] * qc[r];
                 d = group_sum(d, G) + qc[j];
@@ -527,7 +563,7 @@ __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau,
             }
         }
         __syncthreads();
-        double* cj = X + int64_t(j) * mx;
+        double* cj = X + I(j) * mx;
         for (int r = tid; r < mx; r += QR_WG) {
             if (r > j)
                 cj[r] *= -tj;
@@ -539,14 +575,14 @@ __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau,
         __syncthreads();
     }
     if (!lq) {
-        for (int64_t e = tid; e < int64_t(m) * k; e += QR_WG) {
+        for (I e = tid; e < I(m) * k; e += QR_WG) {
             const int r = int(e / k), c = int(e % k);
-            f1[e] = T(X[int64_t(c) * mx + r]);
+            f1[e] = T(X[I(c) * mx + r]);
         }
     } else {
-        for (int64_t e = tid; e < int64_t(k) * n; e += QR_WG) {
+        for (I e = tid; e < I(k) * n; e += QR_WG) {
             const int r = int(e / n), i = int(e % n);
-            f2[e] = T(X[int64_t(r) * mx + i]);
+            f2[e] = T(X[I(r) * mx + i]);
         }
     }
 }
@@ -554,20 +590,20 @@ __device__ __forceinline__ void qr_body(const QrDev& tk, double* X, double* tau,
 template<typename T>
 __global__ __launch_bounds__(QR_WG) void qr_kernel_lds(const QrDev* __restrict__ tasks) {
     extern __shared__ double smem[];
-    __shared__ double red[QR_WG / WAVE];
+    __shared__ double red[2 * QR_WG / WAVE];
     __shared__ double bc[1];
     const QrDev tk = tasks[blockIdx.x];
     const int mx = tk.lq ? tk.n : tk.m, nx = tk.lq ? tk.m : tk.n;
-    qr_body<T>(tk, smem, smem + int64_t(mx) * nx, red, bc);
+    qr_body<T, uint32_t>(tk, smem, smem + int64_t(mx) * nx, red, bc);
 }
 
 template<typename T>
 __global__ __launch_bounds__(QR_WG) void qr_kernel_glb(const QrDev* __restrict__ tasks) {
-    __shared__ double red[QR_WG / WAVE];
+    __shared__ double red[2 * QR_WG / WAVE];
     __shared__ double bc[1];
     const QrDev tk = tasks[blockIdx.x];
     const int mx = tk.lq ? tk.n : tk.m, nx = tk.lq ? tk.m : tk.n;
-    qr_body<T>(tk, tk.work, tk.work + int64_t(mx) * nx, red, bc);
+    qr_body<T, int64_t>(tk, tk.work, tk.work + int64_t(mx) * nx, red, bc);
 }
 
 // Blocked Householder QR for blocks that do not fit LDS (X in global
