@@ -91,7 +91,7 @@ int tns_plan_run(tns_plan* p, int dtype, const void* const* inputs, void* const*
  * reference (TAT allocates per op); it is for callers that cannot allocate:
  * code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc.  The plan's workspace (at most 64 MiB) and its task records (at
- * most 4 MiB) come from one static device array the library holds on each GPU
+ * most 9 MiB) come from one static device array the library holds on each GPU
  * until the process ends, instead of a caller workspace and the library's
  * growable staging.  A plan needing more workspace fails with an error
  * (before any device call); svd plans are refused (tns_svd_factor writes into

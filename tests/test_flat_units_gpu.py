@@ -1,6 +1,5 @@
-"""Permute and fill launches at the edges of their units (one wave handles 64
-elements, 512 per step, 512 / 2048 / 4096 per unit depending on the launch's
-total) against numpy.  Copies are exact, so results must be equal."""
+"""Permute and fill launches at the edges of their chunks (2048 elements, one
+workgroup) and units (the rest of a task, 512 per wave) against numpy.  Copies are exact, so results must be equal."""
 import numpy as np
 import pytest
 
@@ -8,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", ["D", "S"])
-@pytest.mark.parametrize("shape", [(1, 1), (3, 21), (8, 8), (5, 13), (7, 73), (16, 32), (27, 19), (2, 1024, 1),
+@pytest.mark.parametrize("shape", [(1, 1), (3, 21), (8, 8), (5, 13), (7, 73), (16, 32), (27, 19), (89, 23), (2, 1024, 1),
                                    (683, 3), (1449, 1449), (5, 29, 14465), (4099, 4097)])
 def test_transpose_equals_numpy(shape, dtype):
     from tnsp_amd import TAT

@@ -1,8 +1,8 @@
 // CDNA4 (gfx950) kernels for the block-sparse tensor path.
 //
 //  permute  : batched strided block copy with the fermion sign folded in; one
-//             wave per unit of a task, destination-ordered so that stores
-//             coalesce.
+//             workgroup per chunk or wave per unit of a task,
+//             destination-ordered so that stores coalesce.
 //  gemm     : grouped GEMM over heterogeneous sector blocks, one workgroup per
 //             32x32 output tile, 4 waves x MFMA 16x16x4 (fp64 / fp32).
 //  qr       : batched Householder QR / LQ, one workgroup per sector block.
@@ -49,19 +49,27 @@ __device__ inline void perm_decode(uint32_t local, int rank, const int32_t* dims
     }
 }
 
-// One wave per unit: FLAT_LANE x 64 consecutive elements of one task per
-// step, `elems` elements per unit, all loads of a step issued before its
-// stores.  What bounds the small launches is the time to the first load, not
-// bytes: a PEPS of bond dimension 4 makes thousands of tasks of 1 to 30
-// elements per launch.  The unit names its task, so a wave reads one
-// descriptor, through scalar loads, and searches nothing (walking prefix sums
-// thread by thread took 94 us per launch of 128 configurations of the 4x4
-// D=4 PEPS, the units 4.2 us; 50 and 32 us on the 8x8 D=8 one).  Lanes idle on a tiny task cost less than
-// the per-element descriptor reads that packing several tasks per wave needs.
+// A workgroup per chunk of a task, a wave per unit (a small task or a small
+// rest); a lane has FLAT_LANE elements, all loads issued before the stores.  What bounds the
+// small launches is the time to the first load, not bytes: a PEPS of bond
+// dimension 4 makes thousands of tasks of 1 to 30 elements per launch.  The
+// record names its task, so a wave reads one descriptor, through scalar loads,
+// and searches nothing (walking prefix sums thread by thread took 94 us per
+// launch of 128 configurations of the 4x4 D=4 PEPS, the units 4.2 us; 50 and
+// 32 us on the 8x8 D=8 one).  Lanes idle on a tiny task cost less than the
+// per-element descriptor reads that packing several tasks per wave needs.
+// Large tasks are bound by bytes and by how many lines their strided side
+// touches at a time: the waves of a chunk walk it side by side (with 2048 or
+// 4096 consecutive elements per wave instead, transposes of 2900, 4096 and 8192
+// squared took 162, 197 and 830 us, with chunks 126, 136 and 472; 5.2 M elements
+// in 85 blocks of a rank 4 tensor 83 and 61; 2048 squared 36 and 49).
 template<typename TS, typename T>
 __global__ __launch_bounds__(WG) void permute_kernel(const PermDev* __restrict__ tasks, const FlatUnit* __restrict__ units,
-                                                     int num_units, int elems) {
-    const int u = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * (WG / WAVE) + int(threadIdx.x) / WAVE);
+                                                     int num_chunks, int num_units) {
+    const bool chunk = int(blockIdx.x) < num_chunks;
+    const int u = chunk ? int(blockIdx.x)
+                        : __builtin_amdgcn_readfirstlane(num_chunks + (int(blockIdx.x) - num_chunks) * (WG / WAVE) +
+                                                         int(threadIdx.x) / WAVE);
     if (u >= num_units) return;
     const FlatUnit unit = units[u];
     const PermDev& tk = tasks[unit.task];
@@ -80,42 +88,49 @@ __global__ __launch_bounds__(WG) void permute_kernel(const PermDev* __restrict__
     const gptr<T> dst = to_global(static_cast<T*>(tk.dst));
     const int neg = tk.neg;
     const uint32_t n = uint32_t(tk.n), lane = threadIdx.x % WAVE;
-    const uint32_t first = uint32_t(unit.step) * uint32_t(elems), end = min(n, first + uint32_t(elems));
-    if (end - first <= WAVE) {
-        if (first + lane < end) {
+    if (!chunk && n - uint32_t(unit.step) * FLAT_UNIT <= WAVE) {
+        const uint32_t e = uint32_t(unit.step) * FLAT_UNIT + lane;
+        if (e < n) {
             int64_t so, dof;
-            perm_decode(first + lane, rank, dims, ss, ds, mul, sh, so, dof);
+            perm_decode(e, rank, dims, ss, ds, mul, sh, so, dof);
             dst[dof] = neg_if(T(src[so]), neg);
         }
         return;
     }
-    for (uint32_t base = first; base < end; base += FLAT_LANE * WAVE) {
-        int64_t so[FLAT_LANE], dof[FLAT_LANE];
+    // either may end with its task
+    const uint32_t stride = chunk ? WG : WAVE;
+    const uint32_t first = chunk ? uint32_t(unit.step) * FLAT_CHUNK + threadIdx.x : uint32_t(unit.step) * FLAT_UNIT + lane;
+    int64_t so[FLAT_LANE], dof[FLAT_LANE];
 #pragma unroll
-        for (int j = 0; j < FLAT_LANE; j++) {
-            const uint32_t e = base + lane + j * WAVE;
-            so[j] = dof[j] = 0;
-            if (e < end) perm_decode(e, rank, dims, ss, ds, mul, sh, so[j], dof[j]);
-        }
-        T v[FLAT_LANE];
-#pragma unroll
-        for (int j = 0; j < FLAT_LANE; j++) v[j] = (base + lane + j * WAVE < end) ? T(src[so[j]]) : T(0);
-#pragma unroll
-        for (int j = 0; j < FLAT_LANE; j++)
-            if (base + lane + j * WAVE < end) dst[dof[j]] = neg_if(v[j], neg);
+    for (int j = 0; j < FLAT_LANE; j++) {
+        const uint32_t e = first + j * stride;
+        so[j] = dof[j] = 0;
+        if (e < n) perm_decode(e, rank, dims, ss, ds, mul, sh, so[j], dof[j]);
     }
+    T v[FLAT_LANE];
+#pragma unroll
+    for (int j = 0; j < FLAT_LANE; j++) v[j] = (first + j * stride < n) ? T(src[so[j]]) : T(0);
+#pragma unroll
+    for (int j = 0; j < FLAT_LANE; j++)
+        if (first + j * stride < n) dst[dof[j]] = neg_if(v[j], neg);
 }
 
 template<typename T>
 __global__ __launch_bounds__(WG) void fill_kernel(const FillDev* __restrict__ tasks, const FlatUnit* __restrict__ units,
-                                                  int num_units, int elems) {
-    const int u = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * (WG / WAVE) + int(threadIdx.x) / WAVE);
+                                                  int num_chunks, int num_units) {
+    const bool chunk = int(blockIdx.x) < num_chunks;
+    const int u = chunk ? int(blockIdx.x)
+                        : __builtin_amdgcn_readfirstlane(num_chunks + (int(blockIdx.x) - num_chunks) * (WG / WAVE) +
+                                                         int(threadIdx.x) / WAVE);
     if (u >= num_units) return;
     const FlatUnit unit = units[u];
     const FillDev& tk = tasks[unit.task];
     const gptr<T> p = to_global(static_cast<T*>(tk.p));
-    const int64_t first = int64_t(unit.step) * elems, end = min(tk.n, first + int64_t(elems));
-    for (int64_t e = first + threadIdx.x % WAVE; e < end; e += WAVE) p[e] = T(0);
+    const int stride = chunk ? WG : WAVE;
+    const int64_t first = chunk ? int64_t(unit.step) * FLAT_CHUNK + threadIdx.x
+                                : int64_t(unit.step) * FLAT_UNIT + threadIdx.x % WAVE;
+    for (int j = 0; j < FLAT_LANE; j++)
+        if (first + j * stride < tk.n) p[first + j * stride] = T(0);
 }
 
 // ------------------------------------------------------------------- gemm
@@ -1608,44 +1623,46 @@ inline void check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// one wave per unit, WG / WAVE units per workgroup
-inline unsigned flat_blocks(int64_t num_units) { return unsigned((num_units + WG / WAVE - 1) / (WG / WAVE)); }
+// a workgroup per chunk, then one for WG / WAVE units
+inline dim3 flat_grid(int64_t num_chunks, int64_t num_units) {
+    return dim3(unsigned(num_chunks + (num_units - num_chunks + WG / WAVE - 1) / (WG / WAVE)));
+}
 
 }  // namespace
 
-void launch_permute(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems, int dtype,
+void launch_permute(const PermDev* tasks, const FlatUnit* units, int64_t num_chunks, int64_t num_units, int dtype,
                     hipStream_t stream) {
     if (num_units <= 0) return;
     if (dtype == 0)
-        hipLaunchKernelGGL((permute_kernel<double, double>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
-                           units, int(num_units), elems);
+        hipLaunchKernelGGL((permute_kernel<double, double>), flat_grid(num_chunks, num_units), dim3(WG), 0, stream, tasks,
+                           units, int(num_chunks), int(num_units));
     else
-        hipLaunchKernelGGL((permute_kernel<float, float>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
-                           units, int(num_units), elems);
+        hipLaunchKernelGGL((permute_kernel<float, float>), flat_grid(num_chunks, num_units), dim3(WG), 0, stream, tasks,
+                           units, int(num_chunks), int(num_units));
     check(hipGetLastError(), "permute launch");
 }
 
-void launch_permute_from_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems,
+void launch_permute_from_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_chunks, int64_t num_units,
                              int dtype, hipStream_t stream) {
     if (num_units <= 0) return;
     if (dtype == 0)
-        hipLaunchKernelGGL((permute_kernel<double, double>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
-                           units, int(num_units), elems);
+        hipLaunchKernelGGL((permute_kernel<double, double>), flat_grid(num_chunks, num_units), dim3(WG), 0, stream, tasks,
+                           units, int(num_chunks), int(num_units));
     else
-        hipLaunchKernelGGL((permute_kernel<double, float>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
-                           units, int(num_units), elems);
+        hipLaunchKernelGGL((permute_kernel<double, float>), flat_grid(num_chunks, num_units), dim3(WG), 0, stream, tasks,
+                           units, int(num_chunks), int(num_units));
     check(hipGetLastError(), "permute launch");
 }
 
-void launch_fill(const FillDev* tasks, const FlatUnit* units, int64_t num_units, int elems, int dtype,
+void launch_fill(const FillDev* tasks, const FlatUnit* units, int64_t num_chunks, int64_t num_units, int dtype,
                  hipStream_t stream) {
     if (num_units <= 0) return;
     if (dtype == 0)
-        hipLaunchKernelGGL(fill_kernel<double>, dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
-                           units, int(num_units), elems);
+        hipLaunchKernelGGL(fill_kernel<double>, flat_grid(num_chunks, num_units), dim3(WG), 0, stream, tasks,
+                           units, int(num_chunks), int(num_units));
     else
-        hipLaunchKernelGGL(fill_kernel<float>, dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
-                           units, int(num_units), elems);
+        hipLaunchKernelGGL(fill_kernel<float>, flat_grid(num_chunks, num_units), dim3(WG), 0, stream, tasks,
+                           units, int(num_chunks), int(num_units));
     check(hipGetLastError(), "fill launch");
 }
 
@@ -1662,11 +1679,11 @@ void launch_gather_f64(const GatherDev* tasks, int64_t num, double* dst, hipStre
     check(hipGetLastError(), "gather launch");
 }
 
-void launch_permute_to_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems,
+void launch_permute_to_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_chunks, int64_t num_units,
                            hipStream_t stream) {
     if (num_units <= 0) return;
-    hipLaunchKernelGGL((permute_kernel<float, double>), dim3(flat_blocks(num_units)), dim3(WG), 0, stream, tasks,
-                           units, int(num_units), elems);
+    hipLaunchKernelGGL((permute_kernel<float, double>), flat_grid(num_chunks, num_units), dim3(WG), 0, stream, tasks,
+                           units, int(num_chunks), int(num_units));
     check(hipGetLastError(), "permute launch");
 }
 

@@ -76,29 +76,26 @@ struct SvdDev {
 constexpr int SVD_MAX_SWEEPS = 60;
 
 // dtype: 0 = float64, 1 = float32
-// A unit of a permute or fill launch, done by one wave: the elements of one
-// task from step * elems on, `elems` (a launch parameter) of them at most.
+// A record of a permute or fill launch: `step` counts chunks of a task (one
+// workgroup each, first in the list) or units of FLAT_UNIT elements (one wave).
+// A task is cut into chunks; a rest of at most FLAT_UNIT elements is a unit, a
+// longer one a shorter chunk.
 struct FlatUnit {
     int32_t task;
     int32_t step;
 };
-// elements per lane and step of the permute kernel
-constexpr int FLAT_LANE = 8;
-// Elements per unit for a launch of `total` elements: one step of a wave
-// (512) while the launch has fewer units than the chip's 8192 wave slots hold,
-// more per unit beyond, where the records (8 bytes per unit) and the
-// descriptor reads would otherwise grow with the launch.
-inline int flat_unit_elems(int64_t total) {
-    return total <= (int64_t(1) << 21) ? 512 : (total <= (int64_t(1) << 24) ? 2048 : 4096);
-}
-void launch_permute(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems, int dtype,
+constexpr int FLAT_LANE = 8;  // elements per lane
+constexpr int FLAT_UNIT = 64 * FLAT_LANE, FLAT_CHUNK = 4 * FLAT_UNIT;
+inline int64_t flat_chunks(int64_t n) { return (n + FLAT_CHUNK - FLAT_UNIT - 1) / FLAT_CHUNK; }
+inline int64_t flat_units(int64_t n) { return n > flat_chunks(n) * FLAT_CHUNK; }
+void launch_permute(const PermDev* tasks, const FlatUnit* units, int64_t num_chunks, int64_t num_units, int dtype,
                     hipStream_t stream);
 // same copy with a float64 source (singular values into S)
-void launch_permute_from_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems,
+void launch_permute_from_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_chunks, int64_t num_units,
                              int dtype, hipStream_t stream);
-void launch_fill(const FillDev* tasks, const FlatUnit* units, int64_t num_units, int elems, int dtype,
+void launch_fill(const FillDev* tasks, const FlatUnit* units, int64_t num_chunks, int64_t num_units, int dtype,
                  hipStream_t stream);
-void launch_permute_to_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_units, int elems,
+void launch_permute_to_f64(const PermDev* tasks, const FlatUnit* units, int64_t num_chunks, int64_t num_units,
                            hipStream_t stream);
 // dtype: 0 float64, 1 float32, 2 float32 operands as split-bf16 x3 (hi*hi +
 // hi*lo + lo*hi), 3 split-bf16 x6 (three-term split, all products of order

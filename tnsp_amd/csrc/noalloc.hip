@@ -23,7 +23,11 @@ namespace {
 // workspace part (contract operands and product, QR factors and the global
 // scratch of large sectors) and task-record part of the array
 constexpr int64_t NOALLOC_WORKSPACE_BYTES = int64_t(64) << 20;
-constexpr int64_t NOALLOC_TASK_BYTES = (int64_t(4) << 20) + (int64_t(128) << 10);  // 4 MiB and the units' excess
+// Records: 4 MiB of tasks with 8 bytes of prefix each and 4 bytes per 2048
+// elements were the limit once.  The same plans need up to 4 bytes more per 2048
+// elements (4 MiB), 8 more per copy (a rest beside its chunks) and 8 more per
+// product (0.4 MiB together, a copy's task taking 192 bytes, a product's 72).
+constexpr int64_t NOALLOC_TASK_BYTES = int64_t(9) << 20;
 
 __device__ __align__(256) unsigned char scratch[NOALLOC_WORKSPACE_BYTES + NOALLOC_TASK_BYTES];
 

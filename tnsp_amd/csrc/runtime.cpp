@@ -184,22 +184,26 @@ void Batch::flush_flat(Kind kind, std::vector<PermDev>& pd, std::vector<FillDev>
     const bool isfill = kind == FILL;
     const size_t T = isfill ? fd.size() : pd.size();
     if (T == 0) return;
-    int64_t total = 0;
-    for (size_t i = 0; i < T; i++) total += isfill ? fd[i].n : pd[i].n;
-    const int64_t elems = flat_unit_elems(total);
-    std::vector<FlatUnit> units;
-    units.reserve(T + size_t(total / elems));
+    auto size = [&](size_t i) { return isfill ? fd[i].n : pd[i].n; };
+    int64_t chunks = 0, total = 0;
     for (size_t i = 0; i < T; i++) {
-        const int64_t n = isfill ? fd[i].n : pd[i].n;
-        for (int64_t k = 0; k * elems < n; k++) units.push_back(FlatUnit{int32_t(i), int32_t(k)});
+        chunks += flat_chunks(size(i));
+        total += flat_chunks(size(i)) + flat_units(size(i));
     }
-    if (int64_t(units.size()) >= (int64_t(1) << 31)) throw Error("permute launch too large");
+    if (total >= (int64_t(1) << 31)) throw Error("permute launch too large");
     Cmd c;
     c.kind = kind;
     c.tasks = isfill ? put(fd) : put(pd);
-    c.prefix = put(units);
-    c.count = elems;
-    c.nwg = int64_t(units.size());
+    c.prefix = put(std::vector<FlatUnit>());
+    blob_.resize(c.prefix + size_t(total) * sizeof(FlatUnit));
+    FlatUnit *c0 = reinterpret_cast<FlatUnit*>(blob_.data() + c.prefix), *u0 = c0 + chunks;
+    for (size_t i = 0; i < T; i++) {
+        const int64_t nc = flat_chunks(size(i));
+        for (int64_t k = 0; k < nc; k++) *c0++ = FlatUnit{int32_t(i), int32_t(k)};
+        if (flat_units(size(i))) *u0++ = FlatUnit{int32_t(i), int32_t(nc * (FLAT_CHUNK / FLAT_UNIT))};
+    }
+    c.count = chunks;
+    c.nwg = total;
     c.units = pend_units_[kind];
     pend_units_[kind] = 0;
     cmds_.push_back(c);
@@ -582,21 +586,21 @@ void Batch::run(hipStream_t st) {
             case PERM:
                 if (c.conv == 1)
                     launch_permute_from_f64(reinterpret_cast<const PermDev*>(base + c.tasks),
-                                            reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), 1, st);
+                                            reinterpret_cast<const FlatUnit*>(base + c.prefix), c.count, c.nwg, 1, st);
                 else if (c.conv == 2)
                     launch_permute_to_f64(reinterpret_cast<const PermDev*>(base + c.tasks),
-                                          reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), st);
+                                          reinterpret_cast<const FlatUnit*>(base + c.prefix), c.count, c.nwg, st);
                 else
                     launch_permute(reinterpret_cast<const PermDev*>(base + c.tasks),
-                                   reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), dtype_, st);
+                                   reinterpret_cast<const FlatUnit*>(base + c.prefix), c.count, c.nwg, dtype_, st);
                 break;
             case DIAG:
                 launch_permute_from_f64(reinterpret_cast<const PermDev*>(base + c.tasks),
-                                        reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), dtype_, st);
+                                        reinterpret_cast<const FlatUnit*>(base + c.prefix), c.count, c.nwg, dtype_, st);
                 break;
             case FILL:
                 launch_fill(reinterpret_cast<const FillDev*>(base + c.tasks),
-                            reinterpret_cast<const FlatUnit*>(base + c.prefix), c.nwg, int(c.count), c.dt >= 0 ? c.dt : dtype_, st);
+                            reinterpret_cast<const FlatUnit*>(base + c.prefix), c.count, c.nwg, c.dt >= 0 ? c.dt : dtype_, st);
                 break;
             case GEMM:
                 launch_gemm(reinterpret_cast<const GemmDev*>(base + c.tasks),

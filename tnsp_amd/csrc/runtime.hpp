@@ -140,7 +140,7 @@ class Batch {
     struct Cmd {
         Kind kind;
         size_t tasks, prefix;  // blob offsets (prefix: GEMM tiles, permute / fill units)
-        int64_t count, nwg;    // permute / fill: elements per unit, units
+        int64_t count, nwg;    // permute / fill: chunks, chunks and units
         double units = 0;  // algorithmic flops or bytes of this launch
         int64_t lds = 0;   // dynamic LDS bytes (decompositions)
         int rpt = 0;       // register tile of the large-block SVD kernel
