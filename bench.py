@@ -243,10 +243,11 @@ def kernel_rates(kstats):
     """Achieved rate of each kernel kind over the launches of the kernel
     timing pass (HIP events on the launch stream): flops for GEMM / QR / SVD
     against the fp64 matrix peak, bytes for permute / fill / diag against
-    HBM."""
+    HBM.  Jacobi kernels that only got what the eigenvector path left over
+    have time but no work of their own, hence no rate."""
     out = {}
     for kind, s in kstats.items():
-        if s["launches"] == 0 or s["ms"] <= 0:
+        if s["launches"] == 0 or s["ms"] <= 0 or s["units"] <= 0:
             continue
         rate = s["units"] / (s["ms"] / 1e3)
         if kind in ("permute", "fill", "diag"):

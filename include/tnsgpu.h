@@ -180,8 +180,11 @@ int tns_engine_stats(const tns_engine* e, double* values, int n);
 int tns_engine_reset_stats(tns_engine* e);
 /* per-kernel device timing with HIP events on the launch stream: permute,
  * fill, gemm, qr (LDS / unblocked), svd (LDS / global), diag, qr_blocked,
- * svd_reg8, svd_reg16, svd_reg24; per kernel: launches, total ms,
- * algorithmic work (bytes for permute/fill/diag, flops for the others) */
+ * svd_reg8, svd_reg16, svd_reg24, svd_eig; per kernel: launches, total ms,
+ * algorithmic work (bytes for permute/fill/diag, flops for the others).  A
+ * sector tried on svd_eig counts there, also where it is left to a Jacobi
+ * kernel: the work of svd and svd_reg* is that of sectors never tried, their
+ * time includes the ones left to them */
 int tns_engine_set_profile(tns_engine* e, int on);
 /* the caller changed the site tensors' values in place (same buffers and
  * block structure), e.g. a gradient step (sampling_lattice/lattice.py:936-948):

@@ -164,3 +164,21 @@ def test_profiling_stops_when_switched_off():
     eng.evaluate(configs[:8])
     eng.set_profile(False)
     assert launches(eng) == {k: 2 * v for k, v in once.items()}
+
+
+def test_kernel_stats_count_each_sector_once():
+    """The flops of the SVD and QR kernels add up to those of the sectors."""
+    from tnsp_amd import peps as ppeps
+    from tnsp_amd.engine import AmplitudeEngine
+
+    spec, storages, configs, _ = golden8("C3_8x8_Z2_D6_Dc36")
+    eng = AmplitudeEngine(ppeps.Lattice(spec, storages), chunk=4, lanes=1)
+    eng.evaluate(configs[:4])
+    eng.reset_stats()
+    eng.set_profile(True)
+    eng.evaluate(configs[:4])
+    stats, ks = eng.stats(), eng.kernel_stats()
+    assert ks["svd_eig"]["units"] > 0
+    for kernel in ("svd", "qr"):
+        units = sum(v["units"] for k, v in ks.items() if k.startswith(kernel))
+        np.testing.assert_allclose(units, stats[kernel + "_flops"], rtol=1e-6)

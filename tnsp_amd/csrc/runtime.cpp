@@ -326,6 +326,11 @@ void Batch::qr(const std::vector<QrTask>& ts, void* const* bufs, int64_t es, dou
     }
 }
 
+// A sector's work counts once: with the eigenvector path where it was tried
+// there, whoever finishes it (only the device knows).
+static bool counted_before(const QrDev&) { return false; }
+static bool counted_before(const SvdDev& t) { return t.done != nullptr; }
+
 // Split a decomposition launch into an LDS-resident part (working set fits
 // the per-workgroup LDS budget) and a global-scratch part; within each,
 // largest blocks first so the long ones start early.
@@ -356,7 +361,7 @@ void Batch::flush_decomp(Kind kind, std::vector<D>& tasks, std::vector<double>& 
             p = bytes <= LDS_CLASS[0] ? 3 : (bytes <= LDS_CLASS[1] ? 2 : 1);
         }
         parts[p].push_back(tasks[i]);
-        units[p] += cost[i];
+        if (!counted_before(tasks[i])) units[p] += cost[i];
         need[p] = std::max(need[p], bytes);
     }
     for (int part = 0; part < NPART; part++) {

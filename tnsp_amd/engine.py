@@ -105,7 +105,9 @@ class AmplitudeEngine:
 
     def kernel_stats(self):
         """{kernel: {"launches", "ms", "units"}}; units are bytes for permute /
-        fill / diag and flops for gemm and the QR / SVD kernels."""
+        fill / diag and flops for gemm and the QR / SVD kernels.  A sector
+        tried on svd_eig counts there, also where a Jacobi kernel (svd,
+        svd_reg*) finishes it."""
         n = 3 * len(self.KERNEL_KINDS)
         vals = (ctypes.c_double * n)()
         _lib.check(_lib.lib().tns_engine_kernel_stats(self.handle, vals, n))
