@@ -65,3 +65,26 @@ def test_layer_beyond_lds_is_refused():
     with pytest.raises(RuntimeError, match="exceeds LDS"):
         _lib.check(_lib.lib().tns_conv3x3_backward_data(p, p, p, p, 2, 3, 64, 32, 32,
                                                         torch.cuda.current_stream().cuda_stream))
+
+
+@pytest.mark.parametrize("v", [1.1454734802246094, 1.1126136779785156, 1.8636400699615479])
+def test_partial_gradients_add_in_short_chains(v):
+    """1024 equal samples, whose sums round one way in a long chain: two
+    additions within a workgroup, then 16 + 3 + 2 over the 512 workgroups, each
+    off by at most 2^-24 of the sum."""
+    import ctypes
+
+    from tnsp_amd import _lib
+
+    lib, check = _lib.lib(), _lib.check
+    B = 1024
+    x, dy = torch.ones(B, device="cuda"), torch.full((B,), v, device="cuda")
+    dw, db = torch.empty(9, device="cuda"), torch.empty(1, device="cuda")
+    ws = ctypes.c_int64()
+    check(lib.tns_conv3x3_backward_weight_workspace(B, 1, 1, ctypes.byref(ws)))
+    work = torch.empty(ws.value // 4, device="cuda")
+    check(lib.tns_conv3x3_backward_weight(dy.data_ptr(), None, x.data_ptr(), dw.data_ptr(), db.data_ptr(), B, 1, 1, 1,
+                                          1, work.data_ptr(), torch.cuda.current_stream().cuda_stream))
+    exact = B * float(dy[0].cpu())
+    for got in (float(dw[4]), float(db[0])):
+        assert abs(got - exact) <= 23 * 2.0 ** -24 * exact

@@ -182,3 +182,15 @@ def test_kernel_stats_count_each_sector_once():
     for kernel in ("svd", "qr"):
         units = sum(v["units"] for k, v in ks.items() if k.startswith(kernel))
         np.testing.assert_allclose(units, stats[kernel + "_flops"], rtol=1e-6)
+
+
+def test_psi_does_not_depend_on_the_batch():
+    """Amplitudes of the 8x8 D=8 PEPS alone and in a batch: the same bits
+    (every sector's route depends on its own size only)."""
+    from tnsp_amd import peps as ppeps
+    from tnsp_amd.engine import AmplitudeEngine
+
+    spec, storages, configs, _ = golden8("C4_8x8_U1_D8_Dc64")
+    eng = AmplitudeEngine(ppeps.Lattice(spec, storages), chunk=8, lanes=1)
+    together = eng.evaluate(configs)
+    assert np.array_equal(together, np.concatenate([eng.evaluate(configs[i:i + 1]) for i in range(len(configs))]))

@@ -230,7 +230,9 @@ __global__ __launch_bounds__(NT) void conv_bwd_weight_kernel(const float* __rest
 // out[k] = sum over the chunks of part[c][k], k < n, for the weights and the
 // biases in one launch: 64 outputs per workgroup, its four waves take every
 // fourth chunk and their sums meet in LDS (one thread per output left most of
-// the chip idle behind a serial chain over the chunks).
+// the chip idle behind a serial chain over the chunks).  A lane keeps eight
+// sums: eight loads in flight, and chains of 16 additions over 512 chunks where
+// one sum would make 128, whose rounding was most of the gradients' error.
 __global__ __launch_bounds__(NT) void reduce_chunks_kernel(const float* __restrict__ part, const float* __restrict__ partb,
                                                            int chunks, int nw, int nb, float* __restrict__ dw,
                                                            float* __restrict__ db) {
@@ -241,12 +243,19 @@ __global__ __launch_bounds__(NT) void reduce_chunks_kernel(const float* __restri
     const int n = bias ? nb : nw;
     const float* src = bias ? partb : part;
     const int k = (int(blockIdx.x) - (bias ? wblocks : 0)) * 64 + lane;
-    float s = 0.f;
+    constexpr int R = 8;
+    float s[R] = {};
     if (k < n) {
-#pragma unroll 4
-        for (int c = wave; c < chunks; c += NT / 64) s += src[int64_t(c) * n + k];
+        for (int c = wave; c < chunks; c += R * (NT / 64)) {
+            float v[R];
+            // beyond the last chunk the last one is read and not added
+#pragma unroll
+            for (int u = 0; u < R; u++) v[u] = src[int64_t(min(c + u * (NT / 64), chunks - 1)) * n + k];
+#pragma unroll
+            for (int u = 0; u < R; u++) s[u] += c + u * (NT / 64) < chunks ? v[u] : 0.f;
+        }
     }
-    red[wave][lane] = s;
+    red[wave][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
     __syncthreads();
     if (wave == 0 && k < n) (bias ? db : dw)[k] = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
 }
