@@ -165,7 +165,11 @@ __device__ inline double block_sum(double v, double* red) {
     return t;
 }
 
-// hardware reciprocal / reciprocal square root refined by two Newton steps
+// hardware reciprocal / reciprocal square root refined by two Newton steps:
+// within a few ulp where argument and result are normal numbers (the Jacobi
+// rotations' arguments lie in [1, inf); the tridiagonalisations' and twisted
+// factorisations' come from blocks scaled to entries of order one, the pivots
+// floored)
 __device__ inline double refined_rcp(double x) {
     double r = __builtin_amdgcn_rcp(x);
     r = fma(r, fma(-x, r, 1.0), r);

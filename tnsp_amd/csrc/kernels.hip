@@ -386,10 +386,9 @@ __device__ inline int group_lanes(int len) { return len <= 48 ? 16 : (len <= 96 
 
 // Jacobi rotation (cs, sn) zeroing the off-diagonal of [[saa, sab], [sab,
 // sbb]] (Rutishauser's formulas, sab != 0).  The two reciprocals after the
-// exact zeta use the hardware reciprocal / reciprocal square root refined by
-// two Newton steps each: their arguments lie in [1, inf), and
-// cs^2 + sn^2 = cs^2 (1 + t^2) stays 1 to rounding, which is what keeps the
-// accumulated transformation orthogonal.
+// exact zeta are the refined hardware ones (device.hpp); both arguments lie in
+// [1, inf) here, and cs^2 + sn^2 = cs^2 (1 + t^2) stays 1 to rounding, which is
+// what keeps the accumulated transformation orthogonal.
 // t = tan of the angle: after a' = cs a - sn b, b' = sn a + cs b the squared
 // norms are exactly saa - t sab and sbb + t sab (t solves t^2 + 2 zeta t = 1)
 __device__ inline void jacobi_rotation(double saa, double sbb, double sab, double& cs, double& sn, double& t) {
@@ -414,10 +413,6 @@ __device__ inline double jacobi_tracked(double old_n, double new_n) {
 }
 
 // --------------------------------------------------------------------- qr
-// Householder QR of X (mx x nx, column-major), X = M (qr) or X = M^T (lq);
-// R is written out first, then Q is formed in place from the reflectors
-// (backward accumulation, as LAPACK's orgqr does).  X lives in LDS when it
-// fits, otherwise in global scratch.
 // Apply the reflector of column j (unit diagonal implied, entries below j in
 // cj) to columns j + 1 .. nc - 1 of X (column stride ld), one group of G
 // lanes per column.  The group that updates column j + 1 also sums the
@@ -464,6 +459,10 @@ __device__ inline int qr_group_lanes(int rows, int cols) {
     return G;
 }
 
+// Householder QR of X (mx x nx, column-major), X = M (qr) or X = M^T (lq);
+// R is written out first, then Q is formed in place from the reflectors
+// (backward accumulation, as LAPACK's orgqr does).  X lives in LDS when it
+// fits, otherwise in global scratch.
 // I: type of element indices.  32 bits where the block is in LDS: the passes that
 // load it and write R and Q divide once per element, and 64-bit divisions took
 // longer there than the range test.

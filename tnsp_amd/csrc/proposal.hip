@@ -140,7 +140,7 @@ __global__ __launch_bounds__(NT) void conv_mfma_kernel(const float* __restrict__
 // Lane l holds dy(co0 + l % 16, p + l / 16) and x(p + l / 16, n0 + l % 16).
 // The VALU version (one thread per weight, 64 samples per workgroup, 16
 // workgroups for 1024 samples) took 3.8 ms per launch on 1024 samples of 32
-// channels, 8 x 8; this kernel 31 us and its reduction 12.
+// channels, 8 x 8; this kernel 31 us and its reduction 8.
 template<int MT, int NPW>
 __global__ __launch_bounds__(NT) void conv_bwd_weight_kernel(const float* __restrict__ dy,
                                                              const float* __restrict__ relu_y,
@@ -439,11 +439,14 @@ void launch_conv_bwd_data(const float* dy, const float* relu_y, const uint16_t* 
 }
 
 namespace {
-// Samples per workgroup of the weight gradient: enough workgroups to fill the
-// chip (each CU holds a few), few enough that their partial gradients (37 KB
-// each at 32 channels) stay a small part of the traffic.  1024 samples of 32
-// channels, 8 x 8, all four layers with the reductions: 143 us with 2 samples
-// per workgroup, 165 us with 4, 296 us with 8.
+// Samples per workgroup of the weight gradient: one while that gives at most
+// 512 workgroups (each CU holds a few; a workgroup's samples are a serial
+// chain), more beyond, so that the partial gradients (37 KB each at 32 channels)
+// stay a small part of the traffic.  All layers with the reductions, 1 / 2 / 4 / 8
+// samples per workgroup: 32 channels, 8 x 8, 64 samples 54 / 91 / 149 / 259 us,
+// 512 samples 94 / 98 / 153 / 267, 1024 samples (2 at least) 128 / 156 / 269; 24
+// channels, 10 x 10, 128 samples 51 / 84 / 145 / 259; 8 channels, 4 x 4, 512 samples
+// 41 / 34 / 35 / 54.
 constexpr int CONV_CHUNKS_MAX = 512;
 int conv_chunk(int B) { return std::max(1, (B + CONV_CHUNKS_MAX - 1) / CONV_CHUNKS_MAX); }
 }  // namespace
