@@ -131,8 +131,11 @@ inline int64_t qr_doubles(int64_t m, int64_t n) { return m * n + (m < n ? m : n)
 // 200), 30 x 20 433 / 909 / 2792 against 360 / 1002 / 3205, 200 x 16 390 / 889 /
 // 2894 against 347 / 965 / 3149: below 24 columns many small sectors lose.  The
 // sector's size alone decides, so that its factors do not depend on what shares
-// its launch.  Above 640 columns the eigenvector strips no longer fit the
-// registers of one wave.
+// its launch.  A sector the path has to leave to the Jacobi kernels pays for
+// both: 150 columns with singular values over 5 decades 7.8 -> 8.8 ms, over 12
+// 12.5 -> 13.6, 32 columns 0.81 -> 1.03 and 0.95 -> 1.18, 210 columns 200 -> 206.
+// Above 640 columns the eigenvector strips no longer fit the registers of one
+// wave.
 constexpr int SVD_EIG_MIN_COLS = 24, SVD_EIG_MAX_COLS = 640;
 inline bool svd_eig_fits(int64_t m, int64_t n) {
     const int64_t mx = m > n ? m : n, kx = m < n ? m : n;
