@@ -1,4 +1,4 @@
-"""The eigenvector path of the sector SVD (blocks of 24 to 640 columns) at the
+"""The eigenvector path of the sector SVD (blocks of 16 to 640 columns) at the
 edges of its tiles, and blocks it has to leave to the Jacobi kernels, against
 numpy's LAPACK.
 
@@ -41,7 +41,7 @@ def check(x, dtype, factors=True):
         assert np.max(np.abs(v @ v.T - np.eye(len(s)))) <= tol
 
 
-@pytest.mark.parametrize("m,n", [(32, 32), (33, 47), (64, 64), (65, 63), (100, 66), (128, 128), (129, 130), (192, 192),
+@pytest.mark.parametrize("m,n", [(16, 16), (17, 40), (100, 23), (32, 32), (33, 47), (64, 64), (65, 63), (100, 66), (128, 128), (129, 130), (192, 192),
                                  (193, 200), (64, 700), (1100, 40), (320, 320), (321, 333), (640, 640), (641, 645)])
 def test_random_blocks(m, n):
     check(np.random.default_rng(m * 1000 + n).standard_normal((m, n)), "D")
@@ -141,7 +141,8 @@ def test_equal_columns_float32(n):
     check_orthonormal(x, "S")
 
 
-@pytest.mark.parametrize("first", [(24, 24), (23, 31), (23, 23), (16, 31), (31, 20), (8, 9)])
+@pytest.mark.parametrize("first", [(24, 24), (23, 31), (16, 16), (16, 31), (15, 31), (15, 15), (31, 20),
+                                   (8, 9)])
 def test_sector_does_not_depend_on_its_company(first):
     """A sector alone and beside a larger one that takes the eigenvector path:
     the same bits."""

@@ -121,22 +121,27 @@ inline int64_t qr_doubles(int64_t m, int64_t n) { return m * n + (m < n ? m : n)
 // Sectors that go through the eigenvectors of their Gram matrix first
 // (svd_eig.hip).  Whole SVD passes with the Jacobi kernels alone and with this
 // path: 64 tensors with sectors up to about 200 x 190 (some beyond the register
-// kernel's 192 rows) 98.6 -> 4.8 ms; 4 tensors with sectors up to about
-// 310 x 260 199 -> 5.4 ms; one stage of 128 8x8 D=8 configurations (register
+// kernel's 192 rows) 99.2 -> 4.4 ms; 4 tensors with sectors up to about
+// 310 x 260 199 -> 5.2 ms; one stage of 128 8x8 D=8 configurations (register
 // 24 / 16 and LDS kernels, one after the other) 11.1 -> 4.9 ms.  The lower line:
 // tensors of one sector, whole passes with the LDS Jacobi kernel against this
 // path, 1, 16 and 200 tensors a call: 31 x 30 599 / 1146 / 3118 against 415 /
 // 1005 / 3152 us, 140 x 28 567 / 1140 / 3193 against 433 / 1045 / 3047, 24 x 24
-// 483 / 1015 / 3029 against 360 / 996 / 3253 (runs of one side differ by 19% at
-// 200), 30 x 20 433 / 909 / 2792 against 360 / 1002 / 3205, 200 x 16 390 / 889 /
-// 2894 against 347 / 965 / 3149: below 24 columns many small sectors lose.  The
-// sector's size alone decides, so that its factors do not depend on what shares
-// its launch.  A sector the path has to leave to the Jacobi kernels pays for
+// 483 / 1015 / 3029 against 360 / 996 / 3253, 30 x 20 433 / 909 / 2792 against 360 /
+// 1002 / 3205, 200 x 16 390 / 889 / 2894 against 347 / 965 / 3149, 16 x 16 369 / 908 /
+// 2864 against 369 / 939 / 3111 (host planning is most of a pass of many tensors,
+// runs of one side differ by up to 20% there).  Where sectors of 16 to 31 columns
+// are the largest of many tensors with smaller ones too, the LDS kernel runs
+// anyway and the path adds 0.13 to 0.2 ms (21 tensors 1.52 -> 1.65 ms, 59 tensors
+// 1.78 -> 1.97); beside larger sectors it adds next to nothing, and a launch of the
+// LDS kernel for those of 16 to 23 columns would cost 10 to 20% of a pass of 1 to
+// 2 ms.  The sector's size alone decides, so that its factors do not depend on
+// what shares its launch.  A sector the path has to leave to the Jacobi kernels pays for
 // both: 150 columns with singular values over 5 decades 7.8 -> 8.8 ms, over 12
 // 12.5 -> 13.6, 32 columns 0.81 -> 1.03 and 0.95 -> 1.18, 210 columns 200 -> 206.
 // Above 640 columns the eigenvector strips no longer fit the registers of one
 // wave.
-constexpr int SVD_EIG_MIN_COLS = 24, SVD_EIG_MAX_COLS = 640;
+constexpr int SVD_EIG_MIN_COLS = 16, SVD_EIG_MAX_COLS = 640;
 inline bool svd_eig_fits(int64_t m, int64_t n) {
     const int64_t mx = m > n ? m : n, kx = m < n ? m : n;
     return kx >= SVD_EIG_MIN_COLS && kx <= SVD_EIG_MAX_COLS && mx * kx <= (int64_t(1) << 28);
